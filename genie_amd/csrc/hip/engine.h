@@ -118,6 +118,12 @@ struct DevIndex {
     uint4* seg_bph = nullptr;       // [n_segments] BP32 block header word offsets, 8 x u16 (BP32 codecs)
     uint32_t* sdir_off = nullptr;   // [n_keys] row of each key with more than 4 segments (compressed)
     uint32_t* sdir = nullptr;       // graded segment-directory rows (compressed)
+    // tile-major copy of the postings (16-bit ids within tiles of 65,536
+    // objects) for the direct-mapped scan; a compressed index has only the
+    // directory, its plans decode into copies of their own
+    uint16_t* run_ids = nullptr;    // [n_postings + kRunPad]   (uncompressed)
+    uint2* run_tf = nullptr;        // [run_tiles * n_keys + 1] (null: no copy)
+    uint32_t run_tiles = 0;
     // forward codes of a single-value table (dense form of the batched search)
     bool dense = false;
     uint32_t dense_dpad = 0;        // dims rounded up to 16

@@ -35,6 +35,7 @@
 #include "kernels_batched.h"
 #include "kernels_dense.h"
 #include "kernels_hash.h"
+#include "kernels_runs.h"
 #include "wave.h"
 
 namespace gh {
@@ -153,6 +154,7 @@ struct genie_plan {
     uint64_t fjobs_alloc = 0;
     genie_dim_t* d_uitems = nullptr;      // [max_items]
     uint32_t* d_full = nullptr;           // [n_postings]
+    uint16_t* d_runs = nullptr;           // [n_postings + kRunPad] the same segments decoded tile-major
     // device buffers
     genie_dim_t* d_items = nullptr;
     uint32_t* d_item_qptr = nullptr;
@@ -332,6 +334,7 @@ static void plan_free_buffers(genie_plan* p)
     dev_free(p->d_fjobs);
     dev_free(p->d_uitems);
     dev_free(p->d_full);
+    dev_free(p->d_runs);
 }
 
 // Count bound of every query: per (query, order) group the largest weight
@@ -481,6 +484,7 @@ int gh::validate_items(const DevIndex& d, const genie_dim_t* items, uint64_t n_i
 
 static bool dense_shape(const genie_index_desc* desc, std::vector<uint32_t>& key_base, std::vector<uint32_t>& per_dim);
 static int build_sets(const genie_index_desc* desc, DevIndex& d);
+static int build_runs(DevIndex& d, const uint32_t* post, bool copy);
 static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t* post, const uint32_t* key_start);
 
 // Compressed index: words, segment offsets, key -> segment map, per-segment
@@ -682,6 +686,8 @@ static int create_compressed(const genie_index_desc* desc, genie_index** out)
         }
         if (want_dense)
             rc = build_dense(desc, d, d_post, d.key_start);
+        if (!rc)
+            rc = build_runs(d, d_post, false);
         if (!rc)
             rc = build_sets(desc, d);
     } while (0);
@@ -1044,6 +1050,52 @@ static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t
     return GENIE_OK;
 }
 
+// Tile-major copy of the postings for the direct-mapped scan (kernels_runs.h):
+// the directory, and with `copy` the 16-bit ids, from the device posting
+// array.  An index whose lists are too short per tile, or a device without
+// room for it, simply has none; only kernel errors fail.
+static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
+{
+    const uint64_t N = d.n_objects, K = d.n_keys, nt = (N + kRunTile - 1) / kRunTile;
+    if (d.n_postings * kRunTile < (uint64_t)kRunMinPerTile * K * N || K * nt >= 0x7FFFFFFFull)
+        return GENIE_OK;
+    const uint32_t n = (uint32_t)(K * nt), nb = (n + 1023) / 1024;
+    uint32_t *cnt = nullptr, *pre = nullptr, *sums = nullptr, *total = nullptr;
+    uint2* tf = nullptr;
+    uint16_t* ids = nullptr;
+    auto room = [](auto** p, uint64_t count) { return hipMalloc((void**)p, count * sizeof(**p)) == hipSuccess; };
+    hipError_t e = hipSuccess;
+    const bool ok = room(&cnt, n) && room(&pre, n) && room(&sums, nb) && room(&total, 1) && room(&tf, n + 1ull) &&
+                    (!copy || room(&ids, d.n_postings + kRunPad));
+    if (ok) {
+        k_run_first<<<(n + 255) / 256, 256>>>(post, d.key_start, d.n_keys, (uint32_t)nt, tf, cnt);
+        k_scan_blocks<<<nb, 256>>>(cnt, pre, n, sums);
+        k_scan_sums<<<1, 256>>>(sums, nb, total);
+        k_scan_add<<<nb, 256>>>(pre, n, sums);
+        k_run_start<<<n / 256 + 1, 256>>>(pre, n, (uint32_t)d.n_postings, tf);
+        if (copy)
+            k_run_fill<<<d.n_keys, 256>>>(post, d.key_start, d.n_keys, tf, ids);
+        if ((e = hipGetLastError()) == hipSuccess)
+            e = hipDeviceSynchronize();
+    } else {
+        (void)hipGetLastError();  // no room: no copy
+    }
+    dev_free(cnt);
+    dev_free(pre);
+    dev_free(sums);
+    dev_free(total);
+    if (!ok || e != hipSuccess) {
+        dev_free(tf);
+        dev_free(ids);
+        return ok ? fail(GENIE_E_RUNTIME, std::string("tile-major copy: ") + hipGetErrorString(e)) : GENIE_OK;
+    }
+    d.run_tf = tf;
+    d.run_ids = ids;
+    d.run_tiles = (uint32_t)nt;
+    d.bytes += (n + 1ull) * sizeof(uint2) + (copy ? (d.n_postings + kRunPad) * sizeof(uint16_t) : 0);
+    return GENIE_OK;
+}
+
 // Forward lists for the set form: for a set-valued table whose postings are
 // given and whose objects hold at most 255 occurrences, every object's keys
 // (an object listed twice in one key's list appears twice).  Laid out for
@@ -1318,6 +1370,8 @@ int genie_hip_index_create(const genie_index_desc* desc, genie_index** out)
     if (!rc)
         rc = build_dense(desc, d, d.post, d.key_start);
     if (!rc)
+        rc = build_runs(d, d.post, true);
+    if (!rc)
         rc = build_sets(desc, d);
     if (rc) {
         genie_hip_index_destroy(ix);
@@ -1346,6 +1400,8 @@ int genie_hip_index_destroy(genie_index* ix)
     dev_free(d.key_seg);
     dev_free(d.sdir_off);
     dev_free(d.sdir);
+    dev_free(d.run_ids);
+    dev_free(d.run_tf);
     dev_free(d.codes);
     dev_free(d.key_slot);
     dev_free(d.obj_perm);
@@ -2036,6 +2092,38 @@ static int plan_decoded_spans(genie_plan* p)
     return GENIE_OK;
 }
 
+// Whether the plain form marks touched counter words and selects sparsely:
+// on average fewer postings per (query, tile) than a quarter of the tile's
+// counter words (each tile still falls back to the dense select when it
+// turns out busier, kSparseWords).
+static bool plain_sparse(const genie_plan* p, uint32_t n_tiles)
+{
+    if (p->sparse_mode >= 0)
+        return p->sparse_mode != 0;
+    if (p->h_dq.empty())
+        return false;
+    const double per = (double)p->est_postings / ((double)p->h_dq.size() * (double)n_tiles);
+    return per <= (double)kCntWords / 4;
+}
+
+// Whether the plain form's direct-mapped queries are counted over the
+// tile-major copy (kernels_runs.h): counts of at most 16 bits, a dense select
+// (a batch of few postings per tile stays on the sparse select, which visits
+// only the words it touched), and a copy to read -- the index's own, or the
+// plan's scratch of a compressed index, which needs the batch decoded first.
+static bool runs_active(const genie_plan* p)
+{
+    const DevIndex& d = p->ix->d;
+    if (!d.run_tf || p->lane_bits > 16 || p->h_dq.empty() || (d.codec != 0 && p->decode_mode == 0))
+        return false;
+    const uint32_t to = tile_objs_for(p->lane_bits);
+    return !plain_sparse(p, (d.n_objects + to - 1) / to);
+}
+
+// Whether the next run's direct-mapped queries are: a compressed batch also
+// has to have been given its decode jobs.
+static bool runs_used(const genie_plan* p) { return runs_active(p) && (p->ix->d.codec == 0 || p->dec_full); }
+
 // Compressed index, plain form: the segments any item of the batch names,
 // each once, become decode jobs into a scratch array of the uncompressed
 // layout, and every item is translated from word to posting positions (items
@@ -2050,10 +2138,15 @@ static int plan_full_decode(genie_plan* p)
     p->n_chunks = p->n_chunks_runs;
     if (d.codec == 0 || p->decode_mode == 0 || !d.key_start || p->n_items == 0)
         return GENIE_OK;
-    if (!p->d_full) {
-        if (dev_alloc(&p->d_full, std::max<uint64_t>(1, d.n_postings)) != GENIE_OK)
+    // the layouts that the batch's kernels read: tile-major for the
+    // direct-mapped scan over runs, the posting lists' for the others
+    const bool tiled = runs_active(p);
+    if (tiled && !p->d_runs)
+        if (dev_alloc(&p->d_runs, d.n_postings + kRunPad) != GENIE_OK)
             return GENIE_OK;  // no room for the scratch: in-kernel decode
-    }
+    if ((!tiled || !p->h_hwork.empty()) && !p->d_full)
+        if (dev_alloc(&p->d_full, std::max<uint64_t>(1, d.n_postings)) != GENIE_OK)
+            return GENIE_OK;
     if (!p->d_uitems)
         if (int rc = dev_alloc(&p->d_uitems, std::max<uint64_t>(1, p->max_items)))
             return rc;
@@ -2437,20 +2530,6 @@ static ScanArgs scan_args(genie_plan* p)
     return a;
 }
 
-// Whether the plain form marks touched counter words and selects sparsely:
-// on average fewer postings per (query, tile) than a quarter of the tile's
-// counter words (each tile still falls back to the dense select when it
-// turns out busier, kSparseWords).
-static bool plain_sparse(const genie_plan* p, uint32_t n_tiles)
-{
-    if (p->sparse_mode >= 0)
-        return p->sparse_mode != 0;
-    if (p->h_dq.empty())
-        return false;
-    const double per = (double)p->est_postings / ((double)p->h_dq.size() * (double)n_tiles);
-    return per <= (double)kCntWords / 4;
-}
-
 template <bool SPARSE>
 static void launch_scan_t(uint32_t lane_bits, const ScanArgs& a, uint32_t blocks, hipStream_t s)
 {
@@ -2469,25 +2548,36 @@ static void launch_scan_t(uint32_t lane_bits, const ScanArgs& a, uint32_t blocks
     }
 }
 
-// k_decode_jobs instantiated for the index's codec.
-static int launch_decode_jobs(const DevIndex& d, const uint2* jobs, uint32_t nj, uint32_t* out, hipStream_t s)
+// k_decode_jobs instantiated for the index's codec; `runs`: into a tile-major
+// copy at `out`.
+template <int CODEC>
+static void launch_decode_t(const DevIndex& d, const uint2* jobs, uint32_t nj, void* out, bool runs, uint32_t g,
+                            hipStream_t s)
+{
+    const RunDst rd{d.run_tf, d.seg_key, d.seg_first, d.seg_last, d.n_keys};
+    if (runs)
+        k_decode_jobs<CODEC, true><<<g, kDecodeWaves * kWave, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out, rd);
+    else
+        k_decode_jobs<CODEC><<<g, kDecodeWaves * kWave, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out, rd);
+}
+
+static int launch_decode_jobs(const DevIndex& d, const uint2* jobs, uint32_t nj, void* out, bool runs, hipStream_t s)
 {
     const uint32_t g = std::min<uint32_t>((nj + kDecodeWaves - 1) / kDecodeWaves, 65535);
-    const dim3 b(kDecodeWaves * kWave);
     switch (d.codec) {
-    case 1: k_decode_jobs<1><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 2: k_decode_jobs<2><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 3: k_decode_jobs<3><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 4: k_decode_jobs<4><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 5: k_decode_jobs<5><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 6: k_decode_jobs<6><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 7: k_decode_jobs<7><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 8: k_decode_jobs<8><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 9: k_decode_jobs<9><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 10: k_decode_jobs<10><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 11: k_decode_jobs<11><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 12: k_decode_jobs<12><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
-    case 13: k_decode_jobs<13><<<g, b, 0, s>>>(d.words, d.seg_cpos, d.seg_bph, jobs, nj, out); break;
+    case 1: launch_decode_t<1>(d, jobs, nj, out, runs, g, s); break;
+    case 2: launch_decode_t<2>(d, jobs, nj, out, runs, g, s); break;
+    case 3: launch_decode_t<3>(d, jobs, nj, out, runs, g, s); break;
+    case 4: launch_decode_t<4>(d, jobs, nj, out, runs, g, s); break;
+    case 5: launch_decode_t<5>(d, jobs, nj, out, runs, g, s); break;
+    case 6: launch_decode_t<6>(d, jobs, nj, out, runs, g, s); break;
+    case 7: launch_decode_t<7>(d, jobs, nj, out, runs, g, s); break;
+    case 8: launch_decode_t<8>(d, jobs, nj, out, runs, g, s); break;
+    case 9: launch_decode_t<9>(d, jobs, nj, out, runs, g, s); break;
+    case 10: launch_decode_t<10>(d, jobs, nj, out, runs, g, s); break;
+    case 11: launch_decode_t<11>(d, jobs, nj, out, runs, g, s); break;
+    case 12: launch_decode_t<12>(d, jobs, nj, out, runs, g, s); break;
+    case 13: launch_decode_t<13>(d, jobs, nj, out, runs, g, s); break;
     default: return fail(GENIE_E_INVALID, "unknown codec " + std::to_string(d.codec));
     }
     return GENIE_OK;
@@ -2503,13 +2593,17 @@ static int launch_scan(genie_plan* p, hipStream_t s)
     const uint64_t blocks = (uint64_t)a.n_tiles * ndq;
     if (blocks >= 0x7FFFFFFFull || nwork >= 0x7FFFFFFFull)
         return fail(GENIE_E_INVALID, "batch too large for one launch");
+    const bool runs = runs_used(p);
     if (p->dec_full) {
         // the batch's segments, each once, into the full-layout scratch; the
         // kernels below then read it as an uncompressed posting array
         const DevIndex& d = p->ix->d;
         const uint32_t nj = (uint32_t)p->h_fjobs.size();
-        if (nj)
-            if (int rc = launch_decode_jobs(d, p->d_fjobs, nj, p->d_full, s))
+        if (nj && runs)
+            if (int rc = launch_decode_jobs(d, p->d_fjobs, nj, p->d_runs, true, s))
+                return rc;
+        if (nj && (!runs || nwork))
+            if (int rc = launch_decode_jobs(d, p->d_fjobs, nj, p->d_full, false, s))
                 return rc;
         if (p->timing) {
             HIP_TRY(hipEventRecord(p->ev[5], s));
@@ -2534,7 +2628,7 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         } else if (p->dec_spans) {
             const uint32_t nj = (uint32_t)p->h_djobs.size();
             if (nj)
-                if (int rc = launch_decode_jobs(d, p->d_djobs, nj, p->d_scratch, s))
+                if (int rc = launch_decode_jobs(d, p->d_djobs, nj, p->d_scratch, false, s))
                     return rc;
             if (p->timing) {
                 HIP_TRY(hipEventRecord(p->ev[5], s));
@@ -2551,7 +2645,21 @@ static int launch_scan(genie_plan* p, hipStream_t s)
     if (ndq) {
         a.qlist = ndq == p->n_queries ? nullptr : p->d_dq;
         a.n_qlist = (uint32_t)ndq;
-        if (plain_sparse(p, a.n_tiles))
+        if (runs) {
+            const DevIndex& d = p->ix->d;
+            RunArgs ra;
+            ra.s = a;
+            ra.r = RunIndex{d.codec == 0 ? d.run_ids : p->d_runs, d.run_tf, d.n_keys, d.run_tiles};
+            ra.items = p->dec_full ? p->d_uitems : p->d_items;
+            ra.item_qptr = p->d_item_qptr;
+            ra.k0 = p->d_nchunks;  // k_item_keys
+            ra.k1 = p->d_chunk_ptr;
+            const uint32_t nb = (uint32_t)(d.run_tiles * ndq);
+            if (p->lane_bits == 8)
+                k_scan_runs<8><<<nb, kRunThreads, 0, s>>>(ra);
+            else
+                k_scan_runs<16><<<nb, kRunThreads, 0, s>>>(ra);
+        } else if (plain_sparse(p, a.n_tiles))
             launch_scan_t<true>(p->lane_bits, a, (uint32_t)blocks, s);
         else
             launch_scan_t<false>(p->lane_bits, a, (uint32_t)blocks, s);
@@ -2760,6 +2868,54 @@ static int settle_overflow(genie_plan* p, hipStream_t s)
     }
 }
 
+// Items into chunks and (chunk, key) pairs (or segment runs) for the hash
+// kernel and the direct-mapped kernels over the posting lists.
+static int launch_compile(genie_plan* p, hipStream_t s)
+{
+    const DevIndex& d = p->ix->d;
+    const uint32_t nq = p->n_queries;
+    const uint32_t ni = (uint32_t)p->n_items;
+    if (ni && (d.codec == 0 || p->dec_full)) {
+        const genie_dim_t* items = p->dec_full ? p->d_uitems : p->d_items;
+        k_chunk_count<<<(ni + 255) / 256, 256, 0, s>>>(items, ni, p->d_nchunks);
+        const uint32_t nb = (ni + 1023) / 1024;
+        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nchunks, p->d_chunk_ptr, ni, p->d_block_sums);
+        k_scan_sums<<<1, 256, 0, s>>>(p->d_block_sums, nb, p->d_total);
+        k_scan_add<<<nb, 256, 0, s>>>(p->d_chunk_ptr, ni, p->d_block_sums);
+        k_chunk_write<<<(ni + 255) / 256, 256, 0, s>>>(items, ni, p->d_chunk_ptr, d.key_start,
+                                                      d.n_keys, p->d_chunks);
+    } else if (ni) {
+        k_crun_flags<<<(ni + 255) / 256, 256, 0, s>>>(p->d_items, ni, d.seg_cpos, d.n_segments, p->d_nchunks);
+        const uint32_t nb = (ni + 1023) / 1024;
+        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nchunks, p->d_chunk_ptr, ni, p->d_block_sums);
+        k_scan_sums<<<1, 256, 0, s>>>(p->d_block_sums, nb, p->d_total);
+        k_scan_add<<<nb, 256, 0, s>>>(p->d_chunk_ptr, ni, p->d_block_sums);
+        k_crun_write<<<(ni + 255) / 256, 256, 0, s>>>(p->d_items, ni, d.seg_cpos, d.n_segments, d.seg_key,
+                                                     p->d_chunk_ptr, p->d_chunks);
+    } else {
+        fill_u32(p->d_total, 0, 1, s);
+    }
+    k_query_chunk_ptr<<<(nq + 1 + 255) / 256, 256, 0, s>>>(p->d_item_qptr, nq, p->d_chunk_ptr, ni,
+                                                          p->d_total, p->d_qc_ptr);
+    // pair prefix: every (chunk, key) pair gets a batch-wide position
+    if (p->n_chunks) {
+        const uint32_t nc = (uint32_t)p->n_chunks;
+        const uint32_t g = std::min<uint32_t>((nc + 255) / 256, 4096);
+        k_chunk_nkeys<<<g, 256, 0, s>>>(p->d_chunks, p->d_total, p->d_nk);
+        const uint32_t nb = (nc + 1023) / 1024;
+        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nk, p->d_kptr, nc, p->d_chunk_sums);
+        k_scan_sums<<<1, 256, 0, s>>>(p->d_chunk_sums, nb, p->d_total_pairs);
+        k_scan_add<<<nb, 256, 0, s>>>(p->d_kptr, nc, p->d_chunk_sums);
+        k_chunk_set_kp<<<g, 256, 0, s>>>(p->d_chunks, p->d_total, p->d_kptr);
+    } else {
+        fill_u32(p->d_total_pairs, 0, 1, s);
+    }
+    k_query_pair_ptr<<<(nq + 1 + 255) / 256, 256, 0, s>>>(p->d_qc_ptr, nq, p->d_kptr, p->d_total,
+                                                         p->d_total_pairs, p->d_qk_ptr);
+    HIP_TRY(hipGetLastError());
+    return GENIE_OK;
+}
+
 static int plan_run_once(genie_plan* p, hipStream_t s)
 {
     const DevIndex& d = p->ix->d;
@@ -2802,43 +2958,15 @@ static int plan_run_once(genie_plan* p, hipStream_t s)
     // segment runs (compressed); the kernels below write n_chunks chunks
     if (p->n_chunks > p->chunks_cap)
         return fail(GENIE_E_RUNTIME, "batch compiles into more chunks than the plan holds");
-    if (ni && (d.codec == 0 || p->dec_full)) {
-        const genie_dim_t* items = p->dec_full ? p->d_uitems : p->d_items;
-        k_chunk_count<<<(ni + 255) / 256, 256, 0, s>>>(items, ni, p->d_nchunks);
-        const uint32_t nb = (ni + 1023) / 1024;
-        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nchunks, p->d_chunk_ptr, ni, p->d_block_sums);
-        k_scan_sums<<<1, 256, 0, s>>>(p->d_block_sums, nb, p->d_total);
-        k_scan_add<<<nb, 256, 0, s>>>(p->d_chunk_ptr, ni, p->d_block_sums);
-        k_chunk_write<<<(ni + 255) / 256, 256, 0, s>>>(items, ni, p->d_chunk_ptr, d.key_start,
-                                                      d.n_keys, p->d_chunks);
-    } else if (ni) {
-        k_crun_flags<<<(ni + 255) / 256, 256, 0, s>>>(p->d_items, ni, d.seg_cpos, d.n_segments, p->d_nchunks);
-        const uint32_t nb = (ni + 1023) / 1024;
-        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nchunks, p->d_chunk_ptr, ni, p->d_block_sums);
-        k_scan_sums<<<1, 256, 0, s>>>(p->d_block_sums, nb, p->d_total);
-        k_scan_add<<<nb, 256, 0, s>>>(p->d_chunk_ptr, ni, p->d_block_sums);
-        k_crun_write<<<(ni + 255) / 256, 256, 0, s>>>(p->d_items, ni, d.seg_cpos, d.n_segments, d.seg_key,
-                                                     p->d_chunk_ptr, p->d_chunks);
-    } else {
-        fill_u32(p->d_total, 0, 1, s);
-    }
-    k_query_chunk_ptr<<<(nq + 1 + 255) / 256, 256, 0, s>>>(p->d_item_qptr, nq, p->d_chunk_ptr, ni,
-                                                          p->d_total, p->d_qc_ptr);
-    // pair prefix: every (chunk, key) pair gets a batch-wide position
-    if (p->n_chunks) {
-        const uint32_t nc = (uint32_t)p->n_chunks;
-        const uint32_t g = std::min<uint32_t>((nc + 255) / 256, 4096);
-        k_chunk_nkeys<<<g, 256, 0, s>>>(p->d_chunks, p->d_total, p->d_nk);
-        const uint32_t nb = (nc + 1023) / 1024;
-        k_scan_blocks<<<nb, 256, 0, s>>>(p->d_nk, p->d_kptr, nc, p->d_chunk_sums);
-        k_scan_sums<<<1, 256, 0, s>>>(p->d_chunk_sums, nb, p->d_total_pairs);
-        k_scan_add<<<nb, 256, 0, s>>>(p->d_kptr, nc, p->d_chunk_sums);
-        k_chunk_set_kp<<<g, 256, 0, s>>>(p->d_chunks, p->d_total, p->d_kptr);
-    } else {
-        fill_u32(p->d_total_pairs, 0, 1, s);
-    }
-    k_query_pair_ptr<<<(nq + 1 + 255) / 256, 256, 0, s>>>(p->d_qc_ptr, nq, p->d_kptr, p->d_total,
-                                                         p->d_total_pairs, p->d_qk_ptr);
+    // chunks are read by the hash kernel and by the direct-mapped kernels over
+    // the posting lists; the scan over runs takes the items and their keys
+    const bool runs = runs_used(p), chunks = !runs || !p->h_hwork.empty();
+    if (chunks)
+        if (int rc = launch_compile(p, s))
+            return rc;
+    if (runs && ni)  // in the chunk kernels' scratch, which they are done with
+        k_item_keys<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, d.key_start, d.n_keys,
+                                                     p->d_nchunks, p->d_chunk_ptr);
     if (p->timing)
         HIP_TRY(hipEventRecord(p->ev[1], s));
     if (int rc = launch_scan(p, s))
@@ -2972,6 +3100,11 @@ int genie_hip_plan_set_sparse(genie_plan* p, int mode)
         return fail(GENIE_E_INVALID, "sparse select mode must be -1, 0 or 1");
     plan_drop_graph(p);
     p->sparse_mode = mode;
+    if (p->n_queries && !lane_form(p) && !dense_active(p)) {  // a compressed batch's decode goes where its kernel reads
+        if (int rc = plan_split_plain(p))
+            return rc;
+        return plan_size_candidates(p);
+    }
     return GENIE_OK;
 }
 

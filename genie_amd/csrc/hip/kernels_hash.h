@@ -39,12 +39,22 @@ struct HashArgs {
 // other; or every segment a batch names, once, at its own posting positions
 // (a scratch of the uncompressed layout).  Segments were validated at index
 // creation.
-template <int CODEC>
+// RUNS: `out` is a tile-major copy (kernels_runs.h): the destination offset is
+// the segment's posting position, and each id goes to its key's run in its
+// tile as 16 bits; a segment whose ids share one tile shifts as a whole.
+struct RunDst {
+    const uint2* tf;
+    const uint32_t *seg_key, *seg_first, *seg_last;
+    uint32_t n_keys;
+};
+
+template <int CODEC, bool RUNS = false>
 __global__ void __launch_bounds__(kDecodeWaves * kWave) __attribute__((amdgpu_waves_per_eu(5)))
     k_decode_jobs(const uint32_t* __restrict__ words, const uint32_t* __restrict__ cpos,
                   const uint4* __restrict__ bph, const uint2* __restrict__ jobs, uint32_t n_jobs,
-                  uint32_t* __restrict__ out)
+                  void* __restrict__ dst, RunDst rd)
 {
+    uint32_t* out = static_cast<uint32_t*>(dst);
     __shared__ DecodeScratch S[kDecodeWaves];
     static_assert(sizeof(DecodeScratch) >= kWave * (kPerLane + 1) * 4, "transpose fits the scratch");
     const int wv = threadIdx.x / kWave, lane = lane_id();
@@ -67,6 +77,7 @@ __global__ void __launch_bounds__(kDecodeWaves * kWave) __attribute__((amdgpu_wa
     for (; j < n_jobs; j += stride) {
         const uint32_t nw = __builtin_amdgcn_readfirstlane(w1 - w0);
         const uint32_t out0 = __builtin_amdgcn_readfirstlane(jb.y);
+        const uint32_t sg = __builtin_amdgcn_readfirstlane(jb.x);
         stage_words_rs(S[wv], words, __builtin_amdgcn_readfirstlane(w0), nw);
         const uint4 hdr = hd;
         if (j + stride < n_jobs) {
@@ -89,6 +100,26 @@ __global__ void __launch_bounds__(kDecodeWaves * kWave) __attribute__((amdgpu_wa
         for (int k = 0; k < kPerLane; ++k)
             t[lane * (kPerLane + 1) + k] = v[k];
         wave_sync();
+        if constexpr (RUNS) {
+            uint16_t* ids = static_cast<uint16_t*>(dst);
+            const uint32_t key = __builtin_amdgcn_readfirstlane(rd.seg_key[sg]);
+            const uint32_t t0 = __builtin_amdgcn_readfirstlane(rd.seg_first[sg]) >> 16;
+            const uint32_t t1 = __builtin_amdgcn_readfirstlane(rd.seg_last[sg]) >> 16;
+            const uint2 f0 = rd.tf[(uint64_t)t0 * rd.n_keys + key];
+#pragma unroll
+            for (int k = 0; k < kPerLane; ++k) {
+                const uint32_t i = (uint32_t)k * kWave + lane;
+                if (i < n) {
+                    const uint32_t id = t[(i / kPerLane) * (kPerLane + 1) + i % kPerLane];
+                    uint2 f = f0;
+                    if (t0 != t1)  // uniform
+                        f = rd.tf[(uint64_t)(id >> 16) * rd.n_keys + key];
+                    ids[f.x + (out0 + i - f.y)] = (uint16_t)id;
+                }
+            }
+            wave_sync();  // the scratch is reused by the next job
+            continue;
+        }
         const __amdgpu_buffer_rsrc_t ro =
             __builtin_amdgcn_make_buffer_rsrc(out + out0, (short)0, (int)(n * 4u), 0x00020000);
 #pragma unroll

@@ -1,0 +1,99 @@
+"""Direct-mapped scan over tile-major runs (the plain form's dense select on
+indexes with long lists) against the oracle's search of the same work items:
+tile edges, items that start and end inside keys, 8- and 16-bit counters,
+ties trimmed and tiles with fewer than k matches, set-valued tables, and
+compressed tables, whose batches are decoded tile-major (with hash-form
+queries in the same batch, also into the posting lists' layout)."""
+import numpy as np
+import pytest
+
+from helpers import assert_topk_equal, oracle_search_sample, posting_items
+
+import genie_amd
+from genie_amd import Plan, Table, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def check(table, items, uitems, n, nq, k, where, hash_mode=0, graph=False):
+    p = Plan(table.device(), nq, max(1, len(items)), int(np.max(k)), 0, mode=0)
+    p.set_hash(hash_mode)
+    p.set_sparse(0)
+    p.upload(items, nq, k)
+    assert not p.sparse_active()
+    p.set_graph(graph)
+    oi, oc = oracle_search_sample(table.export()["inv"].view(np.uint32), uitems, n, np.broadcast_to(k, (nq,)),
+                                  np.arange(nq))
+    for _ in range(3 if graph else 1):
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, nq, where)
+    return p
+
+
+def clip(items, rng):
+    """Items cut at random positions: they start and end inside keys."""
+    out = items.copy()
+    span = out["end_pos"] - out["start_pos"]
+    out["start_pos"] += (rng.random(len(out)) * span * 0.4).astype(np.int32)
+    out["end_pos"] -= (rng.random(len(out)) * span * 0.4).astype(np.int32)
+    return out
+
+
+@pytest.mark.parametrize("n,d,values,radius,wmax,k", [
+    (65_535, 9, 300, 6, 1, 50),
+    (65_536, 130, 40, 3, 1, 7),      # more items than one window of 64 a query
+    (65_537, 12, 700, 40, 1, 3000),  # k above the last tile's objects
+    (200_003, 20, 256, 2, 40, 100),  # counts past 255: 16-bit counters
+    (131_072, 3, 64, 0, 1, 4096),    # few distinct counts: long ties
+    (140_000, 70, 90, 20, 900, 33),  # 16-bit counts in several histogram windows
+])
+def test_runs_equal_oracle(n, d, values, radius, wmax, k):
+    q = 7
+    rows = genie_amd.synth.rows(n + d, n, d, genie_amd.synth.ZIPF_PERM, 0.4, 0.0, 0, values - 1, values)
+    qv, _ = genie_amd.synth.queries(n + 1, rows, q, noise=radius, lo=0, hi=values - 1)
+    w = genie_amd.synth.uniform_int(n + 2, 0, q * d, 1, wmax)
+    t = Table.from_rows(rows)
+    items = t.compile(W.single_ranges(qv, radius, w), q)
+    items = items[items["query"] != 3]  # a query without items
+    check(t, items, items, n, q, k, "whole keys", graph=True)
+    cut = clip(items, np.random.default_rng(n))
+    check(t, cut, cut, n, q, k, "clipped")
+
+
+@pytest.mark.parametrize("codec", [5, 11, 13])
+@pytest.mark.parametrize("n", [65_600, 300_001])
+def test_runs_compressed(n, codec):
+    d, q = 24, 9
+    rows = genie_amd.synth.rows(77, n, d, genie_amd.synth.ZIPF_PERM, 1.1, 0.0, 0, 255, 256)
+    qv, _ = genie_amd.synth.queries(78, rows, q, noise=2, lo=0, hi=255)
+    r = W.single_ranges(qv, np.where(np.arange(q) < 6, 3, 0).astype(np.int32))
+    r = r[(r["query"] < 6) | (r["dim"] == 0)].copy()  # the last three: one exact value each
+    rare = np.argsort(np.bincount(rows[:, 0], minlength=256))[100:103]
+    r["low"][r["query"] >= 6] = rare
+    r["up"][r["query"] >= 6] = rare
+    t = Table.from_rows(rows, 1024, True, codec=codec)
+    k = np.array([5, 100, 700, 20, 1, 64, 30, 400, 3], np.uint32)
+    for merge in (False, True):
+        items = t.compile(r, q, merge_runs=merge)
+        u = posting_items(t.export(), items)
+        p = check(t, items, u, n, q, k, f"codec {codec}", hash_mode=0)
+        assert p.decode_active()
+        p = check(t, items, u, n, q, k, f"codec {codec} with hash-form queries", hash_mode=-1)
+        assert 0 < p.hash_queries() < q
+        p.set_sparse(1)  # the posting lists' layout for every query
+        p.run()
+        a = p.download()
+        p.set_sparse(0)
+        p.run()
+        b = p.download()
+        assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1])
+
+
+def test_runs_sets():
+    n, q = 90_000, 12
+    rp, v = genie_amd.synth.sets(5, n, 3, 30, 300, 0.6)
+    qp, qv = genie_amd.synth.sets(6, q, 1, 40, 300, 0.6)
+    t = Table.from_sets(rp, v)
+    items = t.compile(W.set_ranges(qp, qv, genie_amd.synth.uniform_int(7, 0, len(qv), 1, 9)), q)
+    check(t, items, items, n, q, 60, "sets")
