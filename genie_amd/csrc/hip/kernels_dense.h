@@ -273,7 +273,11 @@ __global__ void __launch_bounds__(256) k_dense_thresh(const uint32_t* __restrict
     auto largest = [&](uint32_t need) {
         return s3 >= need ? b + 3 : (s2 >= need ? b + 2 : (s1 >= need ? b + 1 : (s0 >= need ? b : 0u)));
     };
-    const uint32_t safe = max(wave_max(largest(k)), 1u);
+    // With a shift, bin 0 (no higher bin reaches `need`) stands for the
+    // threshold 1, whose objects are counted in no bin of their own: at most
+    // the whole sample.
+    const uint32_t sh = hshift ? hshift[q] : 0u, least = sh ? 0u : 1u;
+    const uint32_t safe = max(wave_max(largest(k)), least);
     const uint32_t spec = max(wave_max(largest(j)), safe);
     // S(spec) and S(safe): from the lane holding that bin
     // (selects on the bits of c - b: a compare chain here becomes a table
@@ -286,11 +290,10 @@ __global__ void __launch_bounds__(256) k_dense_thresh(const uint32_t* __restrict
     const uint32_t at_spec = (uint32_t)__shfl((int)(spec >= b && spec < b + 4 ? s_of(spec) : 0u), (int)(spec / 4), kWave);
     const uint32_t at_safe = (uint32_t)__shfl((int)(safe >= b && safe < b + 4 ? s_of(safe) : 0u), (int)(safe / 4), kWave);
     if (lane == 0) {
-        const uint32_t sh = hshift ? hshift[q] : 0u;
         gthr[q] = max(spec << sh, 1u);
         gsafe[q] = max(safe << sh, 1u);
-        want[q] = dense_want(at_spec, k, ratio16, n_objects, mult);
-        want_safe[q] = dense_want(at_safe, k, ratio16, n_objects, mult);
+        want[q] = dense_want(spec ? at_spec : n_sample, k, ratio16, n_objects, mult);
+        want_safe[q] = dense_want(safe ? at_safe : n_sample, k, ratio16, n_objects, mult);
     }
 }
 
