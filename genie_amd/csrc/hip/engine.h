@@ -138,6 +138,16 @@ struct DevIndex {
     uint32_t* obj_perm = nullptr;   // [set_slots] object of each slot (kSetEmpty: none)
     uint32_t* blk_off = nullptr;    // [set_slots / 64 + 1] first word of each 64-slot block
     uint32_t* blk_key = nullptr;    // [blk_off[last]] keys + 1 (0: padding), column-major per block
+    // matrix form of the same tables (kernels_sets.h): hot keys as byte
+    // columns, mid keys tile-major, the other keys' postings as they are
+    bool sm = false;
+    uint32_t sm_tiles = 0, sm_mid = 0, sm_max_tail = 0;  // tiles, mid keys, longest tail list
+    uint8_t* sm_hot = nullptr;      // [sm_tiles * 2048][64]
+    uint16_t* sm_mid_ids = nullptr;
+    uint32_t* sm_mid_ptr = nullptr; // [sm_tiles * sm_mid + 1]
+    uint32_t* sm_post = nullptr;    // compressed tables: the postings (uncompressed tables read `post`)
+    std::vector<uint32_t> h_sm_class;  // [n_keys] hot column, kSmHot + mid rank, or kSmTail
+    std::vector<uint32_t> h_sm_slots;  // [sm_mid] slots of a (query, key) pair
     uint64_t bytes = 0;
     // host copies used for validation and count bounds
     std::vector<uint64_t> h_key_start;

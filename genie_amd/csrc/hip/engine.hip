@@ -19,6 +19,7 @@
 #include <algorithm>
 #include <atomic>
 #include <chrono>
+#include <cmath>
 #include <thread>
 #include <cstdio>
 #include <cstring>
@@ -36,6 +37,7 @@
 #include "kernels_dense.h"
 #include "kernels_hash.h"
 #include "kernels_runs.h"
+#include "kernels_sets.h"
 #include "wave.h"
 
 namespace gh {
@@ -218,6 +220,19 @@ struct genie_plan {
     uint32_t* d_sgptr = nullptr;
     uint32_t* d_sshift = nullptr;
     uint64_t sent_alloc = 0, smask_alloc = 0;
+    // set form on the matrix cores (kernels_sets.h)
+    bool sm_ok = false;              // the uploaded batch runs it
+    std::vector<uint8_t> h_sm_wq;    // [groups][32][64] hot weights
+    std::vector<uint2> h_sm_slots, h_sm_pairs;                       // mid slots, tail pairs
+    std::vector<uint32_t> h_sm_slot_ptr, h_sm_pair_ptr, h_sm_evbase; // per group
+    std::vector<uint32_t> h_sm_units8, h_sm_units16;                 // groups on byte counters, half groups on 16-bit ones
+    uint64_t sm_events = 0;
+    uint8_t* d_sm_wq = nullptr;
+    uint2 *d_sm_slots = nullptr, *d_sm_pairs = nullptr;
+    uint32_t *d_sm_slot_ptr = nullptr, *d_sm_pair_ptr = nullptr, *d_sm_evbase = nullptr, *d_sm_units8 = nullptr,
+             *d_sm_units16 = nullptr, *d_sm_events = nullptr, *d_sm_evptr = nullptr;
+    uint64_t sm_wq_alloc = 0, sm_slots_alloc = 0, sm_pairs_alloc = 0, sm_slot_ptr_alloc = 0, sm_pair_ptr_alloc = 0,
+             sm_evbase_alloc = 0, sm_units8_alloc = 0, sm_units16_alloc = 0, sm_events_alloc = 0, sm_evptr_alloc = 0;
     uint32_t dn_groups = 0;
     uint32_t* d_dtab = nullptr;      // [dn_groups][dpad * 256] query masks
     uint64_t dtab_alloc = 0;
@@ -335,6 +350,16 @@ static void plan_free_buffers(genie_plan* p)
     dev_free(p->d_uitems);
     dev_free(p->d_full);
     dev_free(p->d_runs);
+    dev_free(p->d_sm_wq);
+    dev_free(p->d_sm_slots);
+    dev_free(p->d_sm_pairs);
+    dev_free(p->d_sm_slot_ptr);
+    dev_free(p->d_sm_pair_ptr);
+    dev_free(p->d_sm_evbase);
+    dev_free(p->d_sm_units8);
+    dev_free(p->d_sm_units16);
+    dev_free(p->d_sm_events);
+    dev_free(p->d_sm_evptr);
 }
 
 // Count bound of every query: per (query, order) group the largest weight
@@ -485,6 +510,7 @@ int gh::validate_items(const DevIndex& d, const genie_dim_t* items, uint64_t n_i
 static bool dense_shape(const genie_index_desc* desc, std::vector<uint32_t>& key_base, std::vector<uint32_t>& per_dim);
 static int build_sets(const genie_index_desc* desc, DevIndex& d);
 static int build_runs(DevIndex& d, const uint32_t* post, bool copy);
+static int build_set_matrix(const genie_index_desc* desc, DevIndex& d);
 static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t* post, const uint32_t* key_start);
 
 // Compressed index: words, segment offsets, key -> segment map, per-segment
@@ -1068,13 +1094,13 @@ static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
     const bool ok = room(&cnt, n) && room(&pre, n) && room(&sums, nb) && room(&total, 1) && room(&tf, n + 1ull) &&
                     (!copy || room(&ids, d.n_postings + kRunPad));
     if (ok) {
-        k_run_first<<<(n + 255) / 256, 256>>>(post, d.key_start, d.n_keys, (uint32_t)nt, tf, cnt);
+        k_run_first<<<(n + 255) / 256, 256>>>(post, d.key_start, nullptr, d.n_keys, (uint32_t)nt, kRunTileLog, tf, cnt);
         k_scan_blocks<<<nb, 256>>>(cnt, pre, n, sums);
         k_scan_sums<<<1, 256>>>(sums, nb, total);
         k_scan_add<<<nb, 256>>>(pre, n, sums);
         k_run_start<<<n / 256 + 1, 256>>>(pre, n, (uint32_t)d.n_postings, tf);
         if (copy)
-            k_run_fill<<<d.n_keys, 256>>>(post, d.key_start, d.n_keys, tf, ids);
+            k_run_fill<<<d.n_keys, 256>>>(post, d.key_start, nullptr, d.n_keys, kRunTileLog, tf, ids);
         if ((e = hipGetLastError()) == hipSuccess)
             e = hipDeviceSynchronize();
     } else {
@@ -1184,6 +1210,112 @@ static int build_sets(const genie_index_desc* desc, DevIndex& d)
     d.blk_off = d_boff;
     d.blk_key = d_bkey;
     d.bytes += bytes;
+    return build_set_matrix(desc, d);
+}
+
+// The matrix form's copies of a set-valued table (kernels_sets.h): keys
+// classed by list length, the hot matrix and the mid keys' tile-major ids
+// built on the device.  An index of too many tiles, or a device without room,
+// has none; only device errors fail.
+static int build_set_matrix(const genie_index_desc* desc, DevIndex& d)
+{
+    const uint32_t K = d.n_keys;
+    const uint64_t nt = ((uint64_t)d.n_objects + kSmTile - 1) >> kSmTileLog;
+    if (nt > kSmMaxTiles)
+        return GENIE_OK;
+    auto len = [&](uint32_t k) { return desc->key_start[k + 1] - desc->key_start[k]; };
+    // hot: the longest lists with multiplicities that an i8 holds; mid: the
+    // next ones down to half an id per tile
+    std::vector<uint32_t> order;
+    for (uint32_t k = 0; k < K; ++k)
+        if (2 * len(k) >= nt)
+            order.push_back(k);
+    std::stable_sort(order.begin(), order.end(), [&](uint32_t a, uint32_t b) { return len(a) > len(b); });
+    d.h_sm_class.assign(K, kSmTail);
+    std::vector<uint32_t> hot, mid;
+    uint64_t n_mid_ids = 0;
+    for (uint32_t k : order) {
+        if (hot.size() < kSmHot && d.h_key_mult[k] <= kSmHotMult) {
+            d.h_sm_class[k] = (uint32_t)hot.size();
+            hot.push_back(k);
+        } else if (mid.size() < kSmMaxMid) {
+            d.h_sm_class[k] = kSmHot + (uint32_t)mid.size();
+            mid.push_back(k);
+            n_mid_ids += len(k);
+            // windows of 8 ids that a run of this key usually spans: its mean
+            // length, the mean offset of its start, 1.5 deviations
+            const double l = (double)len(k) / (double)nt;
+            d.h_sm_slots.push_back((uint32_t)std::max(1.0, std::ceil((l + 3.5 + 1.5 * std::sqrt(l)) / 8.0)));
+        }
+    }
+    d.sm_max_tail = 0;
+    for (uint32_t k = 0; k < K; ++k)
+        if (d.h_sm_class[k] == kSmTail)
+            d.sm_max_tail = std::max(d.sm_max_tail, (uint32_t)len(k));
+    if (n_mid_ids >= 1ull << 30) {  // the kernels read them through 32-bit byte offsets
+        d.h_sm_class.clear();
+        return GENIE_OK;
+    }
+    const uint32_t R = (uint32_t)mid.size(), n = (uint32_t)(nt * R), nb = (n + 1023) / 1024;
+    uint32_t *d_hot_keys = nullptr, *d_mid_keys = nullptr, *cnt = nullptr, *sums = nullptr, *total = nullptr;
+    uint2* tf = nullptr;
+    auto room = [](auto** p, uint64_t count) {
+        return hipMalloc((void**)p, std::max<uint64_t>(1, count) * sizeof(**p)) == hipSuccess;
+    };
+    hipError_t e = hipSuccess;
+    const uint64_t hot_bytes = nt * kSmTile * kSmHot;
+    const bool ok = room(&d_hot_keys, hot.size()) && room(&d_mid_keys, R) && room(&cnt, n) && room(&sums, nb) &&
+                    room(&total, 1) && room(&tf, n + 1ull) && room(&d.sm_hot, hot_bytes) &&
+                    room(&d.sm_mid_ids, n_mid_ids + kSmMidPad) && room(&d.sm_mid_ptr, n + 1ull) &&
+                    (d.codec == 0 || room(&d.sm_post, d.n_postings));
+    if (ok) {
+        const uint32_t* post = d.codec == 0 ? d.post : d.sm_post;
+        if (d.codec != 0)
+            e = hipMemcpy(d.sm_post, desc->postings, d.n_postings * 4, hipMemcpyHostToDevice);
+        if (!e)
+            e = hipMemset(d.sm_hot, 0, hot_bytes);
+        if (!e && !hot.empty())
+            e = hipMemcpy(d_hot_keys, hot.data(), hot.size() * 4, hipMemcpyHostToDevice);
+        if (!e && R)
+            e = hipMemcpy(d_mid_keys, mid.data(), R * 4ull, hipMemcpyHostToDevice);
+        const uint32_t last = (uint32_t)n_mid_ids;
+        if (!e)
+            e = hipMemcpy(d.sm_mid_ptr + n, &last, 4, hipMemcpyHostToDevice);
+        if (!e) {
+            if (!hot.empty())
+                k_set_hot<<<dim3((uint32_t)hot.size(), 64), 256>>>(post, d.key_start, d_hot_keys, d.sm_hot);
+            if (R) {
+                k_run_first<<<(n + 255) / 256, 256>>>(post, d.key_start, d_mid_keys, R, (uint32_t)nt, kSmTileLog, tf, cnt);
+                k_scan_blocks<<<nb, 256>>>(cnt, d.sm_mid_ptr, n, sums);
+                k_scan_sums<<<1, 256>>>(sums, nb, total);
+                k_scan_add<<<nb, 256>>>(d.sm_mid_ptr, n, sums);
+                k_run_start<<<n / 256 + 1, 256>>>(d.sm_mid_ptr, n, last, tf);
+                k_run_fill<<<R, 256>>>(post, d.key_start, d_mid_keys, R, kSmTileLog, tf, d.sm_mid_ids);
+            }
+            if ((e = hipGetLastError()) == hipSuccess)
+                e = hipDeviceSynchronize();
+        }
+    } else {
+        (void)hipGetLastError();
+    }
+    dev_free(d_hot_keys);
+    dev_free(d_mid_keys);
+    dev_free(cnt);
+    dev_free(sums);
+    dev_free(total);
+    dev_free(tf);
+    if (!ok || e) {
+        dev_free(d.sm_hot);
+        dev_free(d.sm_mid_ids);
+        dev_free(d.sm_mid_ptr);
+        dev_free(d.sm_post);
+        d.h_sm_class.clear();
+        return e ? fail(GENIE_E_RUNTIME, std::string("matrix form: ") + hipGetErrorString(e)) : GENIE_OK;
+    }
+    d.sm = true;
+    d.sm_tiles = (uint32_t)nt;
+    d.sm_mid = R;
+    d.bytes += hot_bytes + (n_mid_ids + kSmMidPad) * 2 + (n + 1ull) * 4 + (d.codec ? d.n_postings * 4 : 0);
     return GENIE_OK;
 }
 
@@ -1407,6 +1539,10 @@ int genie_hip_index_destroy(genie_index* ix)
     dev_free(d.obj_perm);
     dev_free(d.blk_off);
     dev_free(d.blk_key);
+    dev_free(d.sm_hot);
+    dev_free(d.sm_mid_ids);
+    dev_free(d.sm_mid_ptr);
+    dev_free(d.sm_post);
     delete ix;
     return GENIE_OK;
 }
@@ -1505,6 +1641,9 @@ int genie_hip_plan_estimate(const genie_index* ix, uint32_t n_queries, uint64_t 
     if (dense)  // query-mask tables per group (8 queries at the fewest) and the sample histograms
         b += (nq + 7) / 8 * (uint64_t)std::max<uint32_t>(d.dense_dpad, 1) * kDenseKeysPerDim * 4 +
              nq * kDenseBins * 4ull;
+    if (d.sm && mode != 0)  // matrix form: hot weights, window slots, tail postings sorted by tile
+        b += (nq + 31) / 32 * (32ull * kSmHot + (d.sm_tiles + 1ull) * 4) + ni * 32 +
+             std::min<uint64_t>(ni * d.sm_max_tail, kSmMaxEvents) * 4;
     if (d.codec != 0 && mode != 1)  // full-layout decode scratch of the plain form
         b += d.n_postings * 4;
     *bytes = b;
@@ -1609,6 +1748,9 @@ static int h2d(genie_plan* p, T** dst, const void* src, uint64_t bytes)
 // Mode 1 (batched) and mode 2 (automatic) run the dense form when the batch
 // allows it; otherwise mode 1 runs the lane form and mode 2 the plain form.
 static bool dense_active(const genie_plan* p) { return p->mode != 0 && p->dense_on && (p->dense_ok || p->sets_ok); }
+
+// Whether a set-form batch runs on the matrix cores.
+static bool sets_matrix(const genie_plan* p) { return !p->dense_ok && p->sm_ok; }
 
 // Queries of one group of the dense or set form: the bits of a mask word
 // over the weight planes per query.
@@ -1790,6 +1932,99 @@ static bool dense_batch_ok(genie_plan* p, uint32_t n_queries)
     return true;
 }
 
+// Gathers a set-valued batch for the matrix form, query by query: the hot
+// weights, a slot per window of the mid keys, the tail pairs, and whether the
+// counts that the scatter adds for a query fit a byte.
+struct SetMatrixBatch {
+    genie_plan* p;
+    const DevIndex& d;
+    uint32_t G, g = 0;
+    bool wide = false;  // some query of the group needs 16-bit counters
+    bool on;
+    std::vector<std::pair<uint32_t, uint32_t>> cold;  // weight, multiplicity
+    SetMatrixBatch(genie_plan* plan, uint32_t groups) : p(plan), d(plan->ix->d), G(groups), on(d.sm)
+    {
+        p->sm_ok = false;
+        p->h_sm_slots.clear();
+        p->h_sm_pairs.clear();
+        p->h_sm_units8.clear();
+        p->h_sm_units16.clear();
+        p->sm_events = 0;
+        if (on) {
+            p->h_sm_wq.assign((uint64_t)G * 32 * kSmHot, 0);
+            p->h_sm_slot_ptr.assign(G + 1, 0);
+            p->h_sm_pair_ptr.assign(G + 1, 0);
+            p->h_sm_evbase.assign(G, 0);
+        }
+    }
+    template <class KW>
+    void query(uint32_t j, const KW* b, const KW* e)
+    {
+        if (!on)
+            return;
+        cold.clear();
+        for (; b != e; ++b) {
+            const uint32_t c = d.h_sm_class[b->key];
+            if (c < kSmHot) {
+                p->h_sm_wq[((uint64_t)g * 32 + j) * kSmHot + c] = (uint8_t)b->w;
+                continue;
+            }
+            cold.push_back({b->w, d.h_key_mult[b->key]});
+            if (c == kSmTail) {
+                p->h_sm_pairs.push_back(make_uint2(b->key, j | b->w << 5));
+                p->sm_events += d.h_key_start[b->key + 1] - d.h_key_start[b->key];
+            } else {
+                const uint32_t n = d.h_sm_slots[c - kSmHot];
+                for (uint32_t i = 0; i < n; ++i)
+                    p->h_sm_slots.push_back(make_uint2((c - kSmHot) | j << 16 | b->w << 21, i | n << 16));
+            }
+        }
+        // an object holds at most set_max_len occurrences, each key's at most
+        // its multiplicity: the largest weights first
+        std::sort(cold.begin(), cold.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+        uint64_t bound = 0;
+        uint32_t left = d.set_max_len;
+        for (const auto& c : cold) {
+            const uint32_t m = std::min(left, c.second);
+            bound += (uint64_t)c.first * m;
+            left -= m;
+        }
+        wide |= bound > 255;
+    }
+    void group_end(uint32_t)
+    {
+        if (!on)
+            return;
+        p->h_sm_slot_ptr[g + 1] = (uint32_t)p->h_sm_slots.size();
+        p->h_sm_pair_ptr[g + 1] = (uint32_t)p->h_sm_pairs.size();
+        if (wide) {
+            p->h_sm_units16.push_back(2 * g);
+            p->h_sm_units16.push_back(2 * g + 1);
+        } else {
+            p->h_sm_units8.push_back(g);
+        }
+        if (p->sm_events > kSmMaxEvents)
+            on = false;
+        else if (g + 1 < G)
+            p->h_sm_evbase[g + 1] = (uint32_t)p->sm_events;
+        wide = false;
+        ++g;
+    }
+    // The matrix form costs a group and tile about 6,000 CU cycles whatever the
+    // documents hold, and 1,260 for every 512 window slots past the 1,024 that
+    // its workgroups keep in registers; the forward lists about 1,030 for every
+    // token of the mean document.  Skewed tables have few slots (2M documents,
+    // Zipf(1.05): 22.6 ms on the lists, 6.0 here); a uniform vocabulary of 300
+    // has 18,000 of them (1.4 ms on the lists, 3.0 here); they meet at 750 per
+    // token (uniform over 2,000: 1.73 and 1.70 ms).
+    bool finish() const
+    {
+        const double slots = (double)p->h_sm_slots.size() / std::max(1u, G);
+        const double mean_len = (double)d.n_postings / std::max(1u, d.n_objects);
+        return on && 1260.0 * (slots / kSmThreads - kSmSlots) <= 750.0 * mean_len;
+    }
+};
+
 // Whether the uploaded batch can run the set form (set-valued tables with
 // forward lists): per query, the sum of its items' weights over the
 // positions (items may repeat a key, or split it into segments or chunks) is
@@ -1819,6 +2054,7 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
     p->h_smask.clear();
     p->h_sgptr.assign(G + 1, 0);
     p->h_sshift.assign(n_queries, 0);
+    SetMatrixBatch sm(p, G);
     for (uint32_t g = 0; g < G; ++g) {
         gk.clear();
         for (uint32_t q = g * 32; q < std::min(n_queries, g * 32 + 32); ++q) {
@@ -1871,7 +2107,9 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
             while ((bound >> sh) > 255)
                 ++sh;
             p->h_sshift[q] = sh;
+            sm.query(q - g * 32, gk.data() + first, gk.data() + gk.size());
         }
+        sm.group_end(g);
         std::sort(gk.begin(), gk.end(), [](const KW& x, const KW& y) { return x.key < y.key; });
         for (size_t i = 0; i < gk.size();) {
             uint32_t m[8] = {};
@@ -1887,6 +2125,7 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
             return false;
         p->h_sgptr[g + 1] = (uint32_t)p->h_skeys.size();
     }
+    p->sm_ok = sm.finish();
     return true;
 }
 
@@ -1898,8 +2137,10 @@ static int prepare_dense(genie_plan* p)
     const DevIndex& d = p->ix->d;
     p->dn_groups = (p->n_queries + dense_qpg(p) - 1) / dense_qpg(p);
     const uint64_t tw = (uint64_t)d.dense_dpad * kDenseKeysPerDim;
-    if (int rc = grow_buf(p, &p->d_dtab, &p->dtab_alloc, p->dn_groups * tw))
-        return rc;
+    if (p->dense_ok) {
+        if (int rc = grow_buf(p, &p->d_dtab, &p->dtab_alloc, p->dn_groups * tw))
+            return rc;
+    }
     if (!p->d_dhist)
         if (int rc = dev_alloc(&p->d_dhist, (uint64_t)p->max_queries * kDenseBins))
             return rc;
@@ -1917,6 +2158,29 @@ static int prepare_dense(genie_plan* p)
             if (int rc = h2d(p, &p->d_sshift, p->h_sshift.data(), p->h_sshift.size() * 4))
                 return rc;
         }
+    } else if (p->sm_ok) {  // set form on the matrix cores
+        auto put = [&](auto** buf, uint64_t* alloc, const auto& v) -> int {
+            if (int rc = grow_buf(p, buf, alloc, std::max<uint64_t>(1, v.size())))
+                return rc;
+            return h2d(p, buf, v.data(), v.size() * sizeof(v[0]));
+        };
+        int rc = 0;
+        if ((rc = put(&p->d_sm_wq, &p->sm_wq_alloc, p->h_sm_wq)) ||
+            (rc = put(&p->d_sm_slots, &p->sm_slots_alloc, p->h_sm_slots)) ||
+            (rc = put(&p->d_sm_pairs, &p->sm_pairs_alloc, p->h_sm_pairs)) ||
+            (rc = put(&p->d_sm_slot_ptr, &p->sm_slot_ptr_alloc, p->h_sm_slot_ptr)) ||
+            (rc = put(&p->d_sm_pair_ptr, &p->sm_pair_ptr_alloc, p->h_sm_pair_ptr)) ||
+            (rc = put(&p->d_sm_evbase, &p->sm_evbase_alloc, p->h_sm_evbase)) ||
+            (rc = put(&p->d_sm_units8, &p->sm_units8_alloc, p->h_sm_units8)) ||
+            (rc = put(&p->d_sm_units16, &p->sm_units16_alloc, p->h_sm_units16)) ||
+            (rc = grow_buf(p, &p->d_sm_events, &p->sm_events_alloc, std::max<uint64_t>(1, p->sm_events))) ||
+            (rc = grow_buf(p, &p->d_sm_evptr, &p->sm_evptr_alloc, p->dn_groups * (d.sm_tiles + 1ull))))
+            return rc;
+        if (!p->d_sshift)
+            if ((rc = dev_alloc(&p->d_sshift, p->max_queries)))
+                return rc;
+        if ((rc = h2d(p, &p->d_sshift, p->h_sshift.data(), p->h_sshift.size() * 4)))
+            return rc;
     } else {  // set form: the groups' key entries
         const uint64_t ne = std::max<uint64_t>(1, p->h_skeys.size());
         if (int rc = grow_buf(p, &p->d_skeys, &p->sent_alloc, ne))
@@ -2746,6 +3010,84 @@ static int launch_dense(uint32_t nblk, const DenseArgs& a, hipStream_t s, int nt
     return launch_dense_w<SAMPLE, 1>(nblk, a, s, nt);
 }
 
+// One pass of the matrix form: over the sample tiles, or over all of them.
+// Units (groups, half groups) times chunks of the tiles, chunk-major, so that
+// the workgroups in flight read the same tiles; as many chunks as give every
+// resident workgroup several blocks and the last wave of blocks the least idle
+// share.
+template <bool SAMPLE, bool W16>
+static int launch_sets_t(SetArgs a, const uint32_t* units, uint32_t n_units, hipStream_t s)
+{
+    if (n_units == 0)
+        return GENIE_OK;
+    int dev = 0, n_cu = 0;
+    HIP_TRY(hipGetDevice(&dev));
+    HIP_TRY(hipDeviceGetAttribute(&n_cu, hipDeviceAttributeMultiprocessorCount, dev));
+    const uint32_t resident = (uint32_t)n_cu * (SAMPLE ? 1u : 2u);  // workgroups whose LDS fits the CUs
+    const uint32_t tiles = SAMPLE ? a.n_list * (kDenseTile / kSmTile) : a.n_tiles;
+    // chunks of about 16 tiles keep the workgroups of an XCD within the tiles
+    // that its L2 holds (their pace differs with their queries): 2M documents,
+    // 512 groups, 5.95 ms, against 6.28 at 32 tiles, 7.90 at 96 and 6.08 at 8; fewer tiles
+    // where there are not enough units to fill the chip, 4 at least, since a
+    // block sets up its table and pipeline once
+    const uint32_t cmax = std::max(1u, tiles / (SAMPLE ? 2u : 4u));
+    const uint32_t lo = std::min(cmax, std::max({1u, SAMPLE ? 1u : tiles / 16u, (2 * resident + n_units - 1) / n_units}));
+    uint32_t best = lo;
+    double waste = 1e9;
+    for (uint32_t c = lo; c <= std::min(cmax, lo + lo / 2 + 2); ++c) {
+        const double waves = (double)n_units * c / resident, w = std::ceil(waves) / waves;
+        if (w < waste - 0.01) {
+            waste = w;
+            best = c;
+        }
+    }
+    a.units = units;
+    a.n_units = n_units;
+    a.chunks = best;
+    k_set_count<SAMPLE, W16><<<n_units * best, kSmThreads, 0, s>>>(a);
+    return GENIE_OK;
+}
+
+template <bool SAMPLE>
+static int launch_sets(const genie_plan* p, const SetArgs& a, hipStream_t s)
+{
+    if (int rc = launch_sets_t<SAMPLE, false>(a, p->d_sm_units8, (uint32_t)p->h_sm_units8.size(), s))
+        return rc;
+    return launch_sets_t<SAMPLE, true>(a, p->d_sm_units16, (uint32_t)p->h_sm_units16.size(), s);
+}
+
+static SetArgs set_args(const genie_plan* p)
+{
+    const DevIndex& d = p->ix->d;
+    SetArgs a{};
+    a.hot = d.sm_hot;
+    a.mid_ids = d.sm_mid_ids;
+    a.mid_ptr = d.sm_mid_ptr;
+    a.n_mid = d.sm_mid;
+    a.n_tiles = d.sm_tiles;
+    a.n_objects = d.n_objects;
+    a.G = p->dn_groups;
+    a.n_queries = p->n_queries;
+    a.wq = p->d_sm_wq;
+    a.slots = p->d_sm_slots;
+    a.slot_ptr = p->d_sm_slot_ptr;
+    a.events = p->d_sm_events;
+    a.ev_base = p->d_sm_evbase;
+    a.ev_ptr = p->d_sm_evptr;
+    a.list = p->d_dlist;
+    a.n_list = p->n_dlist;
+    a.gthr = p->d_gthr;
+    a.redo = nullptr;
+    a.hist = p->d_dhist;
+    a.hshift = p->d_sshift;
+    a.cand_cnt = p->d_cand_cnt;
+    a.cand_cap = p->d_cand_cap;
+    a.cand_base = p->d_cand_base;
+    a.cand = p->d_cand;
+    a.overflow = p->d_overflow;
+    return a;
+}
+
 // Dense form: query masks, sample pass + thresholds, main pass, merge.
 static int run_dense(genie_plan* p, hipStream_t s)
 {
@@ -2788,8 +3130,18 @@ static int run_dense(genie_plan* p, hipStream_t s)
     a.set_gptr = p->d_sgptr;
     a.hshift = (p->dense_ok && p->dense_wp == 1) ? nullptr : p->d_sshift;
     const uint32_t nblk = p->dense_ok ? d.dense_dpad / 16 : 0;  // 0: the set form
-    if (int rc = launch_dense<true>(nblk, a, s, p->dense_nt, p->dense_wp))
+    const bool sm = sets_matrix(p);
+    SetArgs sa{};
+    if (sm) {
+        sa = set_args(p);
+        k_set_events<<<p->dn_groups, 1024, 0, s>>>(d.codec == 0 ? d.post : d.sm_post, d.key_start, p->d_sm_pairs,
+                                                   p->d_sm_pair_ptr, d.sm_tiles, p->d_sm_evbase, p->d_sm_evptr,
+                                                   p->d_sm_events);
+        if (int rc = launch_sets<true>(p, sa, s))
+            return rc;
+    } else if (int rc = launch_dense<true>(nblk, a, s, p->dense_nt, p->dense_wp)) {
         return rc;
+    }
     // thresholds, then every query's candidate space from its sample
     const uint32_t mult = p->dense_mult;
     const uint32_t ratio16 = (uint32_t)std::min<uint64_t>(
@@ -2802,7 +3154,7 @@ static int run_dense(genie_plan* p, hipStream_t s)
         HIP_TRY(hipEventRecord(p->ev[4], s));
     a.list = nullptr;
     a.n_list = 0;
-    if (int rc = launch_dense<false>(nblk, a, s, p->dense_nt, p->dense_wp))
+    if (int rc = sm ? launch_sets<false>(p, sa, s) : launch_dense<false>(nblk, a, s, p->dense_nt, p->dense_wp))
         return rc;
     // queries the speculative threshold left short: their groups again
     k_dense_check<<<p->dn_groups, 64, 0, s>>>(p->d_kq, nq, p->d_gthr, p->d_gsafe, p->d_cand_cnt, p->d_redo,
@@ -2810,8 +3162,8 @@ static int run_dense(genie_plan* p, hipStream_t s)
                                               p->total_cap,
                                               (p->dense_ok && p->dense_wp == 1) ? kDenseNoQuery : kSetNoQuery,
                                               dense_qpg(p));
-    a.redo = p->d_redo;
-    if (int rc = launch_dense<false>(nblk, a, s, p->dense_nt, p->dense_wp))
+    a.redo = sa.redo = p->d_redo;
+    if (int rc = sm ? launch_sets<false>(p, sa, s) : launch_dense<false>(nblk, a, s, p->dense_nt, p->dense_wp))
         return rc;
     if (p->timing)
         HIP_TRY(hipEventRecord(p->ev[2], s));

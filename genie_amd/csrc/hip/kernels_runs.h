@@ -34,17 +34,19 @@ struct RunIndex {
 
 // ---- index creation --------------------------------------------------------
 
-// One thread per (tile, key): the position of the key's first id at or past
-// the tile, and (cnt) the ids the key holds in the tile.
+// One thread per (tile of 2^log objects, key): the position of the key's first
+// id at or past the tile, and (cnt) the ids the key holds in the tile.  `keys`:
+// the keys of the copy (null: all n_keys of the index).
 __global__ void __launch_bounds__(256) k_run_first(const uint32_t* __restrict__ post,
-                                                   const uint32_t* __restrict__ key_start, uint32_t n_keys,
-                                                   uint32_t n_tiles, uint2* __restrict__ tf,
+                                                   const uint32_t* __restrict__ key_start,
+                                                   const uint32_t* __restrict__ keys, uint32_t n_keys,
+                                                   uint32_t n_tiles, uint32_t log, uint2* __restrict__ tf,
                                                    uint32_t* __restrict__ cnt)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
     if (i >= n_keys * n_tiles)
         return;
-    const uint32_t t = i / n_keys, k = i % n_keys;
+    const uint32_t t = i / n_keys, k = keys ? keys[i % n_keys] : i % n_keys;
     const uint32_t s = key_start[k], e = key_start[k + 1];
     auto first_at = [&](uint64_t target) {
         uint32_t lo = s, hi = e;
@@ -57,7 +59,7 @@ __global__ void __launch_bounds__(256) k_run_first(const uint32_t* __restrict__ 
         }
         return lo;
     };
-    const uint32_t a = first_at((uint64_t)t << kRunTileLog), b = first_at((uint64_t)(t + 1) << kRunTileLog);
+    const uint32_t a = first_at((uint64_t)t << log), b = first_at((uint64_t)(t + 1) << log);
     tf[i].y = a;
     cnt[i] = b - a;
 }
@@ -73,16 +75,17 @@ __global__ void __launch_bounds__(256) k_run_start(const uint32_t* __restrict__ 
         tf[i] = make_uint2(total, total);
 }
 
-// One workgroup per key: its ids to their runs.
+// One workgroup per key: its ids within the tiles (log <= 16) to their runs.
 __global__ void __launch_bounds__(256) k_run_fill(const uint32_t* __restrict__ post,
-                                                  const uint32_t* __restrict__ key_start, uint32_t n_keys,
+                                                  const uint32_t* __restrict__ key_start,
+                                                  const uint32_t* __restrict__ keys, uint32_t n_keys, uint32_t log,
                                                   const uint2* __restrict__ tf, uint16_t* __restrict__ ids)
 {
-    const uint32_t k = blockIdx.x;
+    const uint32_t r = blockIdx.x, k = keys ? keys[r] : r;
     for (uint32_t p = key_start[k] + threadIdx.x; p < key_start[k + 1]; p += blockDim.x) {
         const uint32_t o = post[p];
-        const uint2 f = tf[(uint64_t)(o >> kRunTileLog) * n_keys + k];
-        ids[f.x + (p - f.y)] = (uint16_t)o;
+        const uint2 f = tf[(uint64_t)(o >> log) * n_keys + r];
+        ids[f.x + (p - f.y)] = (uint16_t)(o & ((1u << log) - 1u));
     }
 }
 

@@ -1,0 +1,67 @@
+"""Set form on the matrix cores (hot keys as a product, mid keys scattered from
+tile-major windows, tail keys from postings sorted by tile) against the
+oracle's search of the same items: tile edges, byte and 16-bit counters,
+repeated tokens, multiplicities an i8 does not hold, keys of one class only,
+partial groups, compressed tables, graph replays."""
+import numpy as np
+import pytest
+
+from helpers import assert_topk_equal, oracle_search_sample, posting_items
+
+import genie_amd
+from genie_amd import Plan, Table, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("n,q,vocab,skew,wmax,k", [
+    (2047, 33, 200, 1.05, 1, 10),        # one tile, one object short of it; a group of one query
+    (2048, 5, 3000, 1.05, 3, 2048),      # k = every object
+    (2049, 32, 60, 0.5, 2, 100),         # every key hot
+    (70_001, 70, 40_000, 1.05, 4, 50),   # hot, mid and tail keys
+    (70_001, 40, 40_000, 1.05, 60, 50),  # 16-bit counters
+    (30_000, 100, 30_000, 0.0, 1, 20),   # a flat vocabulary: short runs, many ties
+])
+@pytest.mark.parametrize("codec", [0, 11])
+def test_matrix_form_equals_oracle(n, q, vocab, skew, wmax, k, codec):
+    rp, v = genie_amd.synth.sets(n, n, 3, 30, vocab, skew)
+    qp, qv = genie_amd.synth.sets(n + 1, q, 1, 40, vocab, skew)
+    w = genie_amd.synth.uniform_int(n + 2, 0, len(qv), 1, wmax)
+    if wmax > 50:  # a token named twice may not pass the largest weight per key
+        _, first = np.unique(np.repeat(np.arange(q), np.diff(qp)) * vocab + qv, return_index=True)
+        keep = np.zeros(len(qv), bool)
+        keep[first] = True
+        cnt = np.add.reduceat(keep.astype(np.int64), qp[:-1])
+        qp, qv, w = np.concatenate([[0], np.cumsum(cnt)]), qv[keep], w[keep]
+    t = Table.from_sets(rp, v, **(dict(max_length=1024, load_balance=True, codec=codec) if codec else {}))
+    check(t, W.set_ranges(qp, qv, w), n, q, k, codec)
+
+
+def test_matrix_form_multiplicities():
+    """The most frequent token 200 times in some documents: not an i8 column."""
+    rng = np.random.default_rng(3)
+    docs = [np.sort(rng.integers(0, 500, rng.integers(3, 20))) for _ in range(5000)]
+    for i in range(0, 5000, 97):
+        docs[i] = np.concatenate([np.full(200, 7), docs[i]])
+    rp = np.concatenate([[0], np.cumsum([len(x) for x in docs])]).astype(np.int64)
+    t = Table.from_sets(rp, np.concatenate(docs).astype(np.int32))
+    q = 20
+    qv = [np.unique(np.append(rng.integers(0, 500, 15), 7 if j % 2 else 3)) for j in range(q)]
+    qp = np.concatenate([[0], np.cumsum([len(x) for x in qv])])
+    flat = np.concatenate(qv).astype(np.int32)
+    check(t, W.set_ranges(qp, flat, rng.integers(1, 9, len(flat))), 5000, q, 30, 0)
+
+
+def check(t, ranges, n, q, k, codec):
+    items = t.compile(ranges, q, merge_runs=bool(codec))
+    export = t.export()
+    u = posting_items(export, items) if codec else items
+    oi, oc = oracle_search_sample(export["inv"].view(np.uint32), u, n, np.full(q, k), np.arange(q))
+    p = Plan(t.device(), q, len(items), k, 0, mode=2)
+    p.upload(items, q, np.full(q, k, np.uint32))
+    assert p.form() == "set"
+    p.set_graph(True)
+    for _ in range(3):
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, q, f"n={n}")
