@@ -37,6 +37,7 @@
 #include "kernels_dense.h"
 #include "kernels_hash.h"
 #include "kernels_runs.h"
+#include "kernels_filter.h"
 #include "kernels_sets.h"
 #include "wave.h"
 
@@ -129,6 +130,9 @@ struct genie_plan {
     bool plain_stats = false;             // h_qpost / h_qbound hold this batch's figures
     uint32_t* d_hwork = nullptr;
     uint64_t hwork_alloc = 0;
+    std::vector<uint32_t> h_fwork, h_fq;  // (query, tile) of the filter kernel, its queries
+    uint32_t *d_fwork = nullptr, *d_fq = nullptr;
+    uint64_t fwork_alloc = 0, fq_alloc = 0;
     uint4* d_hq = nullptr;
     uint32_t* d_dq = nullptr;
     uint32_t* d_hov = nullptr;
@@ -334,6 +338,8 @@ static void plan_free_buffers(genie_plan* p)
     dev_free(p->d_cap_used);
     dev_free(p->d_dkeys);
     dev_free(p->d_hwork);
+    dev_free(p->d_fwork);
+    dev_free(p->d_fq);
     dev_free(p->d_hq);
     dev_free(p->d_dq);
     dev_free(p->d_hov);
@@ -2408,7 +2414,7 @@ static int plan_full_decode(genie_plan* p)
     if (tiled && !p->d_runs)
         if (dev_alloc(&p->d_runs, d.n_postings + kRunPad) != GENIE_OK)
             return GENIE_OK;  // no room for the scratch: in-kernel decode
-    if ((!tiled || !p->h_hwork.empty()) && !p->d_full)
+    if ((!tiled || !p->h_hwork.empty() || !p->h_fq.empty()) && !p->d_full)
         if (dev_alloc(&p->d_full, std::max<uint64_t>(1, d.n_postings)) != GENIE_OK)
             return GENIE_OK;
     if (!p->d_uitems)
@@ -2461,81 +2467,140 @@ static int plan_full_decode(genie_plan* p)
     return GENIE_OK;
 }
 
+// The weight that all of a query's items with postings share; 0 if they have
+// several or none.
+static uint32_t query_weight(const genie_plan* p, uint32_t q)
+{
+    uint32_t w = 0;
+    for (uint32_t i = p->h_qptr[q]; i < p->h_qptr[q + 1]; ++i) {
+        const genie_dim_t& it = p->h_items[i];
+        if (it.end_pos <= it.start_pos || it.weight == 0.0f)
+            continue;
+        if (w != 0 && w != (uint32_t)it.weight)
+            return 0;
+        w = (uint32_t)it.weight;
+    }
+    return w;
+}
+
+// Tiles of a selective query: directory tiles per tile for about `target` of
+// its P postings each, and the bits of a tile-local key (id + 1) beside which
+// the query's counts fit (tiles shrink until they do); dtpt = 0 if they never
+// do.  Tiles start on multiples of 16 directory tiles (of a power of two below
+// that), so that directory rows up to grade 4 clip the spans exactly; `most`:
+// rounding up may give a tile this many postings at most (0: no limit).
+static void selective_tiles(const genie_plan* p, uint32_t q, uint64_t target, uint64_t most, uint64_t* out_dtpt,
+                            uint32_t* out_kb)
+{
+    const uint64_t P = p->h_qpost[q], N = p->ix->d.n_objects;
+    const uint64_t nt0 = std::max<uint64_t>(1, (P + target - 1) / target);
+    const uint64_t want = std::max<uint64_t>(1, ((N + nt0 - 1) / nt0 + kDirTile - 1) / kDirTile);
+    uint64_t dtpt = want;
+    if (dtpt >= 16) {
+        dtpt = (dtpt + 15) / 16 * 16;
+    } else {
+        uint64_t pow2 = 1;
+        while (pow2 < dtpt)
+            pow2 <<= 1;
+        dtpt = pow2;
+    }
+    if (most && nt0 > 1 && P * std::min(dtpt * kDirTile, N) / N > most)
+        dtpt = want >= 32 ? want / 16 * 16 : std::max<uint64_t>(1, dtpt / 2);
+    uint32_t kb = 0;
+    for (;;) {
+        const uint64_t tobj = dtpt * kDirTile;
+        kb = 64u - (uint32_t)__builtin_clzll(tobj);  // bits of tobj (keys are 1..tobj)
+        if (kb < 32 && p->h_qbound[q] < (1u << (32 - kb)))
+            break;
+        if (dtpt == 1) {
+            dtpt = 0;
+            break;
+        }
+        dtpt = (dtpt + 1) / 2;
+    }
+    *out_dtpt = dtpt;
+    *out_kb = kb;
+}
+
+// Which kernel counts each query of a plain batch, and its tiles.
+static void split_queries(genie_plan* p, bool filter)
+{
+    const DevIndex& d = p->ix->d;
+    const uint32_t nq = p->n_queries;
+    const uint64_t N = d.n_objects;
+    p->h_hwork.clear();
+    p->h_fwork.clear();
+    p->h_fq.clear();
+    p->h_dq.clear();
+    p->h_hq.assign(nq, make_uint4(0, 0, 0, 0));
+    p->max_hash_tiles = 0;
+    p->est_postings = 0;
+    std::vector<uint8_t> filtered(nq, 0);
+    for (uint32_t q = 0; q < nq; ++q) {
+        const uint64_t P = p->h_qpost[q];
+        uint64_t dtpt = 0;
+        uint32_t kb = 0;
+        if (p->hash_mode != 0 && !p->h_force_direct[q] && (p->hash_mode == 1 || P * 16 <= N)) {
+            // one weight: objects of several postings rank above those of one
+            const uint32_t w = filter && p->h_kq[q] <= kFiltMaxK ? query_weight(p, q) : 0;
+            if (w) {
+                selective_tiles(p, q, kFiltTarget, kFiltTarget + kFiltTarget / 16, &dtpt, &kb);
+                if (dtpt) {
+                    const uint64_t tobj = dtpt * kDirTile;
+                    p->h_hq[q] = make_uint4((uint32_t)dtpt, kb, w, (uint32_t)((N + tobj - 1) / tobj));
+                    filtered[q] = 1;
+                    p->h_fq.push_back(q);
+                }
+            } else {
+                selective_tiles(p, q, kHashTarget, 0, &dtpt, &kb);
+                if (dtpt) {
+                    const uint64_t tobj = dtpt * kDirTile;
+                    const uint64_t nt = (N + tobj - 1) / tobj;
+                    const uint64_t per = (P + nt - 1) / nt;
+                    uint32_t lhs = 9;
+                    while (lhs < (uint32_t)kHashLogMax && (1ull << lhs) < 2 * per)
+                        ++lhs;
+                    p->h_hq[q] = make_uint4((uint32_t)dtpt, kb, lhs, (uint32_t)nt);
+                }
+            }
+            p->max_hash_tiles = std::max(p->max_hash_tiles, p->h_hq[q].w);
+        }
+        if (!dtpt) {
+            p->h_dq.push_back(q);
+            p->est_postings += P;
+        }
+    }
+    // the work tile-major (every query's first tile, then every second one,
+    // ...), so that a query's later tiles mostly start after its first has
+    // published its k-th key, and select from fewer eligible slots
+    for (uint32_t t = 0; t < p->max_hash_tiles; ++t)
+        for (uint32_t q = 0; q < nq; ++q)
+            if (t < p->h_hq[q].w) {
+                auto& work = filtered[q] ? p->h_fwork : p->h_hwork;
+                work.push_back(q);
+                work.push_back(t);
+            }
+}
+
 // The plain form's split of the batch: a query with at most N / 16 postings
 // (every query whose counts fit, when the hash form is forced) runs the hash
 // kernel over tiles of whole directory tiles holding about kHashTarget of its
 // postings each, with 2x that many table slots; the others, and queries
 // whose table filled up in an earlier run, run the direct-mapped kernels.
-// Key bits: key = tile-local id + 1, so tiles shrink until the counts fit in
-// the remaining bits.
+// Queries whose items share one weight, with k up to kFiltMaxK, take the filter
+// kernel instead: tiles of four times the postings.
 static int plan_split_plain(genie_plan* p)
 {
     plain_query_stats(p);
     const DevIndex& d = p->ix->d;
     const uint32_t nq = p->n_queries;
-    const uint64_t N = d.n_objects;
-    p->h_hwork.clear();
-    p->h_dq.clear();
-    p->h_hq.assign(nq, make_uint4(0, 0, 0, 0));
-    p->max_hash_tiles = 0;
-    p->est_postings = 0;
-    for (uint32_t q = 0; q < nq; ++q) {
-        const uint64_t P = p->h_qpost[q];
-        bool hashed = false;
-        if (p->hash_mode != 0 && !p->h_force_direct[q] && (p->hash_mode == 1 || P * 16 <= N)) {
-            const uint64_t nt0 = std::max<uint64_t>(1, (P + kHashTarget - 1) / kHashTarget);
-            uint64_t dtpt = std::max<uint64_t>(1, ((N + nt0 - 1) / nt0 + kDirTile - 1) / kDirTile);
-            // tiles start on multiples of 16 directory tiles (of a power of two
-            // below that), so that directory rows up to grade 4 clip the spans
-            // exactly
-            if (dtpt >= 16) {
-                dtpt = (dtpt + 15) / 16 * 16;
-            } else {
-                uint64_t pow2 = 1;
-                while (pow2 < dtpt)
-                    pow2 <<= 1;
-                dtpt = pow2;
-            }
-            uint32_t kb = 0;
-            for (;;) {
-                const uint64_t tobj = dtpt * kDirTile;
-                kb = 64u - (uint32_t)__builtin_clzll(tobj);  // bits of tobj (keys are 1..tobj)
-                if (kb < 32 && p->h_qbound[q] < (1u << (32 - kb)))
-                    break;
-                if (dtpt == 1) {
-                    dtpt = 0;
-                    break;
-                }
-                dtpt = (dtpt + 1) / 2;
-            }
-            if (dtpt) {
-                const uint64_t tobj = dtpt * kDirTile;
-                const uint64_t nt = (N + tobj - 1) / tobj;
-                const uint64_t per = (P + nt - 1) / nt;
-                uint32_t lhs = 9;
-                while (lhs < (uint32_t)kHashLogMax && (1ull << lhs) < 2 * per)
-                    ++lhs;
-                p->h_hq[q] = make_uint4((uint32_t)dtpt, kb, lhs, (uint32_t)nt);
-                p->max_hash_tiles = std::max(p->max_hash_tiles, (uint32_t)nt);
-                hashed = true;
-            }
-        }
-        if (!hashed) {
-            p->h_dq.push_back(q);
-            p->est_postings += P;
-        }
-    }
-    // the hash work tile-major (every query's first tile, then every second
-    // one, ...), so that a query's later tiles mostly start after its first
-    // has published its k-th key, and select from fewer eligible slots
-    for (uint32_t t = 0; t < p->max_hash_tiles; ++t)
-        for (uint32_t q = 0; q < nq; ++q)
-            if (t < p->h_hq[q].w) {
-                p->h_hwork.push_back(q);
-                p->h_hwork.push_back(t);
-            }
+    // the filter form reads posting lists, decoded ones on a compressed index
+    bool filter = d.key_start && (d.codec == 0 || p->decode_mode != 0) && d.n_objects < (1u << 30);
+    split_queries(p, filter);
     if (int rc = plan_full_decode(p))
         return rc;
+    if (d.codec != 0 && !p->dec_full && !p->h_fq.empty())
+        split_queries(p, filter = false);
     if (p->dec_full)
         p->dec_spans = false;
     else if (int rc = plan_decoded_spans(p))
@@ -2550,6 +2615,16 @@ static int plan_split_plain(genie_plan* p)
     if (!p->h_hwork.empty())
         if (int rc = h2d(p, &p->d_hwork, p->h_hwork.data(), p->h_hwork.size() * 4))
             return rc;
+    if (!p->h_fq.empty()) {
+        if (int rc = grow_buf(p, &p->d_fwork, &p->fwork_alloc, p->h_fwork.size()))
+            return rc;
+        if (int rc = grow_buf(p, &p->d_fq, &p->fq_alloc, p->h_fq.size()))
+            return rc;
+        if (int rc = h2d(p, &p->d_fwork, p->h_fwork.data(), p->h_fwork.size() * 4))
+            return rc;
+        if (int rc = h2d(p, &p->d_fq, p->h_fq.data(), p->h_fq.size() * 4))
+            return rc;
+    }
     if (int rc = h2d(p, &p->d_hq, p->h_hq.data(), nq * sizeof(uint4)))
         return rc;
     if (!p->h_dq.empty())
@@ -2852,10 +2927,10 @@ static int launch_decode_jobs(const DevIndex& d, const uint2* jobs, uint32_t nj,
 static int launch_scan(genie_plan* p, hipStream_t s)
 {
     ScanArgs a = scan_args(p);
-    const uint64_t nwork = p->h_hwork.size() / 2;
+    const uint64_t nwork = p->h_hwork.size() / 2, nfwork = p->h_fwork.size() / 2;
     const uint64_t ndq = p->h_dq.size();
     const uint64_t blocks = (uint64_t)a.n_tiles * ndq;
-    if (blocks >= 0x7FFFFFFFull || nwork >= 0x7FFFFFFFull)
+    if (blocks >= 0x7FFFFFFFull || nwork >= 0x7FFFFFFFull || nfwork >= 0x7FFFFFFFull)
         return fail(GENIE_E_INVALID, "batch too large for one launch");
     const bool runs = runs_used(p);
     if (p->dec_full) {
@@ -2866,7 +2941,7 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         if (nj && runs)
             if (int rc = launch_decode_jobs(d, p->d_fjobs, nj, p->d_runs, true, s))
                 return rc;
-        if (nj && (!runs || nwork))
+        if (nj && (!runs || nwork || nfwork))
             if (int rc = launch_decode_jobs(d, p->d_fjobs, nj, p->d_full, false, s))
                 return rc;
         if (p->timing) {
@@ -2905,6 +2980,22 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         } else {
             k_scan_hash<true><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
         }
+    }
+    if (nfwork) {
+        FilterArgs fa;
+        fa.s = a;
+        fa.work = p->d_fwork;
+        fa.hq = p->d_hq;
+        fa.fq = p->d_fq;
+        fa.items = p->dec_full ? p->d_uitems : p->d_items;
+        fa.item_qptr = p->d_item_qptr;
+        fa.k0 = p->d_nchunks;  // k_item_keys
+        fa.k1 = p->d_chunk_ptr;
+        fa.hov = p->d_hov;
+        fa.hov_any = p->d_hov_any;
+        fa.gkey = p->d_gkey;
+        k_scan_filter<<<(uint32_t)nfwork, kFiltThreads, 0, s>>>(fa);
+        k_filter_fill<<<(uint32_t)p->h_fq.size(), kFiltThreads, 0, s>>>(fa);
     }
     if (ndq) {
         a.qlist = ndq == p->n_queries ? nullptr : p->d_dq;
@@ -3311,12 +3402,13 @@ static int plan_run_once(genie_plan* p, hipStream_t s)
     if (p->n_chunks > p->chunks_cap)
         return fail(GENIE_E_RUNTIME, "batch compiles into more chunks than the plan holds");
     // chunks are read by the hash kernel and by the direct-mapped kernels over
-    // the posting lists; the scan over runs takes the items and their keys
-    const bool runs = runs_used(p), chunks = !runs || !p->h_hwork.empty();
+    // the posting lists; the filter and the scan over runs take the items and
+    // their keys
+    const bool runs = runs_used(p), chunks = !p->h_hwork.empty() || (!runs && !p->h_dq.empty());
     if (chunks)
         if (int rc = launch_compile(p, s))
             return rc;
-    if (runs && ni)  // in the chunk kernels' scratch, which they are done with
+    if ((runs || !p->h_fq.empty()) && ni)  // in the chunk kernels' scratch, which they are done with
         k_item_keys<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, d.key_start, d.n_keys,
                                                      p->d_nchunks, p->d_chunk_ptr);
     if (p->timing)

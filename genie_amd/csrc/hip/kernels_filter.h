@@ -1,0 +1,382 @@
+// Filter form of the plain scan, for selective queries of one weight: most
+// objects that such a query touches occur in one of its lists only, and the
+// top k is made of those that occur in several.
+//
+// k_scan_hash inserts every posting into an LDS hash table (a compare-and-swap
+// and its probes each, eight tiles and eight radix selects a query on LSH
+// batches) to find that out.  Here a tile's ids first go through a bit per
+// hashed id: an id that meets its bit set is entered in a small table; a second
+// pass over the same ids (kept in registers) counts those that are in the
+// table, so that every object of two or more postings has its exact count.
+// Tiles hold four times the postings.  Queries left with fewer than k such
+// objects take the smallest ids among the objects of one posting
+// (k_filter_fill).
+#pragma once
+#include "kernels_hash.h"
+#include "kernels_runs.h"
+
+namespace gh {
+
+constexpr int kFiltThreads = 1024;
+constexpr int kFiltWaves = kFiltThreads / kWave;
+constexpr uint32_t kFiltBitsLog = 18;          // 32 KiB of bits: 1 in 16 set when a full tile is done
+constexpr uint32_t kFiltLogSlots = 13;         // table slots, 32 KiB
+constexpr uint32_t kFiltTarget = 16384;        // postings per (query, tile) aimed at
+constexpr uint32_t kFiltMost = kFiltTarget + kFiltTarget / 8;  // a tile of more flags its query for the direct kernels
+constexpr uint32_t kFiltMaxK = 1024;
+constexpr uint32_t kFiltUnit = 4 * kWave;      // ids a wave loads at a time, 16 bytes a lane
+constexpr int kFiltUnits = 7;                  // units a wave keeps in registers
+constexpr uint32_t kFiltFillMost = (1u << kHashLogMax) / 4 * 3;  // postings k_filter_fill enters in its table
+
+struct FilterArgs {
+    ScanArgs s;
+    const uint32_t* work;       // [n_work][2]: query, tile
+    const uint4* hq;            // [n_queries]: directory tiles per tile, key bits, weight, tiles
+    const uint32_t* fq;         // [n_fq] the queries (fill)
+    const genie_dim_t* items;
+    const uint32_t* item_qptr;
+    const uint32_t *k0, *k1;    // first and last key of every item (k_item_keys)
+    uint32_t* hov;
+    uint32_t* hov_any;
+    unsigned long long* gkey;
+};
+
+// f(lo, hi, valid) for the query's (item, key) pairs, 64 at a time, one a lane:
+// the span of the pair's postings that can hold ids of directory tiles
+// [dt0, dt1).  With `whole` (the tile is the index) an item is one span however
+// many keys it covers.  Called by whole waves.
+template <class F>
+__device__ __forceinline__ void filter_spans(const FilterArgs& fa, uint32_t q, uint32_t dt0, uint32_t dt1, bool whole,
+                                             F f)
+{
+    const ScanArgs& a = fa.s;
+    const int lane = lane_id();
+    const uint32_t i0 = fa.item_qptr[q], i1 = fa.item_qptr[q + 1];
+    for (uint32_t ib = i0; ib < i1; ib += kWave) {
+        uint32_t sp = 0, ep = 0, ka = 0, nk = 0;
+        if (ib + lane < i1) {
+            const genie_dim_t it = fa.items[ib + lane];
+            if (it.end_pos > it.start_pos && it.weight != 0.0f) {
+                sp = (uint32_t)it.start_pos;
+                ep = (uint32_t)it.end_pos;
+                ka = fa.k0[ib + lane];
+                nk = whole ? 1u : fa.k1[ib + lane] - ka + 1u;
+            }
+        }
+        const uint32_t incl = wave_incl_scan(nk);
+        const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
+        const bool single = ballot(nk == 1u || ib + lane >= i1) == ~0ull;  // one pair an item
+        for (uint32_t p0 = 0; p0 < total; p0 += kWave) {
+            const uint32_t p = p0 + lane;
+            // the item of pair p: the first whose prefix passes it
+            int j = 0;
+            if (single) {
+                j = lane;
+            } else {
+#pragma unroll
+                for (int step = 32; step > 0; step >>= 1) {
+                    const uint32_t v = (uint32_t)__shfl((int)incl, j + step - 1, kWave);
+                    if (v <= p)
+                        j += step;
+                }
+            }
+            uint32_t lo = (uint32_t)__shfl((int)sp, j, kWave), hi = (uint32_t)__shfl((int)ep, j, kWave);
+            const uint32_t first = (uint32_t)__shfl((int)(incl - nk), j, kWave);
+            const uint32_t k = (uint32_t)__shfl((int)ka, j, kWave) + (p - first);
+            if (p < total && !whole) {
+                const uint32_t ks = a.key_start[k], doff = a.dir_off[k];
+                lo = max(lo, ks);
+                hi = min(hi, a.key_start[k + 1]);
+                if (doff != kNoDir)
+                    dir_clip(a.dir, doff, ks, dt0, dt1, a.n_dtiles, lo, hi);
+                hi = max(lo, hi);
+            }
+            if (p >= total)
+                lo = hi = 0;
+            f(lo, hi);
+        }
+    }
+}
+
+__device__ __forceinline__ uint32_t filter_bit(uint32_t loc) { return (loc * 0x9E3779B1u) >> (32u - kFiltBitsLog); }
+
+// One workgroup per (query, tile).  Ids are kept tile-local; lanes past a
+// span's end, and ids of other tiles, hold 0xFFFFFFFF.
+// 4M x 64 LSH (8,192 buckets), 4,096 queries: k_scan_hash 1.20 ms; this and the
+// fill: see the profile beside it.
+__global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
+{
+    __shared__ uint32_t s_bits[1u << (kFiltBitsLog - 5)];
+    __shared__ uint32_t s_tab[1u << kFiltLogSlots];
+    __shared__ uint32_t s_red[3 * kMaxWaves];
+    __shared__ uint32_t s_res[8];
+    __shared__ uint32_t s_posts;  // ids of this tile
+    const ScanArgs& a = fa.s;
+    const uint32_t q = fa.work[2 * blockIdx.x], t = fa.work[2 * blockIdx.x + 1];
+    const uint4 prm = fa.hq[q];
+    const uint32_t kb = prm.y, w = prm.z;
+    const uint32_t obj0 = t * prm.x * kDirTile;
+    const uint32_t nobj = min(prm.x * kDirTile, a.n_objects - obj0);
+    const uint32_t dt0 = t * prm.x, dt1 = min(dt0 + prm.x, a.n_dtiles);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    for (uint32_t i = tid; i < 1u << (kFiltBitsLog - 7); i += kFiltThreads)
+        reinterpret_cast<uint4*>(s_bits)[i] = make_uint4(0, 0, 0, 0);
+    for (uint32_t i = tid; i < 1u << (kFiltLogSlots - 2); i += kFiltThreads)
+        reinterpret_cast<uint4*>(s_tab)[i] = make_uint4(0, 0, 0, 0);
+    if (tid == 0) {
+        s_res[7] = 0;
+        s_posts = 0;
+    }
+    __syncthreads();
+
+    // every 16th unit of the spans (uint4 of the lanes from an aligned
+    // position), the first kFiltUnits of the wave in registers; take(v) on
+    // the units past them, in each pass
+    auto units = [&](auto&& keep, auto&& take) {
+        uint32_t turn = wv, mine = 0;
+        filter_spans(fa, q, dt0, dt1, prm.w == 1, [&](uint32_t lo, uint32_t hi) {
+            const uint32_t len = hi - lo;
+            const uint32_t nu = len ? ((lo & 3u) + len + (kFiltUnit - 1)) / kFiltUnit : 0u;
+            const uint32_t incl = wave_incl_scan(nu);
+            const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
+            for (uint32_t u = turn; u < total; u += kFiltWaves, ++mine) {
+                const int r = __popcll(ballot(incl <= u));
+                const uint32_t s = __builtin_amdgcn_readlane(lo, r), n = __builtin_amdgcn_readlane(len, r);
+                const uint32_t p = (s & ~3u) + (u - __builtin_amdgcn_readlane(incl - nu, r)) * kFiltUnit + 4u * lane;
+                auto load = [&]() {
+                    uint4 v = make_uint4(~0u, ~0u, ~0u, ~0u);
+                    if (p + 4u > s && p < s + n) {  // the array ends on a multiple of 16 bytes or past it
+                        if (p >= s && p + 4u <= s + n) {
+                            v = *reinterpret_cast<const uint4*>(a.post + p);
+                        } else {
+                            v.x = p - s < n ? a.post[p] : ~0u;
+                            v.y = p + 1u - s < n ? a.post[p + 1u] : ~0u;
+                            v.z = p + 2u - s < n ? a.post[p + 2u] : ~0u;
+                            v.w = p + 3u - s < n ? a.post[p + 3u] : ~0u;
+                        }
+                    }
+                    return v;
+                };
+                if (mine < (uint32_t)kFiltUnits)
+                    keep(mine, load);
+                else
+                    take(load());
+            }
+            turn = (turn + kFiltWaves - total % kFiltWaves) % kFiltWaves;
+        });
+    };
+    // a posting id as a tile-local one
+    auto local = [&](uint32_t id) { return id - obj0 < nobj ? id - obj0 : ~0u; };
+    bool ok = true;
+    uint32_t posts = 0;
+    auto pass1 = [&](const uint4& v) {
+        const uint32_t x[4] = {local(v.x), local(v.y), local(v.z), local(v.w)};
+        uint32_t old[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t h = filter_bit(x[j]);
+            old[j] = 0;
+            posts += x[j] != ~0u;
+            if (x[j] != ~0u)
+                old[j] = atomicOr(&s_bits[h >> 5], 1u << (h & 31u)) & 1u << (h & 31u);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (old[j])
+                ok &= hash_add(s_tab, kFiltLogSlots, kb, x[j], 0u);
+    };
+    auto pass2 = [&](const uint4& v) {
+        const uint32_t x[4] = {local(v.x), local(v.y), local(v.z), local(v.w)};
+        uint32_t in[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t h = filter_bit(x[j]);
+            in[j] = x[j] != ~0u ? s_bits[h >> 5] >> (h & 31u) & 1u : 0u;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (in[j]) {
+                const uint32_t key = (x[j] + 1u) << (32u - kb), kmask = ~0u << (32u - kb);
+                uint32_t s = (x[j] * 0x9E3779B1u) >> (32u - kFiltLogSlots);
+                for (uint32_t probe = 0; probe < 1u << kFiltLogSlots; ++probe) {
+                    const uint32_t y = s_tab[s];
+                    if (y == 0)
+                        break;  // another id of the same bit
+                    if ((y & kmask) == key) {
+                        atomicAdd(&s_tab[s], w);
+                        break;
+                    }
+                    s = (s + 1u) & ((1u << kFiltLogSlots) - 1u);
+                }
+            }
+    };
+    uint4 kept[kFiltUnits];
+#pragma unroll
+    for (int i = 0; i < kFiltUnits; ++i)
+        kept[i] = make_uint4(~0u, ~0u, ~0u, ~0u);
+    units([&](uint32_t m, auto&& load) {
+        const uint4 v = load();
+#pragma unroll
+        for (int i = 0; i < kFiltUnits; ++i)
+            if (m == (uint32_t)i)  // uniform
+                kept[i] = v;
+    }, pass1);
+#pragma unroll
+    for (int i = 0; i < kFiltUnits; ++i)
+        pass1(kept[i]);
+    posts = wave_sum(posts);
+    if (lane == 0)
+        atomicAdd(&s_posts, posts);
+    if (!ok)
+        s_res[7] = 1;
+    __syncthreads();
+    if (s_res[7] || s_posts > kFiltMost) {
+        if (tid == 0) {
+            fa.hov[q] = 1u;
+            *fa.hov_any = 1u;
+        }
+        return;
+    }
+    // the bits of the table's ids in place of those of every id
+    for (uint32_t i = tid; i < 1u << (kFiltBitsLog - 7); i += kFiltThreads)
+        reinterpret_cast<uint4*>(s_bits)[i] = make_uint4(0, 0, 0, 0);
+    __syncthreads();
+    bool any = false;
+#pragma unroll
+    for (uint32_t i = 0; i < (1u << kFiltLogSlots) / kFiltThreads; ++i) {
+        const uint32_t y = s_tab[tid + i * kFiltThreads];
+        if (y) {
+            const uint32_t h = filter_bit((y >> (32u - kb)) - 1u);
+            atomicOr(&s_bits[h >> 5], 1u << (h & 31u));
+            any = true;
+        }
+    }
+    if (!__syncthreads_or(any))
+        return;  // no object of two postings
+#pragma unroll
+    for (int i = 0; i < kFiltUnits; ++i)
+        pass2(kept[i]);
+    units([](uint32_t, auto&&) {}, pass2);
+    __syncthreads();
+    hash_select(a, fa.gkey, s_tab, 1u << kFiltLogSlots, kb, q, obj0, s_res, s_red, a.kq[q], 2u * w, 0xFFFFFFFFu, true);
+}
+
+// Marks an id in the fill's table: a word of key << (32 - kb) | 1 after one
+// posting, | 3 after more.  The table is at most three quarters full.
+__device__ __forceinline__ void fill_add(uint32_t* tab, uint32_t kb, uint32_t id)
+{
+    const uint32_t key = (id + 1u) << (32u - kb), kmask = ~0u << (32u - kb);
+    uint32_t h = (id * 0x9E3779B1u) >> (32u - kHashLogMax);
+    for (uint32_t probe = 0; probe < 1u << kHashLogMax; ++probe) {
+        const uint32_t v = atomicCAS(&tab[h], 0u, key | 1u);
+        if (v == 0)
+            return;
+        if ((v & kmask) == key) {
+            atomicOr(&tab[h], 2u);
+            return;
+        }
+        h = (h + 1u) & ((1u << kHashLogMax) - 1u);
+    }
+}
+
+// Queries that the filter left with fewer than k candidates: the smallest ids
+// among the objects of one posting.  Lists ascend, so these lie in the first
+// postings of every list: all ids below a bound are counted in a table, the
+// bound first set for the number needed and doubled until enough objects of
+// one posting are below it.
+__global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
+{
+    __shared__ uint32_t s_tab[1u << kHashLogMax];
+    __shared__ uint32_t s_red[3 * kMaxWaves];
+    __shared__ uint32_t s_res[8];
+    __shared__ uint32_t s_posts, s_in, s_ones;
+    const ScanArgs& a = fa.s;
+    const uint32_t q = fa.fq[blockIdx.x];
+    const uint32_t k = a.kq[q], have = a.cand_cnt[q];
+    if (have >= k || fa.hov[q])
+        return;
+    const uint32_t need = k - have;
+    const uint32_t w = fa.hq[q].z;
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (tid == 0)
+        s_posts = 0;
+    __syncthreads();
+    if (wv == 0) {
+        uint32_t n = 0;
+        filter_spans(fa, q, 0, a.n_dtiles, true, [&](uint32_t lo, uint32_t hi) { n += hi - lo; });
+        n = wave_sum(n);
+        if (lane == 0)
+            s_posts = n;
+    }
+    __syncthreads();
+    const uint32_t posts = s_posts;
+    if (posts == 0)
+        return;
+    // ids that should lie below the bound: those needed, the objects of more
+    // postings, and a margin
+    uint64_t x = (uint64_t)a.n_objects * (need + need / 4 + 64u) / posts + 1;
+    for (;;) {
+        const uint32_t bound = (uint32_t)min<uint64_t>(x, a.n_objects);
+        const uint32_t kb = 32u - (uint32_t)__builtin_clz(bound);  // keys are 1..bound (below 2^30)
+        // f(id) for the ids below the bound, a wave a span, every 16th of 64
+        auto below = [&](auto&& f) {
+            filter_spans(fa, q, 0, a.n_dtiles, false, [&](uint32_t lo, uint32_t hi) {
+                const uint64_t some = ballot(hi > lo);
+                for (uint32_t r = wv; r < (uint32_t)kWave; r += kFiltWaves) {
+                    if (!((some >> r) & 1u))
+                        continue;
+                    const uint32_t s = __builtin_amdgcn_readlane(lo, r), e = __builtin_amdgcn_readlane(hi, r);
+                    for (uint32_t p = s; p < e; p += kWave) {
+                        const uint32_t id = p + lane < e ? a.post[p + lane] : ~0u;
+                        if (id < bound)
+                            f(id);
+                        if (ballot(id < bound) != ~0ull)
+                            break;  // the list ascends: the rest is past the bound
+                    }
+                }
+            });
+        };
+        for (uint32_t i = tid; i < 1u << kHashLogMax; i += kFiltThreads)
+            s_tab[i] = 0;
+        if (tid == 0) {
+            s_in = 0;
+            s_ones = 0;
+        }
+        __syncthreads();
+        uint32_t in = 0;
+        below([&](uint32_t) { ++in; });
+        in = wave_sum(in);
+        if (lane == 0)
+            atomicAdd(&s_in, in);
+        __syncthreads();
+        if (s_in > kFiltFillMost) {
+            if (tid == 0) {
+                fa.hov[q] = 1u;  // too crowded for the table: the direct kernels
+                *fa.hov_any = 1u;
+            }
+            return;
+        }
+        below([&](uint32_t id) { fill_add(s_tab, kb, id); });
+        __syncthreads();
+        uint32_t ones = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < (1u << kHashLogMax) / kFiltThreads; ++i) {
+            const uint32_t y = s_tab[tid + i * kFiltThreads];
+            ones += y != 0 && (y & ((1u << (32u - kb)) - 1u)) == 1u;
+        }
+        ones = wave_sum(ones);
+        if (lane == 0)
+            atomicAdd(&s_ones, ones);
+        __syncthreads();
+        if (s_ones >= need || bound == a.n_objects) {
+            hash_select(a, fa.gkey, s_tab, 1u << kHashLogMax, kb, q, 0, s_res, s_red, need, 1u, 1u, false, w);
+            return;
+        }
+        x *= 2;
+        __syncthreads();
+    }
+}
+
+}  // namespace gh

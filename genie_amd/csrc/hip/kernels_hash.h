@@ -176,17 +176,22 @@ constexpr int kHashPer = (1 << kHashLogMax) / kScanThreads;  // slots per thread
 constexpr uint32_t kSelDigit = 11;                             // bits per radix pass
 constexpr uint32_t kSelBins = 1u << kSelDigit;
 
+// `least`, `most`: the counts that are eligible at all (the filter kernels,
+// kernels_filter.h, take objects of one posting apart from the others);
+// `k`: how many to take; `scale`: count of a table count of 1; `publish`: whether the tile's k-th count and key bound
+// the query's later tiles.
 __device__ __forceinline__ void hash_select(const ScanArgs& a, unsigned long long* gkey, uint32_t* tab, uint32_t ns,
-                                            uint32_t kb, uint32_t q, uint32_t obj0, uint32_t* s_res, uint32_t* s_red)
+                                            uint32_t kb, uint32_t q, uint32_t obj0, uint32_t* s_res, uint32_t* s_red,
+                                            uint32_t k, uint32_t least, uint32_t most, bool publish,
+                                            uint32_t scale = 1u)
 {
     static_assert(kSelBins <= (1u << kHashLogMax) && kSelBins == 32 * kWave, "histogram in the table, 32 bins a lane");
     const int tid = threadIdx.x, lane = lane_id(), wv = tid >> 6, nw = blockDim.x / kWave;
-    const uint32_t k = a.kq[q];
     const uint32_t cb = 32u - kb;
     const uint32_t cmask = (1u << cb) - 1u;
     const uint32_t kfull = (1u << kb) - 1u;
     const uint32_t per = ns / blockDim.x;  // uniform, 1..kHashPer
-    if (tid == 0) {
+    if (tid == 0 && publish) {
         uint32_t lo = __hip_atomic_load(&a.gthr[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         const uint64_t g = __hip_atomic_load(&gkey[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         if (g) {
@@ -196,7 +201,7 @@ __device__ __forceinline__ void hash_select(const ScanArgs& a, unsigned long lon
         s_res[0] = lo;
     }
     __syncthreads();
-    const uint32_t lower = max(1u, s_res[0]);
+    const uint32_t lower = max(least, publish ? s_res[0] : 0u);
     uint32_t rk[kHashPer];
     uint32_t e = 0, rmax = 0, rmin = 0xFFFFFFFFu;
 #pragma unroll
@@ -205,7 +210,7 @@ __device__ __forceinline__ void hash_select(const ScanArgs& a, unsigned long lon
         if ((uint32_t)j < per) {
             const uint32_t v = tab[tid + j * blockDim.x];
             const uint32_t c = v & cmask;
-            if (c >= lower) {
+            if (c >= lower && c <= most) {
                 rk[j] = (c << kb) | (kfull - (v >> cb));
                 ++e;
                 rmax = max(rmax, rk[j]);
@@ -315,7 +320,7 @@ __device__ __forceinline__ void hash_select(const ScanArgs& a, unsigned long lon
                 wb = atomicAdd(&s_res[5], (uint32_t)__popcll(bm));
             wb = (uint32_t)__shfl((int)wb, __builtin_ctzll(bm), kWave);
             if (take) {
-                out[wb + lane_prefix(bm)] = make_key(r >> kb, obj0 + (kfull - (r & kfull)) - 1u);
+                out[wb + lane_prefix(bm)] = make_key((r >> kb) * scale, obj0 + (kfull - (r & kfull)) - 1u);
                 rmin_sel = min(rmin_sel, r);
             }
         }
@@ -324,7 +329,7 @@ __device__ __forceinline__ void hash_select(const ScanArgs& a, unsigned long lon
     if (lane == 0 && rmin_sel != 0xFFFFFFFFu)
         atomicMin(&s_res[6], rmin_sel);
     __syncthreads();
-    if (tid == 0 && E >= k) {
+    if (tid == 0 && E >= k && publish) {
         const uint32_t r = s_res[6];
         atomicMax(&a.gthr[q], r >> kb);
         atomicMax(&gkey[q], (unsigned long long)make_key(r >> kb, obj0 + (kfull - (r & kfull)) - 1u));
@@ -471,7 +476,7 @@ __global__ void __launch_bounds__(kScanThreads) k_scan_hash(HashArgs h)
         }
         return;
     }
-    hash_select(a, h.gkey, s_tab, ns, kb, q, obj0, s_res, s_red);
+    hash_select(a, h.gkey, s_tab, ns, kb, q, obj0, s_res, s_red, a.kq[q], 1u, 0xFFFFFFFFu, true);
 }
 
 }  // namespace gh
