@@ -20,6 +20,8 @@ constexpr uint32_t kShortList = 256;
 // device so that the waves of a workgroup share long lists evenly.
 constexpr uint32_t kChunk = 32768;
 constexpr uint32_t kNoDir = 0xFFFFFFFFu;
+// Entries past a posting array's last that a 16-byte load may read.
+constexpr uint32_t kPostPad = 4;
 
 // Directory rows are graded: key k's row has an entry for every 2^s-th
 // directory tile boundary (entry j describes boundary (j << s) * kDirTile,
@@ -118,6 +120,9 @@ struct DevIndex {
     uint4* seg_bph = nullptr;       // [n_segments] BP32 block header word offsets, 8 x u16 (BP32 codecs)
     uint32_t* sdir_off = nullptr;   // [n_keys] row of each key with more than 4 segments (compressed)
     uint32_t* sdir = nullptr;       // graded segment-directory rows (compressed)
+    // device copy of a PosIndex over the key starts in posting positions
+    uint32_t* kpos = nullptr;       // [kpos_n + 1]
+    uint32_t kpos_n = 0, kpos_shift = 0;
     // tile-major copy of the postings (16-bit ids within tiles of 65,536
     // objects) for the direct-mapped scan; a compressed index has only the
     // directory, its plans decode into copies of their own

@@ -122,6 +122,7 @@ struct genie_plan {
     int hash_mode = -1;         // -1 automatic, 0 off, 1 every query whose counts fit
     std::vector<uint64_t> h_qpost;        // postings of every query
     std::vector<uint32_t> h_qbound;       // count bound of every query
+    std::vector<uint8_t> h_qmulti;        // queries with an item of several keys
     std::vector<uint8_t> h_force_direct;  // queries whose table filled up in an earlier run
     std::vector<uint32_t> h_hwork;        // (query, tile) of the hash kernel
     std::vector<uint4> h_hq;              // per query: directory tiles per tile, key bits, log2 slots, tiles
@@ -131,8 +132,11 @@ struct genie_plan {
     uint32_t* d_hwork = nullptr;
     uint64_t hwork_alloc = 0;
     std::vector<uint32_t> h_fwork, h_fq;  // (query, tile) of the filter kernel, its queries
+    std::vector<uint4> h_fhq;             // per query: directory tiles per tile, key bits, weight, tiles
     uint32_t *d_fwork = nullptr, *d_fq = nullptr;
-    uint64_t fwork_alloc = 0, fq_alloc = 0;
+    uint4* d_fhq = nullptr;
+    uint2* d_fspan = nullptr;             // [tiles][items]
+    uint64_t fwork_alloc = 0, fq_alloc = 0, fhq_alloc = 0, fspan_alloc = 0;
     uint4* d_hq = nullptr;
     uint32_t* d_dq = nullptr;
     uint32_t* d_hov = nullptr;
@@ -340,6 +344,8 @@ static void plan_free_buffers(genie_plan* p)
     dev_free(p->d_hwork);
     dev_free(p->d_fwork);
     dev_free(p->d_fq);
+    dev_free(p->d_fhq);
+    dev_free(p->d_fspan);
     dev_free(p->d_hq);
     dev_free(p->d_dq);
     dev_free(p->d_hov);
@@ -373,9 +379,10 @@ static void plan_free_buffers(genie_plan* p)
 // dim for single-value tables; the sum of per-key multiplicities for
 // bijectMap tables), summed over groups.  Items are bucketed by query and
 // each query's entries sorted on their own (one entry per item when the item
-// lies in one dim of a single-value table, one per key otherwise).
+// lies in one dim of a single-value table, one per key otherwise).  `multi`
+// (optional): set for the queries with an item of several keys.
 static int compute_bounds(const DevIndex& d, const genie_dim_t* items, uint64_t n_items,
-                          uint32_t n_queries, uint32_t* out)
+                          uint32_t n_queries, uint32_t* out, uint8_t* multi = nullptr)
 {
     std::vector<uint32_t> qptr(n_queries + 1, 0), idx(n_items);
     for (uint64_t i = 0; i < n_items; ++i)
@@ -412,6 +419,8 @@ static int compute_bounds(const DevIndex& d, const genie_dim_t* items, uint64_t 
                 k0 = d.h_seg_key[s0];
                 k1 = d.h_seg_key[s1];
             }
+            if (multi && k0 != k1)
+                multi[q] = 1;
             const uint32_t w = (uint32_t)it.weight;
             if (d.single_value && d.h_key_dim[k0] == d.h_key_dim[k1])
                 v.push_back({it.order, d.h_key_dim[k0], w});
@@ -515,6 +524,7 @@ int gh::validate_items(const DevIndex& d, const genie_dim_t* items, uint64_t n_i
 
 static bool dense_shape(const genie_index_desc* desc, std::vector<uint32_t>& key_base, std::vector<uint32_t>& per_dim);
 static int build_sets(const genie_index_desc* desc, DevIndex& d);
+static int build_key_pos(DevIndex& d);
 static int build_runs(DevIndex& d, const uint32_t* post, bool copy);
 static int build_set_matrix(const genie_index_desc* desc, DevIndex& d);
 static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t* post, const uint32_t* key_start);
@@ -718,6 +728,8 @@ static int create_compressed(const genie_index_desc* desc, genie_index** out)
         }
         if (want_dense)
             rc = build_dense(desc, d, d_post, d.key_start);
+        if (!rc)
+            rc = build_key_pos(d);
         if (!rc)
             rc = build_runs(d, d_post, false);
         if (!rc)
@@ -1079,6 +1091,21 @@ static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t
     d.codes = codes;
     d.key_slot = key_slot;
     d.bytes += bytes;
+    return GENIE_OK;
+}
+
+// Device copy of the key lookup (key_at): a PosIndex over the key starts in
+// posting positions.
+static int build_key_pos(DevIndex& d)
+{
+    PosIndex px;
+    px.build(d.h_key_start);
+    d.kpos_n = (uint32_t)px.first.size() - 1;
+    d.kpos_shift = px.shift;
+    if (int rc = dev_alloc(&d.kpos, px.first.size(), &d.bytes))
+        return rc;
+    if (hipError_t e = hipMemcpy(d.kpos, px.first.data(), px.first.size() * 4, hipMemcpyHostToDevice))
+        return fail(GENIE_E_RUNTIME, std::string("key index upload: ") + hipGetErrorString(e));
     return GENIE_OK;
 }
 
@@ -1481,7 +1508,7 @@ int genie_hip_index_create(const genie_index_desc* desc, genie_index** out)
     int rc = GENIE_OK;
     uint32_t* d_dir_keys = nullptr;
     do {
-        if ((rc = dev_alloc(&d.post, d.n_postings, &d.bytes))) break;
+        if ((rc = dev_alloc(&d.post, d.n_postings + kPostPad, &d.bytes))) break;
         if ((rc = dev_alloc(&d.key_start, d.n_keys + 1, &d.bytes))) break;
         if ((rc = dev_alloc(&d.dir_off, d.n_keys, &d.bytes))) break;
         if ((rc = dev_alloc(&d.dir, dir_words, &d.bytes))) break;
@@ -1507,6 +1534,8 @@ int genie_hip_index_create(const genie_index_desc* desc, genie_index** out)
     dev_free(d_dir_keys);
     if (!rc)
         rc = build_dense(desc, d, d.post, d.key_start);
+    if (!rc)
+        rc = build_key_pos(d);
     if (!rc)
         rc = build_runs(d, d.post, true);
     if (!rc)
@@ -1538,6 +1567,7 @@ int genie_hip_index_destroy(genie_index* ix)
     dev_free(d.key_seg);
     dev_free(d.sdir_off);
     dev_free(d.sdir);
+    dev_free(d.kpos);
     dev_free(d.run_ids);
     dev_free(d.run_tf);
     dev_free(d.codes);
@@ -2267,9 +2297,11 @@ static void plain_query_stats(genie_plan* p)
     const uint32_t nq = p->n_queries;
     if (p->count_bound != 0) {
         p->h_qbound.assign(nq, p->count_bound);
+        p->h_qmulti.assign(nq, 1);  // not looked at
     } else if (p->h_qbound.size() != nq || p->dense_ok) {  // upload skips a dense batch's bounds
         p->h_qbound.resize(nq);
-        compute_bounds(d, p->h_items.data(), p->n_items, nq, p->h_qbound.data());
+        p->h_qmulti.assign(nq, 0);
+        compute_bounds(d, p->h_items.data(), p->n_items, nq, p->h_qbound.data(), p->h_qmulti.data());
     }
     p->h_qpost.assign(nq, 0);
     const uint32_t* cp = d.h_seg_cpos.data();
@@ -2415,7 +2447,7 @@ static int plan_full_decode(genie_plan* p)
         if (dev_alloc(&p->d_runs, d.n_postings + kRunPad) != GENIE_OK)
             return GENIE_OK;  // no room for the scratch: in-kernel decode
     if ((!tiled || !p->h_hwork.empty() || !p->h_fq.empty()) && !p->d_full)
-        if (dev_alloc(&p->d_full, std::max<uint64_t>(1, d.n_postings)) != GENIE_OK)
+        if (dev_alloc(&p->d_full, d.n_postings + kPostPad) != GENIE_OK)
             return GENIE_OK;
     if (!p->d_uitems)
         if (int rc = dev_alloc(&p->d_uitems, std::max<uint64_t>(1, p->max_items)))
@@ -2522,6 +2554,16 @@ static void selective_tiles(const genie_plan* p, uint32_t q, uint64_t target, ui
     *out_kb = kb;
 }
 
+// Spans of the filter kernel: an entry per item and tile of the most any of its
+// queries has.
+static uint64_t filter_span_count(const genie_plan* p)
+{
+    uint32_t nt = 0;
+    for (uint32_t q : p->h_fq)
+        nt = std::max(nt, p->h_fhq[q].w);
+    return nt * p->n_items;
+}
+
 // Which kernel counts each query of a plain batch, and its tiles.
 static void split_queries(genie_plan* p, bool filter)
 {
@@ -2535,20 +2577,20 @@ static void split_queries(genie_plan* p, bool filter)
     p->h_hq.assign(nq, make_uint4(0, 0, 0, 0));
     p->max_hash_tiles = 0;
     p->est_postings = 0;
-    std::vector<uint8_t> filtered(nq, 0);
+    p->h_fhq.assign(nq, make_uint4(0, 0, 0, 0));
     for (uint32_t q = 0; q < nq; ++q) {
         const uint64_t P = p->h_qpost[q];
         uint64_t dtpt = 0;
         uint32_t kb = 0;
         if (p->hash_mode != 0 && !p->h_force_direct[q] && (p->hash_mode == 1 || P * 16 <= N)) {
             // one weight: objects of several postings rank above those of one
-            const uint32_t w = filter && p->h_kq[q] <= kFiltMaxK ? query_weight(p, q) : 0;
+            const uint32_t w = filter && p->h_kq[q] <= kFiltMaxK && !p->h_qmulti[q] ? query_weight(p, q) : 0;
             if (w) {
                 selective_tiles(p, q, kFiltTarget, kFiltTarget + kFiltTarget / 16, &dtpt, &kb);
                 if (dtpt) {
                     const uint64_t tobj = dtpt * kDirTile;
-                    p->h_hq[q] = make_uint4((uint32_t)dtpt, kb, w, (uint32_t)((N + tobj - 1) / tobj));
-                    filtered[q] = 1;
+                    p->h_fhq[q] = make_uint4((uint32_t)dtpt, kb, w, (uint32_t)((N + tobj - 1) / tobj));
+                    p->h_hq[q] = p->h_fhq[q];
                     p->h_fq.push_back(q);
                 }
             } else {
@@ -2576,7 +2618,7 @@ static void split_queries(genie_plan* p, bool filter)
     for (uint32_t t = 0; t < p->max_hash_tiles; ++t)
         for (uint32_t q = 0; q < nq; ++q)
             if (t < p->h_hq[q].w) {
-                auto& work = filtered[q] ? p->h_fwork : p->h_hwork;
+                auto& work = p->h_fhq[q].w ? p->h_fwork : p->h_hwork;
                 work.push_back(q);
                 work.push_back(t);
             }
@@ -2597,6 +2639,8 @@ static int plan_split_plain(genie_plan* p)
     // the filter form reads posting lists, decoded ones on a compressed index
     bool filter = d.key_start && (d.codec == 0 || p->decode_mode != 0) && d.n_objects < (1u << 30);
     split_queries(p, filter);
+    if (filter_span_count(p) > 1ull << 27)  // a GiB of spans: many items over many tiles
+        split_queries(p, filter = false);
     if (int rc = plan_full_decode(p))
         return rc;
     if (d.codec != 0 && !p->dec_full && !p->h_fq.empty())
@@ -2619,6 +2663,12 @@ static int plan_split_plain(genie_plan* p)
         if (int rc = grow_buf(p, &p->d_fwork, &p->fwork_alloc, p->h_fwork.size()))
             return rc;
         if (int rc = grow_buf(p, &p->d_fq, &p->fq_alloc, p->h_fq.size()))
+            return rc;
+        if (int rc = grow_buf(p, &p->d_fhq, &p->fhq_alloc, nq))
+            return rc;
+        if (int rc = grow_buf(p, &p->d_fspan, &p->fspan_alloc, filter_span_count(p)))
+            return rc;
+        if (int rc = h2d(p, &p->d_fhq, p->h_fhq.data(), nq * sizeof(uint4)))
             return rc;
         if (int rc = h2d(p, &p->d_fwork, p->h_fwork.data(), p->h_fwork.size() * 4))
             return rc;
@@ -2698,7 +2748,8 @@ static int plan_upload(genie_plan* p, const genie_dim_t* items, uint64_t n_items
             p->lane_bits = 8;  // dense, unit weights: each dim once, counts <= 128
         } else {  // weighted dense batches count up to 128 x 15
             p->h_qbound.resize(n_queries);
-            compute_bounds(d, p->h_items.data(), n_items, n_queries, p->h_qbound.data());
+            p->h_qmulti.assign(n_queries, 0);
+            compute_bounds(d, p->h_items.data(), n_items, n_queries, p->h_qbound.data(), p->h_qmulti.data());
             uint32_t mx = 0;
             for (uint32_t v : p->h_qbound)
                 mx = std::max(mx, v);
@@ -2922,6 +2973,8 @@ static int launch_decode_jobs(const DevIndex& d, const uint2* jobs, uint32_t nj,
     return GENIE_OK;
 }
 
+static KeyPos key_pos_of(const DevIndex& d) { return KeyPos{d.kpos, d.kpos_n, d.kpos_shift, d.key_start}; }
+
 // The plain form's scan: the hash kernel over the (query, tile) work of the
 // selective queries, then the direct-mapped kernel over the other queries.
 static int launch_scan(genie_plan* p, hipStream_t s)
@@ -2985,15 +3038,16 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         FilterArgs fa;
         fa.s = a;
         fa.work = p->d_fwork;
-        fa.hq = p->d_hq;
+        fa.hq = p->d_fhq;
         fa.fq = p->d_fq;
         fa.items = p->dec_full ? p->d_uitems : p->d_items;
+        fa.n_items = (uint32_t)p->n_items;
         fa.item_qptr = p->d_item_qptr;
-        fa.k0 = p->d_nchunks;  // k_item_keys
-        fa.k1 = p->d_chunk_ptr;
+        fa.spans = p->d_fspan;
         fa.hov = p->d_hov;
         fa.hov_any = p->d_hov_any;
         fa.gkey = p->d_gkey;
+        k_filter_spans<<<(fa.n_items + 255) / 256, 256, 0, s>>>(fa, key_pos_of(p->ix->d));
         k_scan_filter<<<(uint32_t)nfwork, kFiltThreads, 0, s>>>(fa);
         k_filter_fill<<<(uint32_t)p->h_fq.size(), kFiltThreads, 0, s>>>(fa);
     }
@@ -3408,8 +3462,8 @@ static int plan_run_once(genie_plan* p, hipStream_t s)
     if (chunks)
         if (int rc = launch_compile(p, s))
             return rc;
-    if ((runs || !p->h_fq.empty()) && ni)  // in the chunk kernels' scratch, which they are done with
-        k_item_keys<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, d.key_start, d.n_keys,
+    if (runs && ni)  // in the chunk kernels' scratch, which they are done with
+        k_item_keys<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, key_pos_of(d),
                                                      p->d_nchunks, p->d_chunk_ptr);
     if (p->timing)
         HIP_TRY(hipEventRecord(p->ev[1], s));

@@ -25,80 +25,80 @@ constexpr uint32_t kFiltTarget = 16384;        // postings per (query, tile) aim
 constexpr uint32_t kFiltMost = kFiltTarget + kFiltTarget / 8;  // a tile of more flags its query for the direct kernels
 constexpr uint32_t kFiltMaxK = 1024;
 constexpr uint32_t kFiltUnit = 4 * kWave;      // ids a wave loads at a time, 16 bytes a lane
-constexpr int kFiltUnits = 7;                  // units a wave keeps in registers
+constexpr int kFiltUnits = 5;                  // units a wave keeps in registers
+constexpr uint32_t kFiltList = 2048;           // ids on their way into (or counted in) the table, a part a wave
 constexpr uint32_t kFiltFillMost = (1u << kHashLogMax) / 4 * 3;  // postings k_filter_fill enters in its table
 
 struct FilterArgs {
     ScanArgs s;
     const uint32_t* work;       // [n_work][2]: query, tile
-    const uint4* hq;            // [n_queries]: directory tiles per tile, key bits, weight, tiles
+    const uint4* hq;            // [n_queries]: directory tiles per tile, key bits, weight, tiles (0: other kernels)
     const uint32_t* fq;         // [n_fq] the queries (fill)
-    const genie_dim_t* items;
+    const genie_dim_t* items;   // one key each
+    uint32_t n_items;
     const uint32_t* item_qptr;
-    const uint32_t *k0, *k1;    // first and last key of every item (k_item_keys)
+    uint2* spans;               // [tiles][n_items] every item's postings that can hold ids of the tile
     uint32_t* hov;
     uint32_t* hov_any;
     unsigned long long* gkey;
 };
 
-// f(lo, hi, valid) for the query's (item, key) pairs, 64 at a time, one a lane:
-// the span of the pair's postings that can hold ids of directory tiles
-// [dt0, dt1).  With `whole` (the tile is the index) an item is one span however
-// many keys it covers.  Called by whole waves.
-template <class F>
-__device__ __forceinline__ void filter_spans(const FilterArgs& fa, uint32_t q, uint32_t dt0, uint32_t dt1, bool whole,
-                                             F f)
+// Every item's span in every tile of its query, resolved once: the key and
+// directory reads are scattered, and a workgroup per (query, tile) whose waves
+// each made them spent most of its time there (4M x 64 LSH: 0.53 of 0.82 ms).
+__global__ void __launch_bounds__(256) k_filter_spans(FilterArgs fa, KeyPos kp)
 {
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= fa.n_items)
+        return;
+    const genie_dim_t it = fa.items[i];
+    const uint4 prm = fa.hq[it.query];
+    if (prm.w == 0)
+        return;
     const ScanArgs& a = fa.s;
-    const int lane = lane_id();
-    const uint32_t i0 = fa.item_qptr[q], i1 = fa.item_qptr[q + 1];
-    for (uint32_t ib = i0; ib < i1; ib += kWave) {
-        uint32_t sp = 0, ep = 0, ka = 0, nk = 0;
-        if (ib + lane < i1) {
-            const genie_dim_t it = fa.items[ib + lane];
-            if (it.end_pos > it.start_pos && it.weight != 0.0f) {
-                sp = (uint32_t)it.start_pos;
-                ep = (uint32_t)it.end_pos;
-                ka = fa.k0[ib + lane];
-                nk = whole ? 1u : fa.k1[ib + lane] - ka + 1u;
-            }
-        }
-        const uint32_t incl = wave_incl_scan(nk);
-        const uint32_t total = __builtin_amdgcn_readlane(incl, kWave - 1);
-        const bool single = ballot(nk == 1u || ib + lane >= i1) == ~0ull;  // one pair an item
-        for (uint32_t p0 = 0; p0 < total; p0 += kWave) {
-            const uint32_t p = p0 + lane;
-            // the item of pair p: the first whose prefix passes it
-            int j = 0;
-            if (single) {
-                j = lane;
-            } else {
-#pragma unroll
-                for (int step = 32; step > 0; step >>= 1) {
-                    const uint32_t v = (uint32_t)__shfl((int)incl, j + step - 1, kWave);
-                    if (v <= p)
-                        j += step;
-                }
-            }
-            uint32_t lo = (uint32_t)__shfl((int)sp, j, kWave), hi = (uint32_t)__shfl((int)ep, j, kWave);
-            const uint32_t first = (uint32_t)__shfl((int)(incl - nk), j, kWave);
-            const uint32_t k = (uint32_t)__shfl((int)ka, j, kWave) + (p - first);
-            if (p < total && !whole) {
-                const uint32_t ks = a.key_start[k], doff = a.dir_off[k];
-                lo = max(lo, ks);
-                hi = min(hi, a.key_start[k + 1]);
-                if (doff != kNoDir)
-                    dir_clip(a.dir, doff, ks, dt0, dt1, a.n_dtiles, lo, hi);
-                hi = max(lo, hi);
-            }
-            if (p >= total)
-                lo = hi = 0;
-            f(lo, hi);
-        }
+    const bool empty = it.end_pos <= it.start_pos || it.weight == 0.0f;
+    const uint32_t sp = empty ? 0u : (uint32_t)it.start_pos, ep = empty ? 0u : (uint32_t)it.end_pos;
+    uint32_t ks = 0, doff = kNoDir;
+    if (!empty && prm.w > 1) {
+        const uint32_t k = key_at(kp, sp);
+        ks = kp.key_start[k];
+        doff = a.dir_off[k];
+    }
+    for (uint32_t t = 0; t < prm.w; ++t) {
+        uint32_t lo = sp, hi = ep;
+        if (doff != kNoDir)
+            dir_clip(a.dir, doff, ks, t * prm.x, min(t * prm.x + prm.x, a.n_dtiles), a.n_dtiles, lo, hi);
+        fa.spans[(uint64_t)t * fa.n_items + i] = make_uint2(lo, max(lo, hi));
     }
 }
 
-__device__ __forceinline__ uint32_t filter_bit(uint32_t loc) { return (loc * 0x9E3779B1u) >> (32u - kFiltBitsLog); }
+// f(lo, hi) for the query's items, 64 at a time, one a lane: the spans of tile
+// t, or (whole) the items' own.  Called by whole waves.
+template <class F>
+__device__ __forceinline__ void filter_spans(const FilterArgs& fa, uint32_t q, uint32_t t, bool whole, F f)
+{
+    const uint32_t i0 = fa.item_qptr[q], i1 = fa.item_qptr[q + 1], lane = lane_id();
+    for (uint32_t ib = i0; ib < i1; ib += kWave) {
+        uint2 sp = make_uint2(0, 0);
+        if (ib + lane < i1) {
+            if (whole) {
+                const genie_dim_t it = fa.items[ib + lane];
+                if (it.end_pos > it.start_pos && it.weight != 0.0f)
+                    sp = make_uint2((uint32_t)it.start_pos, (uint32_t)it.end_pos);
+            } else {
+                sp = fa.spans[(uint64_t)t * fa.n_items + ib + lane];
+            }
+        }
+        f(sp.x, sp.y);
+    }
+}
+
+// Bit of an id: a full-rate 24-bit product (bits of an id above 24 do not
+// enter; ids that share a bit only pass the filter together).
+__device__ __forceinline__ uint32_t filter_bit(uint32_t loc)
+{
+    return ((loc & 0xFFFFFFu) * 0x9E3779u) >> (32u - kFiltBitsLog);
+}
 
 // One workgroup per (query, tile).  Ids are kept tile-local; lanes past a
 // span's end, and ids of other tiles, hold 0xFFFFFFFF.
@@ -110,14 +110,15 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     __shared__ uint32_t s_tab[1u << kFiltLogSlots];
     __shared__ uint32_t s_red[3 * kMaxWaves];
     __shared__ uint32_t s_res[8];
+    __shared__ uint32_t s_list[kFiltList];
     __shared__ uint32_t s_posts;  // ids of this tile
+    __shared__ uint32_t s_n;      // some id is listed
     const ScanArgs& a = fa.s;
     const uint32_t q = fa.work[2 * blockIdx.x], t = fa.work[2 * blockIdx.x + 1];
     const uint4 prm = fa.hq[q];
     const uint32_t kb = prm.y, w = prm.z;
     const uint32_t obj0 = t * prm.x * kDirTile;
     const uint32_t nobj = min(prm.x * kDirTile, a.n_objects - obj0);
-    const uint32_t dt0 = t * prm.x, dt1 = min(dt0 + prm.x, a.n_dtiles);
     const uint32_t tid = threadIdx.x, lane = lane_id();
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (uint32_t i = tid; i < 1u << (kFiltBitsLog - 7); i += kFiltThreads)
@@ -127,6 +128,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     if (tid == 0) {
         s_res[7] = 0;
         s_posts = 0;
+        s_n = 0;
     }
     __syncthreads();
 
@@ -135,7 +137,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     // the units past them, in each pass
     auto units = [&](auto&& keep, auto&& take) {
         uint32_t turn = wv, mine = 0;
-        filter_spans(fa, q, dt0, dt1, prm.w == 1, [&](uint32_t lo, uint32_t hi) {
+        filter_spans(fa, q, t, false, [&](uint32_t lo, uint32_t hi) {
             const uint32_t len = hi - lo;
             const uint32_t nu = len ? ((lo & 3u) + len + (kFiltUnit - 1)) / kFiltUnit : 0u;
             const uint32_t incl = wave_incl_scan(nu);
@@ -145,17 +147,15 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
                 const uint32_t s = __builtin_amdgcn_readlane(lo, r), n = __builtin_amdgcn_readlane(len, r);
                 const uint32_t p = (s & ~3u) + (u - __builtin_amdgcn_readlane(incl - nu, r)) * kFiltUnit + 4u * lane;
                 auto load = [&]() {
-                    uint4 v = make_uint4(~0u, ~0u, ~0u, ~0u);
-                    if (p + 4u > s && p < s + n) {  // the array ends on a multiple of 16 bytes or past it
-                        if (p >= s && p + 4u <= s + n) {
-                            v = *reinterpret_cast<const uint4*>(a.post + p);
-                        } else {
-                            v.x = p - s < n ? a.post[p] : ~0u;
-                            v.y = p + 1u - s < n ? a.post[p + 1u] : ~0u;
-                            v.z = p + 2u - s < n ? a.post[p + 2u] : ~0u;
-                            v.w = p + 3u - s < n ? a.post[p + 3u] : ~0u;
-                        }
-                    }
+                    uint4 v = make_uint4(0, 0, 0, 0);
+                    if (p + 4u > s && p < s + n)  // (the postings are padded to whole loads)
+                        v = *reinterpret_cast<const uint4*>(a.post + p);
+                    // tile-local ids; those of other tiles and other spans are ~0
+                    const uint32_t d = p - s;
+                    v.x = d < n && v.x - obj0 < nobj ? v.x - obj0 : ~0u;
+                    v.y = d + 1u < n && v.y - obj0 < nobj ? v.y - obj0 : ~0u;
+                    v.z = d + 2u < n && v.z - obj0 < nobj ? v.z - obj0 : ~0u;
+                    v.w = d + 3u < n && v.w - obj0 < nobj ? v.w - obj0 : ~0u;
                     return v;
                 };
                 if (mine < (uint32_t)kFiltUnits)
@@ -166,50 +166,70 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
             turn = (turn + kFiltWaves - total % kFiltWaves) % kFiltWaves;
         });
     };
-    // a posting id as a tile-local one
-    auto local = [&](uint32_t id) { return id - obj0 < nobj ? id - obj0 : ~0u; };
     bool ok = true;
-    uint32_t posts = 0;
+    uint32_t posts = 0, listed = 0;
+    // the few ids that hit go on the wave's part of the list, which all lanes
+    // work off together afterwards (a hash insert by the odd lane of nearly
+    // every wave took most of the kernel's instructions); `now` when it is full
+    auto list_hit = [&](bool hit, uint32_t id, auto&& now) {
+        const uint64_t b = ballot(hit);
+        if (!b)
+            return;
+        const uint32_t at = listed + lane_prefix(b);
+        listed += (uint32_t)__popcll(b);
+        if (hit) {
+            if (at < kFiltList / kFiltWaves)
+                s_list[wv * (kFiltList / kFiltWaves) + at] = id;
+            else
+                now(id);
+        }
+    };
     auto pass1 = [&](const uint4& v) {
-        const uint32_t x[4] = {local(v.x), local(v.y), local(v.z), local(v.w)};
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
         uint32_t old[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t h = filter_bit(x[j]);
+            posts += (uint32_t)__popcll(ballot(x[j] != ~0u));
             old[j] = 0;
-            posts += x[j] != ~0u;
-            if (x[j] != ~0u)
-                old[j] = atomicOr(&s_bits[h >> 5], 1u << (h & 31u)) & 1u << (h & 31u);
+            if (x[j] != ~0u)  // (lanes without an id would meet in one word)
+                old[j] = atomicOr(&s_bits[h >> 5], 1u << (h & 31u)) >> (h & 31u) & 1u;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (old[j])
-                ok &= hash_add(s_tab, kFiltLogSlots, kb, x[j], 0u);
+            list_hit(old[j] != 0, x[j], [&](uint32_t id) { ok &= hash_add(s_tab, kFiltLogSlots, kb, id, 0u); });
+    };
+    // counts a posting of an id that is in the table (another id of its bit is not)
+    auto count = [&](uint32_t id) {
+        const uint32_t key = (id + 1u) << (32u - kb), kmask = ~0u << (32u - kb);
+        uint32_t s = (id * 0x9E3779B1u) >> (32u - kFiltLogSlots);
+        for (uint32_t probe = 0; probe < 1u << kFiltLogSlots; ++probe) {
+            const uint32_t y = s_tab[s];
+            if (y == 0)
+                break;
+            if ((y & kmask) == key) {
+                atomicAdd(&s_tab[s], w);
+                break;
+            }
+            s = (s + 1u) & ((1u << kFiltLogSlots) - 1u);
+        }
     };
     auto pass2 = [&](const uint4& v) {
-        const uint32_t x[4] = {local(v.x), local(v.y), local(v.z), local(v.w)};
+        const uint32_t x[4] = {v.x, v.y, v.z, v.w};
         uint32_t in[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t h = filter_bit(x[j]);
-            in[j] = x[j] != ~0u ? s_bits[h >> 5] >> (h & 31u) & 1u : 0u;
+            in[j] = s_bits[h >> 5] >> (h & 31u) & 1u;
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            if (in[j]) {
-                const uint32_t key = (x[j] + 1u) << (32u - kb), kmask = ~0u << (32u - kb);
-                uint32_t s = (x[j] * 0x9E3779B1u) >> (32u - kFiltLogSlots);
-                for (uint32_t probe = 0; probe < 1u << kFiltLogSlots; ++probe) {
-                    const uint32_t y = s_tab[s];
-                    if (y == 0)
-                        break;  // another id of the same bit
-                    if ((y & kmask) == key) {
-                        atomicAdd(&s_tab[s], w);
-                        break;
-                    }
-                    s = (s + 1u) & ((1u << kFiltLogSlots) - 1u);
-                }
-            }
+            list_hit(in[j] != 0 && x[j] != ~0u, x[j], count);
+    };
+    // f on the listed ids, every lane of the wave one
+    auto list_all = [&](auto&& f) {
+        for (uint32_t i = lane; i < min(listed, kFiltList / kFiltWaves); i += kWave)
+            f(s_list[wv * (kFiltList / kFiltWaves) + i]);
     };
     uint4 kept[kFiltUnits];
 #pragma unroll
@@ -225,9 +245,12 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
 #pragma unroll
     for (int i = 0; i < kFiltUnits; ++i)
         pass1(kept[i]);
-    posts = wave_sum(posts);
-    if (lane == 0)
+    list_all([&](uint32_t id) { ok &= hash_add(s_tab, kFiltLogSlots, kb, id, 0u); });
+    if (lane == 0) {
         atomicAdd(&s_posts, posts);
+        if (listed)
+            s_n = 1;
+    }
     if (!ok)
         s_res[7] = 1;
     __syncthreads();
@@ -238,26 +261,27 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
         }
         return;
     }
+    if (s_n == 0)
+        return;  // no object of two postings
     // the bits of the table's ids in place of those of every id
     for (uint32_t i = tid; i < 1u << (kFiltBitsLog - 7); i += kFiltThreads)
         reinterpret_cast<uint4*>(s_bits)[i] = make_uint4(0, 0, 0, 0);
     __syncthreads();
-    bool any = false;
 #pragma unroll
     for (uint32_t i = 0; i < (1u << kFiltLogSlots) / kFiltThreads; ++i) {
         const uint32_t y = s_tab[tid + i * kFiltThreads];
         if (y) {
             const uint32_t h = filter_bit((y >> (32u - kb)) - 1u);
             atomicOr(&s_bits[h >> 5], 1u << (h & 31u));
-            any = true;
         }
     }
-    if (!__syncthreads_or(any))
-        return;  // no object of two postings
+    listed = 0;
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < kFiltUnits; ++i)
         pass2(kept[i]);
     units([](uint32_t, auto&&) {}, pass2);
+    list_all(count);
     __syncthreads();
     hash_select(a, fa.gkey, s_tab, 1u << kFiltLogSlots, kb, q, obj0, s_res, s_red, a.kq[q], 2u * w, 0xFFFFFFFFu, true);
 }
@@ -305,7 +329,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
     __syncthreads();
     if (wv == 0) {
         uint32_t n = 0;
-        filter_spans(fa, q, 0, a.n_dtiles, true, [&](uint32_t lo, uint32_t hi) { n += hi - lo; });
+        filter_spans(fa, q, 0, true, [&](uint32_t lo, uint32_t hi) { n += hi - lo; });
         n = wave_sum(n);
         if (lane == 0)
             s_posts = n;
@@ -322,7 +346,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
         const uint32_t kb = 32u - (uint32_t)__builtin_clz(bound);  // keys are 1..bound (below 2^30)
         // f(id) for the ids below the bound, a wave a span, every 16th of 64
         auto below = [&](auto&& f) {
-            filter_spans(fa, q, 0, a.n_dtiles, false, [&](uint32_t lo, uint32_t hi) {
+            filter_spans(fa, q, 0, true, [&](uint32_t lo, uint32_t hi) {
                 const uint64_t some = ballot(hi > lo);
                 for (uint32_t r = wv; r < (uint32_t)kWave; r += kFiltWaves) {
                     if (!((some >> r) & 1u))

@@ -91,9 +91,31 @@ __global__ void __launch_bounds__(256) k_run_fill(const uint32_t* __restrict__ p
 
 // ---- per run ---------------------------------------------------------------
 
+// The key of a posting position: the buckets of the index's PosIndex leave a
+// search of a few keys (a binary search of all 524,288 keys of an LSH index
+// takes 19 dependent loads).
+struct KeyPos {
+    const uint32_t* first;
+    uint32_t n, shift;
+    const uint32_t* key_start;
+};
+
+__device__ __forceinline__ uint32_t key_at(const KeyPos& kp, uint32_t pos)
+{
+    const uint32_t b = min(pos >> kp.shift, kp.n - 1u);
+    uint32_t lo = kp.first[b], hi = kp.first[b + 1];
+    while (lo < hi) {  // first key that starts past pos
+        const uint32_t mid = (lo + hi) >> 1;
+        if (kp.key_start[mid] <= pos)
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo - 1u;
+}
+
 // First and last key of every item (items without postings get none).
-__global__ void __launch_bounds__(256) k_item_keys(const genie_dim_t* __restrict__ items, uint32_t n_items,
-                                                   const uint32_t* __restrict__ key_start, uint32_t n_keys,
+__global__ void __launch_bounds__(256) k_item_keys(const genie_dim_t* __restrict__ items, uint32_t n_items, KeyPos kp,
                                                    uint32_t* __restrict__ k0, uint32_t* __restrict__ k1)
 {
     const uint32_t i = blockIdx.x * 256u + threadIdx.x;
@@ -102,8 +124,8 @@ __global__ void __launch_bounds__(256) k_item_keys(const genie_dim_t* __restrict
     const genie_dim_t it = items[i];
     if (it.end_pos <= it.start_pos)
         return;
-    k0[i] = key_of(key_start, n_keys, (uint32_t)it.start_pos);
-    k1[i] = key_of(key_start, n_keys, (uint32_t)it.end_pos - 1);
+    k0[i] = key_at(kp, (uint32_t)it.start_pos);
+    k1[i] = key_at(kp, (uint32_t)it.end_pos - 1);
 }
 
 struct RunArgs {

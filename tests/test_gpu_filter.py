@@ -1,0 +1,69 @@
+"""Filter form of selective single-key, one-weight queries (objects of several
+postings by a bit filter, the rest from the heads of the lists) against the
+oracle's search: k past the objects of several postings, one list only, a
+weight above 1, tile counts, short lists without directory rows, empty
+queries, crowded low ids, repeated ids in set-valued lists."""
+import numpy as np
+import pytest
+
+from helpers import assert_topk_equal, oracle_search_sample, posting_items
+
+import genie_amd
+from genie_amd import Plan, Table, workloads as W
+
+pytestmark = pytest.mark.gpu
+
+
+def check(t, items, u, n, q, k, hashed=None):
+    oi, oc = oracle_search_sample(t.export()["inv"].view(np.uint32), u, n, np.broadcast_to(k, (q,)), np.arange(q))
+    kq = np.ascontiguousarray(np.broadcast_to(np.asarray(k, np.uint32), (q,)))
+    p = Plan(t.device(), q, max(1, len(items)), int(kq.max()), 0, mode=0)
+    p.upload(items, q, kq)
+    if hashed is not None:
+        assert p.hash_queries() == hashed
+    p.set_graph(True)
+    for _ in range(3):
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, q, f"n={n}")
+
+
+@pytest.mark.parametrize("n,d,buckets,k,weight", [
+    (100_000, 40, 900, 20, 1),     # one tile, lists of about 111 (no directory rows)
+    (300_000, 24, 512, 1024, 3),   # most of the result are objects of one posting
+    (600_001, 120, 2048, 60, 1),   # three tiles of 293-id lists
+    (400_000, 1, 4096, 200, 2),    # one list: k past its length
+    (2_000_003, 64, 1100, 100, 1), # eight tiles
+])
+@pytest.mark.parametrize("codec", [0, 13])
+def test_filter_equals_oracle(n, d, buckets, k, weight, codec):
+    q = 9
+    rows = genie_amd.synth.rows(n, n, d, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, buckets - 1, buckets)
+    qv, _ = genie_amd.synth.queries(n + 1, rows, q, redraw_p=0.5, n_values=buckets)
+    r = W.single_ranges(qv, 0, np.full(q * d, weight))
+    r = r[(r["query"] != 4) & ((r["query"] != 6) | (r["dim"] == 0))]  # 4 empty, 6 a single list
+    t = Table.from_rows(rows, **(dict(max_length=1024, load_balance=True, codec=codec) if codec else {}))
+    items = t.compile(r, q, merge_runs=bool(codec))
+    check(t, items, posting_items(t.export(), items) if codec else items, n, q, k)
+
+
+def test_filter_crowded_low_ids():
+    """Every matching object lies at the start of the index: the first bound of
+    the fill holds far more ids than it aims at."""
+    n, d, q = 600_000, 6, 5
+    rows = genie_amd.synth.rows(3, n, d, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 3999, 4000)
+    rows[:9000] = 4000 + np.arange(9000)[:, None] // 1500 + np.zeros(d, np.int32)
+    r = W.single_ranges(np.tile(np.arange(4000, 4000 + q)[:, None], (1, d)).astype(np.int32), 0)
+    r = r[(r["dim"] == 0) | (r["query"] > 2)]
+    t = Table.from_rows(rows)
+    items = t.compile(r, q)
+    check(t, items, items, n, q, 300)
+
+
+def test_filter_sets():
+    n, q = 500_000, 20
+    rp, v = genie_amd.synth.sets(5, n, 3, 30, 3000, 0.2)
+    qp, qv = genie_amd.synth.sets(6, q, 1, 6, 3000, 0.2)
+    t = Table.from_sets(rp, v)
+    items = t.compile(W.set_ranges(qp, qv, np.full(len(qv), 2)), q)
+    check(t, items, items, n, q, 90)
