@@ -132,6 +132,7 @@ struct genie_plan {
     uint32_t* d_hwork = nullptr;
     uint64_t hwork_alloc = 0;
     std::vector<uint32_t> h_fwork, h_fq;  // (query, tile) of the filter kernel, its queries
+    bool hash_whole = false;              // every query of the hash kernel has one tile
     std::vector<uint4> h_fhq;             // per query: directory tiles per tile, key bits, weight, tiles
     uint32_t *d_fwork = nullptr, *d_fq = nullptr;
     uint4* d_fhq = nullptr;
@@ -2578,13 +2579,17 @@ static void split_queries(genie_plan* p, bool filter)
     p->max_hash_tiles = 0;
     p->est_postings = 0;
     p->h_fhq.assign(nq, make_uint4(0, 0, 0, 0));
+    p->hash_whole = true;
     for (uint32_t q = 0; q < nq; ++q) {
         const uint64_t P = p->h_qpost[q];
         uint64_t dtpt = 0;
         uint32_t kb = 0;
         if (p->hash_mode != 0 && !p->h_force_direct[q] && (p->hash_mode == 1 || P * 16 <= N)) {
             // one weight: objects of several postings rank above those of one
-            const uint32_t w = filter && p->h_kq[q] <= kFiltMaxK && !p->h_qmulti[q] ? query_weight(p, q) : 0;
+            // (a query that one hash table holds is counted in one pass there)
+            const uint32_t w = filter && P > kHashTarget && p->h_kq[q] <= kFiltMaxK && !p->h_qmulti[q]
+                                   ? query_weight(p, q)
+                                   : 0;
             if (w) {
                 selective_tiles(p, q, kFiltTarget, kFiltTarget + kFiltTarget / 16, &dtpt, &kb);
                 if (dtpt) {
@@ -2603,6 +2608,7 @@ static void split_queries(genie_plan* p, bool filter)
                     while (lhs < (uint32_t)kHashLogMax && (1ull << lhs) < 2 * per)
                         ++lhs;
                     p->h_hq[q] = make_uint4((uint32_t)dtpt, kb, lhs, (uint32_t)nt);
+                    p->hash_whole &= nt == 1;
                 }
             }
             p->max_hash_tiles = std::max(p->max_hash_tiles, p->h_hq[q].w);
@@ -2649,6 +2655,10 @@ static int plan_split_plain(genie_plan* p)
         p->dec_spans = false;
     else if (int rc = plan_decoded_spans(p))
         return rc;
+    p->hash_whole = p->hash_whole && !p->h_hwork.empty() && (d.codec == 0 || p->dec_full);
+    if (p->hash_whole)
+        if (int rc = grow_buf(p, &p->d_sspan, &p->sspan_alloc, std::max<uint64_t>(1, p->n_items)))
+            return rc;
     if (p->h_hwork.size() > p->hwork_alloc) {
         dev_free(p->d_hwork);
         p->hwork_alloc = 0;
@@ -3015,7 +3025,13 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         h.spans = nullptr;
         h.sq_ptr = nullptr;
         const DevIndex& d = p->ix->d;
-        if (a.codec == 0) {
+        if (p->hash_whole) {
+            const uint32_t ni = (uint32_t)p->n_items;
+            k_item_spans<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, p->d_sspan);
+            h.spans = p->d_sspan;
+            h.sq_ptr = p->d_item_qptr;
+            k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
+        } else if (a.codec == 0) {
             k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
         } else if (p->dec_spans) {
             const uint32_t nj = (uint32_t)p->h_djobs.size();
@@ -3455,10 +3471,10 @@ static int plan_run_once(genie_plan* p, hipStream_t s)
     // segment runs (compressed); the kernels below write n_chunks chunks
     if (p->n_chunks > p->chunks_cap)
         return fail(GENIE_E_RUNTIME, "batch compiles into more chunks than the plan holds");
-    // chunks are read by the hash kernel and by the direct-mapped kernels over
-    // the posting lists; the filter and the scan over runs take the items and
+    // chunks are read by the hash kernel (queries of several tiles) and by the
+    // direct-mapped kernels over the posting lists; the filter and the scan over runs take the items and
     // their keys
-    const bool runs = runs_used(p), chunks = !p->h_hwork.empty() || (!runs && !p->h_dq.empty());
+    const bool runs = runs_used(p), chunks = (!p->h_hwork.empty() && !p->hash_whole) || (!runs && !p->h_dq.empty());
     if (chunks)
         if (int rc = launch_compile(p, s))
             return rc;

@@ -33,6 +33,21 @@ struct HashArgs {
     const uint32_t* sq_ptr;
 };
 
+// The work items as spans (HashArgs::spans): for queries of one tile, whose
+// items' postings are all the tile's whatever keys they cover.
+__global__ void __launch_bounds__(256) k_item_spans(const genie_dim_t* __restrict__ items, uint32_t n_items,
+                                                    Span* __restrict__ spans)
+{
+    const uint32_t i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= n_items)
+        return;
+    const genie_dim_t it = items[i];
+    Span s{0u, 0u, 0u};
+    if (it.end_pos > it.start_pos)
+        s = Span{(uint32_t)it.start_pos, (uint32_t)it.end_pos, (uint32_t)it.weight << 1 | 1u};
+    spans[i] = s;
+}
+
 // Decodes segments of a compressed index into a scratch posting array: job =
 // (segment, destination offset); one wave per job.  Two uses: the segments
 // of a batch's hash-form queries, once per query item, packed one after the
