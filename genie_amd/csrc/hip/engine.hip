@@ -288,6 +288,8 @@ static uint32_t bits_for(uint32_t bound)
     return bound <= 255 ? 8u : (bound <= 65535 ? 16u : 32u);
 }
 
+static uint32_t id_bits_for(uint32_t n) { return n <= 1 ? 1u : 32u - (uint32_t)__builtin_clz(n - 1); }
+
 static uint32_t tile_objs_for(uint32_t lane_bits) { return (uint32_t)kCntWords * (32u / lane_bits); }
 
 static void plan_drop_graph(genie_plan* p)
@@ -3503,6 +3505,7 @@ static int launch_merge(genie_plan* p, hipStream_t s)
     m.out_ids = p->d_out_ids;
     m.out_counts = p->d_out_counts;
     m.key_bits = 32 + p->lane_bits;
+    m.id_bits = id_bits_for(p->ix->d.n_objects);
     m.flag_a = p->d_overflow;
     m.flag_b = p->d_hov_any;
     m.flag_any = p->d_flag_any;
@@ -4383,6 +4386,7 @@ int genie_hip_match_topk_static(genie_index* ix, const genie_dim_t* items, uint6
     m.out_ids = v.d_out_ids;
     m.out_counts = v.d_out_counts;
     m.key_bits = 32 + lane_bits;
+    m.id_bits = id_bits_for(d.n_objects);
     m.flag_a = v.d_overflow;
     m.flag_b = v.d_hov_any;
     m.flag_any = v.d_flag_any;

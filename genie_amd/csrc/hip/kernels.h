@@ -1334,6 +1334,7 @@ struct MergeArgs {
     int32_t* out_ids;
     int32_t* out_counts;
     uint32_t key_bits;  // significant bits of a key (32 + bits of the count bound)
+    uint32_t id_bits;   // bits of an object id
     // the run's two rerun flags (candidate overflow, a hash table filled up)
     // folded into one word for an asynchronous download; every kernel that
     // sets them has finished when the merge starts
@@ -1342,18 +1343,8 @@ struct MergeArgs {
     uint32_t* flag_any;
 };
 
-// Queries with k <= kMergeSmallK and at most kMergeSmallM candidates are
-// merged by the first wave of their workgroup alone, with no workgroup
-// barrier (merge_wave).  A wave alone serializes its histogram atomics, so
-// longer candidate lists (the headline batch's ~450 a query) merge faster on
-// the whole workgroup.
-constexpr uint32_t kMergeSmallK = 128;
-constexpr uint32_t kMergeSmallM = 256;  // 4 keys per lane
-
-__device__ __forceinline__ bool merge_small(uint32_t k, uint32_t m)
-{
-    return k <= kMergeSmallK && m <= kMergeSmallM;
-}
+constexpr uint32_t kMergePacked = kMergeMaxK;  // candidates sorted whole as 32-bit words
+constexpr uint32_t kMergeWave = 8 * kWave;     // ... by one wave
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
 {
@@ -1414,101 +1405,156 @@ __device__ __forceinline__ void wave_sort_out(const MergeArgs& a, uint32_t q, ui
     }
 }
 
-// k_merge of one query by one wave (k <= 128, at most 256 candidates): the
-// candidates in registers (4 per lane), the radix select of k_merge with the
-// histogram in `hist` (256 words), the selected keys compacted into `sel`
-// (kMergeSmallK keys) and sorted descending across the lanes by a bitonic
-// network of shuffles (64 keys, one a lane, or 128, two), with no workgroup
-// barrier.
-__device__ __forceinline__ void merge_wave(const MergeArgs& a, uint32_t q, uint32_t k, uint32_t M, uint32_t* hist,
-                                           uint64_t* sel)
+// Up to 512 64-bit keys sorted through LDS by one wave, the first k written.
+__device__ __forceinline__ void merge_wave64(const MergeArgs& a, const uint64_t* keys, uint32_t q, uint32_t k, uint32_t M,
+                                             uint64_t* s)
 {
-    constexpr int PL = (int)(kMergeSmallM / kWave);
-    const int lane = lane_id();
-    const uint64_t* keys = a.cand + a.cand_base[q];
-    const uint32_t rows = (M + kWave - 1) / kWave;  // uniform
-    uint64_t v[PL];
-#pragma unroll
-    for (int j = 0; j < PL; ++j) {
-        const uint32_t i = (uint32_t)lane + (uint32_t)j * kWave;
-        v[j] = ((uint32_t)j < rows && i < M) ? keys[i] : 0ull;
-    }
-    uint64_t kth = 0;  // every key >= kth is in the result
-    if (M > k) {
-        uint64_t prefix = 0, mask = 0;
-        uint32_t remaining = k;
-        for (int shift = ((int)((a.key_bits + 7) / 8) - 1) * 8; shift >= 0; shift -= 8) {
-#pragma unroll
-            for (int b = 0; b < 4; ++b)
-                hist[lane + b * kWave] = 0;
-            wave_sync();
-#pragma unroll
-            for (int j = 0; j < PL; ++j) {
-                const uint32_t i = (uint32_t)lane + (uint32_t)j * kWave;
-                if ((uint32_t)j < rows && i < M && (v[j] & mask) == prefix)
-                    atomicAdd(&hist[(uint32_t)(v[j] >> shift) & 255u], 1u);
-            }
-            wave_sync();
-            // lane l holds bins 255 - 4l .. 252 - 4l, counted from the top
-            const uint32_t top = 255u - 4u * (uint32_t)lane;
-            uint32_t h[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                h[j] = hist[top - j];
-            const uint32_t sum = h[0] + h[1] + h[2] + h[3];
-            const uint32_t above = wave_incl_scan(sum) - sum;  // keys in higher bins
-            const bool here = above < remaining && above + sum >= remaining;
-            uint32_t bin = 0, rem = 0, inbin = 0;
-            if (here) {
-                uint32_t ab = above;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    if (ab + h[j] >= remaining) {
-                        bin = top - j;
-                        rem = remaining - ab;
-                        inbin = h[j];
-                        break;
+    const uint32_t l = (uint32_t)lane_id();
+    uint32_t n2 = kWave;
+    while (n2 < M)
+        n2 <<= 1;
+    for (uint32_t i = l; i < n2; i += kWave)
+        s[i] = i < M ? keys[i] : 0ull;
+    wave_sync();
+    for (uint32_t size = 2; size <= n2; size <<= 1)
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            for (uint32_t i = l; i < n2; i += kWave) {
+                const uint32_t j = i ^ stride;
+                if (j > i) {
+                    const uint64_t x = s[i], y = s[j];
+                    if ((i & size) == 0 ? x < y : x > y) {
+                        s[i] = y;
+                        s[j] = x;
                     }
-                    ab += h[j];
                 }
             }
-            const int src = __builtin_ctzll(ballot(here));  // exactly one lane
-            bin = (uint32_t)__shfl((int)bin, src, kWave);
-            rem = (uint32_t)__shfl((int)rem, src, kWave);
-            inbin = (uint32_t)__shfl((int)inbin, src, kWave);
-            prefix |= (uint64_t)bin << shift;
-            mask |= (uint64_t)255 << shift;
-            remaining = rem;
-            wave_sync();  // the histogram is read before the next pass clears it
-            if (inbin == rem)
-                break;  // the whole bin is needed: prefix with zero low bytes bounds it
+            wave_sync();
         }
-        kth = prefix;
+    const uint64_t o = a.out_off[q];
+    for (uint32_t i = l; i < k; i += kWave) {
+        const uint64_t key = i < min(M, n2) ? s[i] : 0ull;
+        a.out_ids[o + i] = key ? (int32_t)(~(uint32_t)key) : 0;
+        a.out_counts[o + i] = key ? (int32_t)(key >> 32) : 0;
     }
-    // the selected keys (min(M, k) of them), compacted; all of them up to
-    // kMergeSmallK are sorted, so that a select that took more (keys with
-    // bits above key_bits) still yields the k largest
-    uint32_t base = 0;
+}
+
+// Sorts E keys a lane of NW waves descending by a bitonic network, element i of
+// the order in thread i / E, register i % E: strides below E are register
+// moves, those below 64 E one shuffle each, and the few above go through LDS
+// (`x`, one word per element).
+template <int E, int NW>
+__device__ __forceinline__ void merge_network(uint32_t (&v)[E], uint32_t* x)
+{
+    const uint32_t tid = threadIdx.x;
 #pragma unroll
-    for (int j = 0; j < PL; ++j) {
-        const uint32_t i = (uint32_t)lane + (uint32_t)j * kWave;
-        const bool take = (uint32_t)j < rows && i < M && v[j] >= kth;
-        const uint64_t bm = ballot(take);
-        const uint32_t slot = base + lane_prefix(bm);
-        if (take && slot < kMergeSmallK)
-            sel[slot] = v[j];
-        base += (uint32_t)__popcll(bm);
+    for (uint32_t size = 2; size <= (uint32_t)(E * NW * kWave); size <<= 1) {
+#pragma unroll
+        for (uint32_t stride = size >> 1; stride > 0; stride >>= 1) {
+            if (stride < (uint32_t)E) {
+#pragma unroll
+                for (uint32_t r = 0; r < (uint32_t)E; ++r)
+                    if (!(r & stride)) {
+                        const bool desc = size < (uint32_t)E ? (r & size) == 0 : ((tid * E) & size) == 0;
+                        const uint32_t hi = max(v[r], v[r | stride]), lo = min(v[r], v[r | stride]);
+                        v[r] = desc ? hi : lo;
+                        v[r | stride] = desc ? lo : hi;
+                    }
+            } else {
+                // the larger of the pair stays in the lower element of a descending run
+                const bool keep_max = ((tid & (stride / E)) == 0) == (((tid * E) & size) == 0);
+                uint32_t y[E];
+                if (stride < (uint32_t)(E * kWave)) {
+#pragma unroll
+                    for (int r = 0; r < E; ++r)
+                        y[r] = (uint32_t)__shfl_xor((int)v[r], (int)(stride / E), kWave);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < E; ++r)
+                        x[r * NW * kWave + tid] = v[r];
+                    __syncthreads();
+#pragma unroll
+                    for (int r = 0; r < E; ++r)
+                        y[r] = x[r * NW * kWave + (tid ^ (stride / E))];
+                    __syncthreads();
+                }
+#pragma unroll
+                for (int r = 0; r < E; ++r)
+                    v[r] = keep_max ? max(v[r], y[r]) : min(v[r], y[r]);
+            }
+        }
     }
-    wave_sync();
-    const uint32_t nsel = min(base, kMergeSmallK);
-    uint64_t e0 = (uint32_t)lane < nsel ? sel[lane] : 0ull;
-    uint64_t e1 = (uint32_t)lane + kWave < nsel ? sel[lane + kWave] : 0ull;
-    wave_sort_out(a, q, k, e0, e1, nsel);
+}
+
+// k_merge of one query whose candidates (at most E NW 64) pack into 32 bits
+// each: (count - least + 1) << id_bits | ~id, sorted whole -- no select, no
+// 64-bit compares -- and the first k written.  False (nothing written) when the
+// counts lie too far apart for that.
+template <int E, int NW>
+__device__ __forceinline__ bool merge_packed(const MergeArgs& a, const uint64_t* keys, uint32_t q, uint32_t k, uint32_t M,
+                                             uint32_t* x, uint32_t* red)
+{
+    const uint32_t tid = threadIdx.x;
+    uint64_t key[E];
+    uint32_t lo = 0xFFFFFFFFu, hi = 0;
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const uint32_t i = (uint32_t)r * NW * kWave + tid;
+        key[r] = i < M ? keys[i] : 0ull;
+    }
+#pragma unroll
+    for (int r = 0; r < E; ++r)
+        if ((uint32_t)r * NW * kWave + tid < M) {
+            lo = min(lo, (uint32_t)(key[r] >> 32));
+            hi = max(hi, (uint32_t)(key[r] >> 32));
+        }
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+    if constexpr (NW > 1) {
+        if (lane_id() == 0) {
+            red[tid / kWave] = lo;
+            red[NW + tid / kWave] = hi;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            lo = min(lo, red[w]);
+            hi = max(hi, red[NW + w]);
+        }
+        __syncthreads();
+    }
+    if (M != 0 && (a.id_bits > 31u || ((uint64_t)(hi - lo) + 1u) >> (32u - a.id_bits) != 0))
+        return false;
+    const uint32_t idm = (1u << a.id_bits) - 1u;
+    uint32_t v[E];
+#pragma unroll
+    for (int r = 0; r < E; ++r)
+        v[r] = (uint32_t)r * NW * kWave + tid < M ? ((uint32_t)(key[r] >> 32) - lo + 1u) << a.id_bits | ((uint32_t)key[r] & idm)
+                                                  : 0u;
+    merge_network<E, NW>(v, x);
+    const uint64_t o = a.out_off[q];
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+        const uint32_t i = tid * E + r;
+        if (i < k) {
+            a.out_ids[o + i] = v[r] ? (int32_t)(~v[r] & idm) : 0;
+            a.out_counts[o + i] = v[r] ? (int32_t)((v[r] >> a.id_bits) + lo - 1u) : 0;
+        }
+    }
+    for (uint32_t i = E * NW * kWave + tid; i < k; i += NW * kWave) {
+        a.out_ids[o + i] = 0;
+        a.out_counts[o + i] = 0;
+    }
+    return true;
 }
 
 // Per query: select the k largest candidate keys (radix select over the key
 // bytes, most significant first), sort them descending, pad with (0, 0).
-// Candidates are staged in LDS when they fit; the bin holding the k-th key
+// Up to 4,096 candidates whose counts lie close enough that a 32-bit word holds
+// count and id are sorted whole instead (merge_packed; up to 512 of them by the
+// first wave alone, with no barrier): 333 queries of k = 1,000, 58 us selected
+// and sorted as 64 bits, 22 here; 384 of k = 100, 12 and 7; the headline batch,
+// 1,024 of k = 100 from ~450, 16 and 19.
+// Otherwise candidates are staged in LDS when they fit; the bin holding the k-th key
 // is found with a wave-parallel suffix scan; the select stops as soon as a
 // bin holds exactly the keys still needed.
 __global__ void __launch_bounds__(kMergeThreads) k_merge(MergeArgs a)
@@ -1524,12 +1570,26 @@ __global__ void __launch_bounds__(kMergeThreads) k_merge(MergeArgs a)
         *a.flag_any = *a.flag_a | *a.flag_b;
     const uint32_t k = a.kq[q];
     const uint32_t M = min(a.cand_cnt[q], a.cand_cap[q]);
-    if (merge_small(k, M)) {  // one wave does it (the whole workgroup decides alike, before any barrier)
-        if (tid < kWave)
-            merge_wave(a, q, k, M, s_hist, s_keys);
+    const uint64_t* keys = a.cand + a.cand_base[q];
+    uint32_t* x = reinterpret_cast<uint32_t*>(s_keys);
+    if (M <= kMergeWave) {  // the first wave's alone
+        if (tid >= kWave)
+            return;
+        const bool done = M <= kWave       ? merge_packed<1, 1>(a, keys, q, k, M, x, s_hist)
+                          : M <= 2 * kWave ? merge_packed<2, 1>(a, keys, q, k, M, x, s_hist)
+                          : M <= 4 * kWave ? merge_packed<4, 1>(a, keys, q, k, M, x, s_hist)
+                                           : merge_packed<8, 1>(a, keys, q, k, M, x, s_hist);
+        if (!done)
+            merge_wave64(a, keys, q, k, M, s_keys);
         return;
     }
-    const uint64_t* keys = a.cand + a.cand_base[q];
+    if (M <= kMergePacked) {
+        constexpr int NW = kMergeThreads / kWave;
+        if (M <= 1024   ? merge_packed<4, NW>(a, keys, q, k, M, x, s_hist)
+            : M <= 2048 ? merge_packed<8, NW>(a, keys, q, k, M, x, s_hist)
+                        : merge_packed<16, NW>(a, keys, q, k, M, x, s_hist))
+            return;
+    }
     const bool staged = M <= (uint32_t)kMergeMaxK;
     if (staged)
         for (uint32_t i = tid; i < M; i += kMergeThreads)
