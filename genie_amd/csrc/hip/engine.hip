@@ -1713,6 +1713,9 @@ int genie_hip_plan_destroy(genie_plan* p)
 
 // ---- uploads ---------------------------------------------------------------
 
+// First bytes of the pinned buffer that uploads leave alone (a download's flag).
+constexpr uint64_t kStageHead = 256;
+
 // Opens the staging of an upload: the copies of the previous one (issued by a
 // run) have left the pinned buffer before it is written again.
 static int stage_begin(genie_plan* p)
@@ -1721,7 +1724,7 @@ static int stage_begin(genie_plan* p)
         HIP_TRY(hipEventSynchronize(p->ev_up));
         p->up_pending = false;
     }
-    p->stage_used = 0;
+    p->stage_used = kStageHead;
     p->staged.clear();
     p->staging = true;
     return GENIE_OK;
@@ -1771,7 +1774,7 @@ static int h2d(genie_plan* p, T** dst, const void* src, uint64_t bytes)
         uint8_t* nb = nullptr;
         if (hipHostMalloc((void**)&nb, cap, hipHostMallocDefault) != hipSuccess)
             return fail(GENIE_E_OOM, "pinned upload buffer of " + std::to_string(cap) + " bytes");
-        if (p->stage_used)
+        if (p->h_stage && p->stage_used)
             std::memcpy(nb, p->h_stage, p->stage_used);
         if (p->h_stage)
             (void)hipHostFree(p->h_stage);
@@ -3883,9 +3886,26 @@ int genie_hip_plan_download(genie_plan* p, void* stream, int32_t* out_ids, int32
     if (!p->ran)
         return fail(GENIE_E_NOT_BUILT, "plan has not run");
     hipStream_t s = (hipStream_t)stream;
-    HIP_TRY(hipStreamSynchronize(s));
-    if (int rc = settle_overflow(p, s))
+    // the rerun flag and the rows are copied together and waited for once (the
+    // buffers may be host or device memory); only a flagged run is settled and
+    // its rows copied again
+    uint32_t* flag = reinterpret_cast<uint32_t*>(p->h_stage);  // its first words are kept for this
+    auto rows = [&]() -> int {
+        HIP_TRY(hipMemcpyAsync(out_ids, p->d_out_ids, p->total_k * 4, hipMemcpyDefault, s));
+        HIP_TRY(hipMemcpyAsync(out_counts, p->d_out_counts, p->total_k * 4, hipMemcpyDefault, s));
+        HIP_TRY(hipStreamSynchronize(s));
+        return GENIE_OK;
+    };
+    if (flag)
+        HIP_TRY(hipMemcpyAsync(flag, p->d_flag_any, 4, hipMemcpyDeviceToHost, s));
+    if (int rc = rows())
         return rc;
+    if (!flag || *flag) {
+        if (int rc = settle_overflow(p, s))
+            return rc;
+        if (int rc = rows())
+            return rc;
+    }
     if (p->timing) {
         float a = 0, b = 0, c = 0, e = 0;
         HIP_TRY(hipEventElapsedTime(&a, p->ev[0], p->ev[1]));
@@ -3901,10 +3921,6 @@ int genie_hip_plan_download(genie_plan* p, void* stream, int32_t* out_ids, int32
         p->ms_scan = b;
         p->ms_merge = c;
     }
-    // on the run's stream; the buffers may be host or device memory
-    HIP_TRY(hipMemcpyAsync(out_ids, p->d_out_ids, p->total_k * 4, hipMemcpyDefault, s));
-    HIP_TRY(hipMemcpyAsync(out_counts, p->d_out_counts, p->total_k * 4, hipMemcpyDefault, s));
-    HIP_TRY(hipStreamSynchronize(s));
     return GENIE_OK;
 }
 
