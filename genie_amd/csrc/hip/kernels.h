@@ -1603,10 +1603,23 @@ __global__ void __launch_bounds__(kMergeThreads) k_merge(MergeArgs a)
         for (int shift = ((int)((a.key_bits + 7) / 8) - 1) * 8; shift >= 0; shift -= 8) {
             s_hist[tid] = 0;  // kMergeThreads == 256 bins
             __syncthreads();
-            for (uint32_t i = tid; i < M; i += kMergeThreads) {
-                const uint64_t key = staged ? s_keys[i] : keys[i];
-                if ((key & mask) == prefix)
-                    atomicAdd(&s_hist[(uint32_t)(key >> shift) & 255u], 1u);
+            if (staged) {
+                for (uint32_t i = tid; i < M; i += kMergeThreads) {
+                    const uint64_t key = s_keys[i];
+                    if ((key & mask) == prefix)
+                        atomicAdd(&s_hist[(uint32_t)(key >> shift) & 255u], 1u);
+                }
+            } else {  // eight loads in flight
+                for (uint32_t i0 = tid; i0 < M; i0 += 8 * kMergeThreads) {
+                    uint64_t key[8];
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        key[j] = i0 + j * kMergeThreads < M ? keys[i0 + j * kMergeThreads] : 0ull;
+#pragma unroll
+                    for (int j = 0; j < 8; ++j)
+                        if (i0 + j * kMergeThreads < M && (key[j] & mask) == prefix)
+                            atomicAdd(&s_hist[(uint32_t)(key[j] >> shift) & 255u], 1u);
+                }
             }
             __syncthreads();
             if (tid < kWave) {
@@ -1639,6 +1652,14 @@ __global__ void __launch_bounds__(kMergeThreads) k_merge(MergeArgs a)
             __syncthreads();
             if (inbin == rem)
                 break;  // the whole bin is needed: prefix with zero low bytes bounds it
+            if (shift == 32 && a.id_bits <= 24u) {
+                // the id's upper bytes are the same in every key (ones, as ~id): the
+                // next pass is the first byte that an id reaches into
+                const uint32_t low = (a.id_bits + 7u) / 8u * 8u;
+                prefix |= (0xFFFFFFFFull >> low) << low;
+                mask |= (0xFFFFFFFFull >> low) << low;
+                shift = (int)low;
+            }
         }
         kth = prefix;
     }
@@ -1682,13 +1703,25 @@ __global__ void __launch_bounds__(kMergeThreads) k_merge(MergeArgs a)
             put(mine[j], i < M && mine[j] >= kth);
         }
     } else {
-        for (uint32_t i0 = 0; i0 < M; i0 += kMergeThreads) {
-            const uint32_t i = i0 + tid;
-            const uint64_t key = i < M ? keys[i] : 0;
-            put(key, i < M && key >= kth);
+        for (uint32_t i0 = tid; i0 - tid < M; i0 += 8 * kMergeThreads) {
+            uint64_t key[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                key[j] = i0 + j * kMergeThreads < M ? keys[i0 + j * kMergeThreads] : 0ull;
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                put(key[j], i0 + j * kMergeThreads < M && key[j] >= kth);
         }
     }
     __syncthreads();
+    if (n2 > 2u * kWave) {  // packed, when the selected counts allow (the stage is left alone if not)
+        constexpr int NW = kMergeThreads / kWave;
+        const uint32_t m = min(s_res[3], n2);
+        if (n2 <= 1024   ? merge_packed<4, NW>(a, s_keys, q, k, m, x, s_hist)
+            : n2 <= 2048 ? merge_packed<8, NW>(a, s_keys, q, k, m, x, s_hist)
+                         : merge_packed<16, NW>(a, s_keys, q, k, m, x, s_hist))
+            return;
+    }
     if (n2 <= 2u * kWave) {  // at most 128 selected keys: the first wave sorts and writes them
         if (tid < kWave)
             wave_sort_out(a, q, k, tid < (int)n2 ? s_keys[tid] : 0ull,
