@@ -3120,6 +3120,7 @@ static int launch_dense_t(const DenseArgs& a, hipStream_t s, int nt)
     auto grid = [&](int per) {
         n_wg = std::max(8u, (uint32_t)(per * n_cu) / 8 * 8);
         b.chunks = dense_chunks(a.G, n_wg / 8, !SAMPLE && !SETS);
+        b.sub = SAMPLE ? dense_sub(a.G, a.n_list, n_wg) : 1;
     };
     if (per_cu >= 1) {
         grid(per_cu);

@@ -94,6 +94,7 @@ struct DenseArgs {
     uint32_t D_pad, G, n_queries, n_objects, n_tiles;
     const uint32_t* list;   // tiles to visit (sample pass), null = every tile
     uint32_t n_list;
+    uint32_t sub;           // sample pass: parts of a listed tile, each a work tile of its own (dense_sub)
     uint32_t* gthr;         // [n_queries] emission threshold (>= 1)
     const uint32_t* redo;   // [G] groups to count again (null = every group)
     uint32_t* hist;         // [n_queries][kDenseBins] sample histogram
@@ -116,6 +117,17 @@ struct DenseArgs {
     // (group, chunk) pairs
     uint32_t chunks;
 };
+
+// Parts that the sample pass cuts its tiles into: as many (of 4) as the chip's
+// workgroups can take at once, since a workgroup of 1,024 threads goes over a
+// whole tile in four dependent rounds of loads and lookups.  One query over
+// 1M x 128: 8 tiles on 8 of 256 CUs take 34 us, 32 quarter tiles 17 (11 groups
+// over 300K x 77: 36 and 28 us with halves).
+__host__ __device__ inline uint32_t dense_sub(uint32_t G, uint32_t n_list, uint32_t n_wg)
+{
+    const uint64_t units = (uint64_t)G * n_list;
+    return units * 4 <= n_wg ? 4u : (units * 2 <= n_wg ? 2u : 1u);
+}
 
 // Tile chunks per group for G groups over P workgroups per XCD.  Chunk c of
 // a group takes the XCD's tiles c, c + C, c + 2 C, ...  With `balance` (the
@@ -777,7 +789,7 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_count(DenseArgs a)
     const uint32_t n_units = a.G * a.chunks, t_step = 8 * a.chunks;
     if (s >= n_units)
         return;  // the whole workgroup leaves before any barrier
-    const uint32_t n_list = a.list ? a.n_list : a.n_tiles;
+    const uint32_t n_list = a.list ? (SAMPLE ? a.n_list * a.sub : a.n_list) : a.n_tiles;
     const uint32_t tab_words = NBLK * 16 * kDenseKeysPerDim;
     const __amdgpu_buffer_rsrc_t rs = codes_rsrc(a.codes);
     const uint32_t row_bytes = a.n_pad * 4u;
@@ -907,11 +919,13 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_count(DenseArgs a)
         uint32_t staged_tiles = 0;
         const uint32_t li_end = min(n_list, w0 + win);
         for (uint32_t li = t_first + w0; li < li_end; li += t_step) {
-            const uint32_t t = a.list ? a.list[li] : li;
-            if constexpr (SAMPLE)
+            uint32_t o0 = li * kDenseTile, part = kDenseTile;
+            if constexpr (SAMPLE) {
                 __syncthreads();
-            const uint32_t o0 = t * kDenseTile;
-            const uint32_t o1 = min(o0 + kDenseTile, SETS ? a.n_slots : a.n_objects);
+                part = kDenseTile / a.sub;
+                o0 = a.list[li / a.sub] * kDenseTile + li % a.sub * part;
+            }
+            const uint32_t o1 = min(o0 + part, SETS ? a.n_slots : a.n_objects);
             for (uint32_t ol = o0 + tid; ol < o1; ol += NT) {
                 uint32_t c[NP];
                 uint32_t o = ol;
