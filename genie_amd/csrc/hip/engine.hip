@@ -1683,8 +1683,10 @@ int genie_hip_plan_estimate(const genie_index* ix, uint32_t n_queries, uint64_t 
     if (d.sm && mode != 0)  // matrix form: hot weights, window slots, tail postings sorted by tile
         b += (nq + 31) / 32 * (32ull * kSmHot + (d.sm_tiles + 1ull) * 4) + ni * 32 +
              std::min<uint64_t>(ni * d.sm_max_tail, kSmMaxEvents) * 4;
-    if (d.codec != 0 && mode != 1)  // full-layout decode scratch of the plain form
-        b += d.n_postings * 4;
+    if (d.codec != 0 && mode != 1)  // decode scratch of the plain form, full-layout and tile-major
+        b += d.n_postings * 4 + (d.run_tf ? (d.n_postings + kRunPad) * 2 : 0);
+    if (mode != 1)  // selective queries' spans: at most N / 16 postings over tiles of kFiltTarget
+        b += std::min<uint64_t>(ni * (d.n_objects / (16ull * kFiltTarget) + 1) * sizeof(uint2), 1ull << 30);
     *bytes = b;
     return GENIE_OK;
 }
@@ -3032,7 +3034,8 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         const DevIndex& d = p->ix->d;
         if (p->hash_whole) {
             const uint32_t ni = (uint32_t)p->n_items;
-            k_item_spans<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, p->d_sspan);
+            if (ni)
+                k_item_spans<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, p->d_sspan);
             h.spans = p->d_sspan;
             h.sq_ptr = p->d_item_qptr;
             k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);

@@ -67,3 +67,14 @@ def test_filter_sets():
     t = Table.from_sets(rp, v)
     items = t.compile(W.set_ranges(qp, qv, np.full(len(qv), 2)), q)
     check(t, items, items, n, q, 90)
+
+
+@pytest.mark.parametrize("mode", [0, 2])
+def test_batch_without_items(mode):
+    rows = genie_amd.synth.rows(3, 50_000, 4, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 3999, 4000)
+    t = Table.from_rows(rows)
+    p = Plan(t.device(), 3, 1, 20, 0, mode=mode)
+    p.upload(np.zeros(0, genie_amd.DIM_DTYPE), 3, np.full(3, 20, np.uint32))
+    p.run()
+    ids, cnt = p.download()
+    assert not ids.any() and not cnt.any()
