@@ -342,7 +342,7 @@ def main():
                                       identical_to_uncompressed=bool(np.array_equal(r2c[0], r2p[0]) and
                                                                      np.array_equal(r2c[1], r2p[1])))
         cp2.close()
-        kernels.append(kernel_row("k_scan_hash", "4M x 64 LSH, 4,096 queries (uncompressed)",
+        kernels.append(kernel_row("k_scan_filter", "4M x 64 LSH, 4,096 queries (uncompressed)",
                                   f2["plain"]["kernel_ms"]["scan"], lsh_compulsory,
                                   "distinct postings of the batch x 4 B (each read by one tile)"))
         d2b, _ = segment_bytes(c2.export(), ci2)
@@ -376,7 +376,7 @@ def main():
             p3.upload(i3, nq3, kq3)
             _, sets_compulsory = p3.bytes()
             p3.close()
-            kernels.append(kernel_row("k_dense_count_sets", "2M sets, 16,384 queries (set form main pass)",
+            kernels.append(kernel_row("k_set_count", "2M sets, 16,384 queries (set form main pass)",
                                       f3["batched"]["kernel_ms"]["scan"], sets_compulsory,
                                       "distinct postings of the batch x 4 B"))
         workloads["cfg3_sets"] = dict(workload="2M sets (5-40 tokens, Zipf(1.05) over 1M), 16,384 queries of "
@@ -419,7 +419,7 @@ def main():
         scan_kernel = ("k_dense_count (bit-sliced count + candidate emission, main pass)" if dense
                        else "k_scan_batched (count + select)")
     else:
-        scan_kernel = "k_scan_tile (count + select)"
+        scan_kernel = "k_scan_runs (count + select)"
     kname = scan_kernel.split()[0]
     traffic, traffic_src = profiled("traffic_bytes_per_dispatch", kname)
     lds_bytes, lds_src = profiled("lds_bytes_per_dispatch", kname)
@@ -430,7 +430,7 @@ def main():
     kernels[:0] = [kernel_row("k_dense_count", "headline batch (dense main pass + check + recount)",
                               forms["batched"]["kernel_ms"]["scan"], compulsory,
                               "distinct postings of the batch x 4 B"),
-                   kernel_row("k_scan_tile", "headline batch (plain form)", forms["plain"]["kernel_ms"]["scan"],
+                   kernel_row("k_scan_runs", "headline batch (plain form)", forms["plain"]["kernel_ms"]["scan"],
                               compulsory, "distinct postings of the batch x 4 B")]
     if lds_bytes:
         # LDS bytes the kernel reads per dispatch (profile) over its live duration
