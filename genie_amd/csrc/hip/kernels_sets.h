@@ -160,12 +160,14 @@ __global__ void __launch_bounds__(1024) k_set_events(const uint32_t* __restrict_
 }
 
 // Byte (or 16-bit) counters of one tile: a row per query, padded by 16 bytes
-// so that the rows of 8 queries start in different banks.
+// so that the rows of 8 queries start in different banks.  A byte counts from 0
+// to the 255 that the host admits, so that no addition carries into the next
+// object's; the products, whose operands are i8, read it less 128 (the top bit
+// flipped).
 template <bool W16>
 struct SmTab {
     static constexpr uint32_t kRows = W16 ? 16u : 32u;
     static constexpr uint32_t kRow = kSmTile * (W16 ? 2u : 1u) + 16u;
-    static constexpr uint32_t kZero = W16 ? 0u : 0x80808080u;  // bytes are i8: a count less 128
     // object o of the row at byte `row` of the table (a multiple of 16)
     static __device__ __forceinline__ void add(uint8_t* tab, uint32_t row, uint32_t o, uint32_t w)
     {
@@ -229,7 +231,7 @@ __global__ void __launch_bounds__(kSmThreads, 4) k_set_count(SetArgs a)
     };
 
     for (uint32_t i = tid; i < Tab::kRows * Tab::kRow / 16; i += kSmThreads)
-        s_tab4[i] = make_uint4(Tab::kZero, Tab::kZero, Tab::kZero, Tab::kZero);
+        s_tab4[i] = make_uint4(0, 0, 0, 0);
     if (tid < 32)
         s_qcnt[tid] = 0;
     if (tid == 0)
@@ -408,9 +410,8 @@ __global__ void __launch_bounds__(kSmThreads, 4) k_set_count(SetArgs a)
                             dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[i], bw[h], ci, 0, 0, 0);
                         }
                     } else {
-                        const sm_v4i cold = *reinterpret_cast<const sm_v4i*>(cell);
-                        const int z = (int)Tab::kZero;
-                        *reinterpret_cast<sm_v4i*>(cell) = sm_v4i{z, z, z, z};
+                        const sm_v4i cold = *reinterpret_cast<const sm_v4i*>(cell) ^ (int)0x80808080u;
+                        *reinterpret_cast<sm_v4i*>(cell) = sm_v4i{0, 0, 0, 0};
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
                             dd[i] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[i], bw[h], sm_v4i{0, 0, 0, 0}, 0, 0, 0);

@@ -52,6 +52,35 @@ def test_matrix_form_multiplicities():
     check(t, W.set_ranges(qp, flat, rng.integers(1, 9, len(flat))), 5000, q, 30, 0)
 
 
+@pytest.mark.parametrize("weights", [
+    [63, 63, 1], [32] * 4, [50, 50, 50, 30], [60, 60, 60], [51] * 5,  # bounds 127, 128, 180, 180, 255 of byte counters
+    [51] * 5 + [1],                                                   # 256: 16-bit counters
+    [1] * 130, [1] * 250, [2] * 125 + [1] * 5,
+])
+@pytest.mark.parametrize("holders", [4, 40])  # tail keys, mid keys
+def test_matrix_form_scattered_counts_past_127(weights, holders):
+    """Documents that hold every token of a query besides the most frequent
+    ones, at each place in a counter word, at both ends of a tile and as the
+    index's last object, beside documents that hold one of them or none; k past
+    the matches."""
+    n, m = 20_003, len(weights)
+    rng = np.random.default_rng(m)
+    docs = [np.sort(rng.choice(64, 2, replace=False)) for _ in range(n)]  # the 64 longest lists
+    at = np.concatenate([[0, 2047, 2049, n - 1], 4100 + 5 * rng.choice(3000, holders - 4, replace=False)])
+    for i, o in enumerate(at):
+        docs[o] = np.append(docs[o], 1000 + np.arange(m))
+        if i % 2 and o + 1 < n:  # a neighbour with a count of its own
+            docs[o + 1] = np.append(docs[o + 1], 1000 + i % m)
+    rp = np.concatenate([[0], np.cumsum([len(x) for x in docs])]).astype(np.int64)
+    t = Table.from_sets(rp, np.concatenate(docs).astype(np.int32))
+    assert {int(o) % 4 for o in at} >= {0, 1, 2, 3}
+    q = 3  # every token; all but one; every token and a frequent one
+    qv = [1000 + np.arange(m), 1000 + np.arange(1, m), np.append(5, 1000 + np.arange(m))]
+    wv = [weights, weights[1:], [3] + list(weights)]
+    qp = np.concatenate([[0], np.cumsum([len(x) for x in qv])])
+    check(t, W.set_ranges(qp, np.concatenate(qv).astype(np.int32), np.concatenate(wv).astype(np.int32)), n, q, 200, 0)
+
+
 def check(t, ranges, n, q, k, codec):
     items = t.compile(ranges, q, merge_runs=bool(codec))
     export = t.export()
