@@ -283,6 +283,9 @@ struct genie_plan {
     bool ran = false;
 };
 
+// Most workgroups of one launch: HIP takes fewer than 2^32 threads.
+static uint32_t launch_limit(uint32_t threads) { return 0xFFFFFFFFu / threads; }
+
 static uint32_t bits_for(uint32_t bound)
 {
     return bound <= 255 ? 8u : (bound <= 65535 ? 16u : 32u);
@@ -1136,7 +1139,7 @@ static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
         k_scan_add<<<nb, 256>>>(pre, n, sums);
         k_run_start<<<n / 256 + 1, 256>>>(pre, n, (uint32_t)d.n_postings, tf);
         if (copy)
-            k_run_fill<<<d.n_keys, 256>>>(post, d.key_start, nullptr, d.n_keys, kRunTileLog, tf, ids);
+            k_run_fill<<<std::min(d.n_keys, 65536u), 256>>>(post, d.key_start, nullptr, d.n_keys, kRunTileLog, tf, ids);
         if ((e = hipGetLastError()) == hipSuccess)
             e = hipDeviceSynchronize();
     } else {
@@ -3061,9 +3064,7 @@ static int launch_scan(genie_plan* p, hipStream_t s)
     if (nfwork) {
         FilterArgs fa;
         fa.s = a;
-        fa.work = p->d_fwork;
         fa.hq = p->d_fhq;
-        fa.fq = p->d_fq;
         fa.items = p->dec_full ? p->d_uitems : p->d_items;
         fa.n_items = (uint32_t)p->n_items;
         fa.item_qptr = p->d_item_qptr;
@@ -3072,8 +3073,15 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         fa.hov_any = p->d_hov_any;
         fa.gkey = p->d_gkey;
         k_filter_spans<<<(fa.n_items + 255) / 256, 256, 0, s>>>(fa, key_pos_of(p->ix->d));
-        k_scan_filter<<<(uint32_t)nfwork, kFiltThreads, 0, s>>>(fa);
-        k_filter_fill<<<(uint32_t)p->h_fq.size(), kFiltThreads, 0, s>>>(fa);
+        const uint64_t most = launch_limit(kFiltThreads), nfq = p->h_fq.size();
+        for (uint64_t b = 0; b < nfwork; b += most) {
+            fa.work = p->d_fwork + 2 * b;
+            k_scan_filter<<<(uint32_t)std::min(most, nfwork - b), kFiltThreads, 0, s>>>(fa);
+        }
+        for (uint64_t b = 0; b < nfq; b += most) {
+            fa.fq = p->d_fq + b;
+            k_filter_fill<<<(uint32_t)std::min(most, nfq - b), kFiltThreads, 0, s>>>(fa);
+        }
     }
     if (ndq) {
         a.qlist = ndq == p->n_queries ? nullptr : p->d_dq;
@@ -3087,11 +3095,15 @@ static int launch_scan(genie_plan* p, hipStream_t s)
             ra.item_qptr = p->d_item_qptr;
             ra.k0 = p->d_nchunks;  // k_item_keys
             ra.k1 = p->d_chunk_ptr;
-            const uint32_t nb = (uint32_t)(d.run_tiles * ndq);
-            if (p->lane_bits == 8)
-                k_scan_runs<8><<<nb, kRunThreads, 0, s>>>(ra);
-            else
-                k_scan_runs<16><<<nb, kRunThreads, 0, s>>>(ra);
+            const uint64_t nb = d.run_tiles * ndq, most = launch_limit(kRunThreads);
+            for (uint64_t b = 0; b < nb; b += most) {
+                const uint32_t n = (uint32_t)std::min(most, nb - b);
+                ra.first = (uint32_t)b;
+                if (p->lane_bits == 8)
+                    k_scan_runs<8><<<n, kRunThreads, 0, s>>>(ra);
+                else
+                    k_scan_runs<16><<<n, kRunThreads, 0, s>>>(ra);
+            }
         } else if (plain_sparse(p, a.n_tiles))
             launch_scan_t<true>(p->lane_bits, a, (uint32_t)blocks, s);
         else
@@ -3200,7 +3212,7 @@ static int launch_sets_t(SetArgs a, const uint32_t* units, uint32_t n_units, hip
     // 512 groups, 5.95 ms, against 6.28 at 32 tiles, 7.90 at 96 and 6.08 at 8; fewer tiles
     // where there are not enough units to fill the chip, 4 at least, since a
     // block sets up its table and pipeline once
-    const uint32_t cmax = std::max(1u, tiles / (SAMPLE ? 2u : 4u));
+    const uint32_t cmax = std::max(1u, std::min(tiles / (SAMPLE ? 2u : 4u), launch_limit(kSmThreads) / n_units));
     const uint32_t lo = std::min(cmax, std::max({1u, SAMPLE ? 1u : tiles / 16u, (2 * resident + n_units - 1) / n_units}));
     uint32_t best = lo;
     double waste = 1e9;

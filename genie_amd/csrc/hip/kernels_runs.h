@@ -75,17 +75,19 @@ __global__ void __launch_bounds__(256) k_run_start(const uint32_t* __restrict__ 
         tf[i] = make_uint2(total, total);
 }
 
-// One workgroup per key: its ids within the tiles (log <= 16) to their runs.
+// A workgroup per key, or every gridDim.x-th: its ids within the tiles (log <= 16) to their runs.
 __global__ void __launch_bounds__(256) k_run_fill(const uint32_t* __restrict__ post,
                                                   const uint32_t* __restrict__ key_start,
                                                   const uint32_t* __restrict__ keys, uint32_t n_keys, uint32_t log,
                                                   const uint2* __restrict__ tf, uint16_t* __restrict__ ids)
 {
-    const uint32_t r = blockIdx.x, k = keys ? keys[r] : r;
-    for (uint32_t p = key_start[k] + threadIdx.x; p < key_start[k + 1]; p += blockDim.x) {
-        const uint32_t o = post[p];
-        const uint2 f = tf[(uint64_t)(o >> log) * n_keys + r];
-        ids[f.x + (p - f.y)] = (uint16_t)(o & ((1u << log) - 1u));
+    for (uint32_t r = blockIdx.x; r < n_keys; r += gridDim.x) {
+        const uint32_t k = keys ? keys[r] : r;
+        for (uint32_t p = key_start[k] + threadIdx.x; p < key_start[k + 1]; p += blockDim.x) {
+            const uint32_t o = post[p];
+            const uint2 f = tf[(uint64_t)(o >> log) * n_keys + r];
+            ids[f.x + (p - f.y)] = (uint16_t)(o & ((1u << log) - 1u));
+        }
     }
 }
 
@@ -134,6 +136,7 @@ struct RunArgs {
     const genie_dim_t* items;   // sorted by query, posting positions
     const uint32_t* item_qptr;
     const uint32_t *k0, *k1;    // first and last key of every item
+    uint32_t first;             // (tile, query) of the launch's first workgroup
 };
 
 // A unit of a run: 512 ids from an 8-id boundary, 8 a lane.
@@ -372,8 +375,8 @@ __global__ void __launch_bounds__(kRunThreads, 8) k_scan_runs(RunArgs ra)
     const ScanArgs& a = ra.s;
     uint32_t* cnt = reinterpret_cast<uint32_t*>(s_cnt4);
     const uint32_t nql = a.qlist ? a.n_qlist : a.n_queries;
-    const uint32_t t = blockIdx.x / nql;
-    const uint32_t q = a.qlist ? a.qlist[blockIdx.x % nql] : blockIdx.x % nql;
+    const uint32_t b = ra.first + blockIdx.x, t = b / nql;
+    const uint32_t q = a.qlist ? a.qlist[b % nql] : b % nql;
     const int tid = threadIdx.x, lane = lane_id();
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     for (uint32_t i = tid; i < kWords / 4; i += kRunThreads)

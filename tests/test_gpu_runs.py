@@ -10,7 +10,7 @@ import pytest
 from helpers import assert_topk_equal, oracle_search_sample, posting_items
 
 import genie_amd
-from genie_amd import Plan, Table, workloads as W
+from genie_amd import DIM_DTYPE, Index, Plan, Table, workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -97,3 +97,51 @@ def test_runs_sets():
     t = Table.from_sets(rp, v)
     items = t.compile(W.set_ranges(qp, qv, genie_amd.synth.uniform_int(7, 0, len(qv), 1, 9)), q)
     check(t, items, items, n, q, 60, "sets")
+
+
+def test_runs_more_pairs_than_a_launch():
+    """(tile, query) pairs past what one launch of 1,024-thread workgroups
+    takes (2^32 threads)."""
+    n, q = 10_000_000, 27_500
+    rows = np.arange(n, dtype=np.int32)[:, None] % 3
+    rows[n // 2 + 1::4] = 3
+    assert -(-n // 65536) * q * 1024 > 1 << 32
+    first = np.array([np.argmax(rows[:, 0] == v) for v in range(4)])
+    t = Table.from_rows(rows)
+    v = np.random.default_rng(1).integers(0, 4, q).astype(np.int32)
+    items = t.compile(W.single_ranges(v[:, None], 0), q)
+    p = Plan(t.device(), q, len(items), 1, 0, mode=0)
+    p.set_hash(0)
+    p.upload(items, q, np.ones(q, np.uint32))
+    assert not p.sparse_active()
+    p.run()
+    ids, cnt = p.download()
+    assert np.array_equal(ids, first[v]) and (cnt == 1).all()
+
+
+def test_runs_of_more_keys_than_a_launch_of_workgroups():
+    """2^24 keys (a workgroup of 256 threads each passed 2^32 threads at index
+    creation), most of them without postings."""
+    n, K, P = 1000, (1 << 24) + 5, 3_200_000
+    rng = np.random.default_rng(2)
+    post = rng.integers(0, n, P).astype(np.uint32)
+    start = np.zeros(K + 1, np.uint64)
+    ends = np.sort(rng.choice(K - 1, P, replace=False)) + 1  # a key of one posting before each
+    start[ends] = 1
+    start[K] = 1
+    start = np.minimum(np.cumsum(start), P).astype(np.uint64)
+    ix = Index.create(n, 1, post, start, np.zeros(K, np.uint32), np.array([0, P], np.uint32), single_value=False)
+    q, k = 3, 50
+    items = np.zeros(q, DIM_DTYPE)
+    items["query"] = np.arange(q)
+    items["start_pos"] = [0, 100_000, P - 700_000]
+    items["end_pos"] = [500_000, P, P]
+    items["weight"] = 1
+    oi, oc = oracle_search_sample(post, items, n, np.full(q, k), np.arange(q))
+    p = Plan(ix, q, q, k, 65535, mode=0)
+    p.set_hash(0)
+    p.set_sparse(0)
+    p.upload(items, q, np.full(q, k, np.uint32))
+    p.run()
+    ids, cnt = p.download()
+    assert_topk_equal(ids, cnt, oi, oc, k, q, "keys")
