@@ -256,9 +256,10 @@ __device__ __forceinline__ uint32_t dense_want(uint32_t s_at, uint32_t k, uint32
     return (uint32_t)min<uint64_t>(w, n_objects);
 }
 
-// With `hshift` (set form), bin b of query q holds the sample counts
-// [b << s, (b + 1) << s), s = hshift[q], and the thresholds are bin edges:
-// S at an edge is exact, so both keep their meaning.
+// With `hshift` (set form, weighted batches), bin b of query q holds the sample
+// counts [b << s, (b + 1) << s), s = hshift[q], without the counts of 0, and
+// the thresholds are bin edges, 1 for bin 0: S at an edge is exact, so both
+// keep their meaning, and a query with few matches asks for room for those.
 __global__ void __launch_bounds__(256) k_dense_thresh(const uint32_t* __restrict__ hist,
                                                       const uint32_t* __restrict__ kq, uint32_t n_queries,
                                                       uint32_t n_sample, uint32_t n_objects, uint32_t ratio16,
@@ -285,9 +286,7 @@ __global__ void __launch_bounds__(256) k_dense_thresh(const uint32_t* __restrict
     auto largest = [&](uint32_t need) {
         return s3 >= need ? b + 3 : (s2 >= need ? b + 2 : (s1 >= need ? b + 1 : (s0 >= need ? b : 0u)));
     };
-    // With a shift, bin 0 (no higher bin reaches `need`) stands for the
-    // threshold 1, whose objects are counted in no bin of their own: at most
-    // the whole sample.
+    // bin 0 (no higher bin reaches `need`) is the threshold 1's with a shift
     const uint32_t sh = hshift ? hshift[q] : 0u, least = sh ? 0u : 1u;
     const uint32_t safe = max(wave_max(largest(k)), least);
     const uint32_t spec = max(wave_max(largest(j)), safe);
@@ -304,8 +303,8 @@ __global__ void __launch_bounds__(256) k_dense_thresh(const uint32_t* __restrict
     if (lane == 0) {
         gthr[q] = max(spec << sh, 1u);
         gsafe[q] = max(safe << sh, 1u);
-        want[q] = dense_want(spec ? at_spec : n_sample, k, ratio16, n_objects, mult);
-        want_safe[q] = dense_want(safe ? at_safe : n_sample, k, ratio16, n_objects, mult);
+        want[q] = dense_want(at_spec, k, ratio16, n_objects, mult);
+        want_safe[q] = dense_want(at_safe, k, ratio16, n_objects, mult);
     }
 }
 
@@ -746,6 +745,17 @@ __device__ __forceinline__ void dense_bin_planes(const uint32_t (&c)[NP], const 
     }
 }
 
+// The nonzero counts of bit-sliced planes, a bit each.
+template <int NP>
+__device__ __forceinline__ uint32_t dense_nonzero(const uint32_t (&c)[NP])
+{
+    uint32_t nz = 0;
+#pragma unroll
+    for (int b = 0; b < NP; ++b)
+        nz |= c[b];
+    return nz;
+}
+
 // Workgroup -> (query group, tiles) so that the groups of one tile run on one
 // XCD (workgroup ids are dealt to the 8 XCDs round robin) and each
 // workgroup loads one group's mask table once.
@@ -944,12 +954,14 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_count(DenseArgs a)
                 }
                 if constexpr (SAMPLE && SETS) {
                     // the bins as 8 planes, filed as the unit form files its
-                    // counts (queries rotated per lane, zero counts too)
+                    // counts (queries rotated per lane; a zero count adds zero)
                     static_assert(HB == 256, "8-bit bins");
                     uint32_t bp[8];
                     dense_bin_planes<NP>(c, by_shift, bp);
                     const uint32_t r = tid & 31u;
                     uint32_t cr[8];
+                    uint32_t nz = dense_nonzero<NP>(c);
+                    nz = __builtin_amdgcn_alignbit(nz, nz, r);
 #pragma unroll
                     for (int b = 0; b < 8; ++b)
                         cr[b] = __builtin_amdgcn_alignbit(bp[b], bp[b], r);  // bit j: query (j + r) mod 32
@@ -960,22 +972,23 @@ __global__ void __launch_bounds__(kDenseThreads) k_dense_count(DenseArgs a)
 #pragma unroll
                         for (int j = 0; j < 8; ++j) {
                             const uint32_t v = (uint32_t)(cnt[q] >> (8 * j)) & 255u;
-                            atomicAdd(&s_hist[((8u * q + j + r) & 31u) * HB + v], 1u);
+                            atomicAdd(&s_hist[((8u * q + j + r) & 31u) * HB + v], (nz >> (8 * q + j)) & 1u);
                         }
                 } else if constexpr (SAMPLE && WEIGHTED) {
                     // the bins as 8 planes at the queries' bit positions WP j,
-                    // transposed once; query j's bin is then byte WP j (zero
-                    // counts are filed too)
+                    // transposed once; query j's bin is then byte WP j (a zero
+                    // count adds zero)
                     static_assert(HB == 256, "8-bit bins");
                     uint32_t bp[8];
                     dense_bin_planes<NP>(c, by_shift, bp);
+                    const uint32_t nz = dense_nonzero<NP>(c);
                     uint64_t cnt[4];
                     dense_all_counts(bp, cnt);
 #pragma unroll
                     for (uint32_t jq = 0; jq < QPG; ++jq) {
                         const uint32_t p = WP * jq;
                         const uint32_t v = (uint32_t)(cnt[p >> 3] >> (8 * (p & 7))) & 255u;
-                        atomicAdd(&s_hist[jq * HB + v], 1u);
+                        atomicAdd(&s_hist[jq * HB + v], (nz >> p) & 1u);
                     }
                 } else if constexpr (SAMPLE) {
                     // lane l files query (i + l) mod 32 at step i, so that one

@@ -419,14 +419,14 @@ __global__ void __launch_bounds__(kSmThreads, 4) k_set_count(SetArgs a)
                         }
                     }
                     if constexpr (SAMPLE) {
-                        // bins >= 1 only: the thresholds read no others
+                        // nonzero counts only (k_dense_thresh)
 #pragma unroll
                         for (int i = 0; i < 4; ++i)
 #pragma unroll
                             for (int r = 0; r < 4; ++r) {
-                                const uint32_t bin = min((uint32_t)(dd[i][r] + kBias) >> shift[h], HB - 1u);
-                                if (bin)
-                                    atomicAdd(&s_hist[(16u * h + n) * HB + bin], 1u);
+                                const uint32_t c = (uint32_t)(dd[i][r] + kBias);
+                                if (c)
+                                    atomicAdd(&s_hist[(16u * h + n) * HB + min(c >> shift[h], HB - 1u)], 1u);
                             }
                     } else {
                         int m[4];
