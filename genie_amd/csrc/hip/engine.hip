@@ -529,10 +529,10 @@ int gh::validate_items(const DevIndex& d, const genie_dim_t* items, uint64_t n_i
 }
 
 static bool dense_shape(const genie_index_desc* desc, std::vector<uint32_t>& key_base, std::vector<uint32_t>& per_dim);
-static int build_sets(const genie_index_desc* desc, DevIndex& d);
+static int build_sets(const genie_index_desc* desc, DevIndex& d, const uint32_t* post);
 static int build_key_pos(DevIndex& d);
 static int build_runs(DevIndex& d, const uint32_t* post, bool copy);
-static int build_set_matrix(const genie_index_desc* desc, DevIndex& d);
+static int build_set_matrix(DevIndex& d, const uint32_t* post);
 static int build_dense(const genie_index_desc* desc, DevIndex& d, const uint32_t* post, const uint32_t* key_start);
 
 // Compressed index: words, segment offsets, key -> segment map, per-segment
@@ -739,7 +739,7 @@ static int create_compressed(const genie_index_desc* desc, genie_index** out)
         if (!rc)
             rc = build_runs(d, d_post, false);
         if (!rc)
-            rc = build_sets(desc, d);
+            rc = build_sets(desc, d, d_post);
     } while (0);
     dev_free(d_upos);
     dev_free(d_dir_keys);
@@ -1171,7 +1171,7 @@ static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
 // so that a wave reads 64 consecutive words per step and loops as often as
 // its block's longest list.  Built on the host; any other index simply has no
 // set form; only device errors fail.
-static int build_sets(const genie_index_desc* desc, DevIndex& d)
+static int build_sets(const genie_index_desc* desc, DevIndex& d, const uint32_t* post)
 {
     if (desc->single_value || !desc->postings || desc->n_postings == 0 || desc->n_keys >= (1u << 24))
         return GENIE_OK;
@@ -1249,20 +1249,21 @@ static int build_sets(const genie_index_desc* desc, DevIndex& d)
     d.blk_off = d_boff;
     d.blk_key = d_bkey;
     d.bytes += bytes;
-    return build_set_matrix(desc, d);
+    return build_set_matrix(d, post);
 }
 
 // The matrix form's copies of a set-valued table (kernels_sets.h): keys
 // classed by list length, the hot matrix and the mid keys' tile-major ids
-// built on the device.  An index of too many tiles, or a device without room,
-// has none; only device errors fail.
-static int build_set_matrix(const genie_index_desc* desc, DevIndex& d)
+// built on the device from its posting array `post` (of a compressed index, the
+// one that its words decoded to: those lists were seen to ascend).  An index of
+// too many tiles, or a device without room, has none; only device errors fail.
+static int build_set_matrix(DevIndex& d, const uint32_t* post)
 {
     const uint32_t K = d.n_keys;
     const uint64_t nt = ((uint64_t)d.n_objects + kSmTile - 1) >> kSmTileLog;
     if (nt > kSmMaxTiles)
         return GENIE_OK;
-    auto len = [&](uint32_t k) { return desc->key_start[k + 1] - desc->key_start[k]; };
+    auto len = [&](uint32_t k) { return d.h_key_start[k + 1] - d.h_key_start[k]; };
     // hot: the longest lists with multiplicities that an i8 holds; mid: the
     // next ones down to half an id per tile
     std::vector<uint32_t> order;
@@ -1308,9 +1309,8 @@ static int build_set_matrix(const genie_index_desc* desc, DevIndex& d)
                     room(&d.sm_mid_ids, n_mid_ids + kSmMidPad) && room(&d.sm_mid_ptr, n + 1ull) &&
                     (d.codec == 0 || room(&d.sm_post, d.n_postings));
     if (ok) {
-        const uint32_t* post = d.codec == 0 ? d.post : d.sm_post;
         if (d.codec != 0)
-            e = hipMemcpy(d.sm_post, desc->postings, d.n_postings * 4, hipMemcpyHostToDevice);
+            e = hipMemcpy(d.sm_post, post, d.n_postings * 4, hipMemcpyDeviceToDevice);
         if (!e)
             e = hipMemset(d.sm_hot, 0, hot_bytes);
         if (!e && !hot.empty())
@@ -1545,7 +1545,7 @@ int genie_hip_index_create(const genie_index_desc* desc, genie_index** out)
     if (!rc)
         rc = build_runs(d, d.post, true);
     if (!rc)
-        rc = build_sets(desc, d);
+        rc = build_sets(desc, d, d.post);
     if (rc) {
         genie_hip_index_destroy(ix);
         return rc;

@@ -9,7 +9,7 @@ import pytest
 from helpers import assert_topk_equal, oracle_search_sample, posting_items
 
 import genie_amd
-from genie_amd import Plan, Table, workloads as W
+from genie_amd import Index, Plan, Table, workloads as W
 
 pytestmark = pytest.mark.gpu
 
@@ -79,6 +79,32 @@ def test_matrix_form_scattered_counts_past_127(weights, holders):
     wv = [weights, weights[1:], [3] + list(weights)]
     qp = np.concatenate([[0], np.cumsum([len(x) for x in qv])])
     check(t, W.set_ranges(qp, np.concatenate(qv).astype(np.int32), np.concatenate(wv).astype(np.int32)), n, q, 200, 0)
+
+
+def test_matrix_form_of_unordered_postings():
+    """A compressed table whose posting array, beside the words, lists every
+    key's objects in descending order: the matrix form is built from the words."""
+    n, q, k = 30_000, 40, 50
+    rp, v = genie_amd.synth.sets(5, n, 3, 30, 20_000, 1.05)
+    docs = [np.unique(v[rp[i]:rp[i + 1]]) for i in range(n)]
+    rp = np.concatenate([[0], np.cumsum([len(x) for x in docs])]).astype(np.int64)
+    t = Table.from_sets(rp, np.concatenate(docs).astype(np.int32), max_length=1024, load_balance=True, codec=11)
+    e = t.export()
+    start = np.concatenate([[0], e["inv_pos"][e["keyseg"][1:]]]).astype(np.int64)
+    post = e["inv"].copy()
+    for a, b in zip(start[:-1], start[1:]):
+        post[a:b] = post[a:b][::-1]
+    ix = Index.create(n, 1, post, start, np.zeros(len(start) - 1, np.uint32), e["inv_pos"], False, 11, e["words"],
+                      e["cpos"])
+    qp, qv = genie_amd.synth.sets(6, q, 1, 40, 20_000, 1.05)
+    items = t.compile(W.set_ranges(qp, qv, np.full(len(qv), 2)), q, merge_runs=True)
+    oi, oc = oracle_search_sample(e["inv"].view(np.uint32), posting_items(e, items), n, np.full(q, k), np.arange(q))
+    p = Plan(ix, q, len(items), k, 0, mode=2)
+    p.upload(items, q, np.full(q, k, np.uint32))
+    assert p.form() == "set"
+    p.run()
+    ids, cnt = p.download()
+    assert_topk_equal(ids, cnt, oi, oc, k, q, "unordered")
 
 
 def check(t, ranges, n, q, k, codec):
