@@ -150,7 +150,8 @@ struct DevIndex {
     uint8_t* sm_hot = nullptr;      // [sm_tiles * 2048][64]
     uint16_t* sm_mid_ids = nullptr;
     uint32_t* sm_mid_ptr = nullptr; // [sm_tiles * sm_mid + 1]
-    uint32_t* sm_post = nullptr;    // compressed tables: the postings (uncompressed tables read `post`)
+    // compressed tables: the tail keys' postings and their starts (uncompressed tables read `post`)
+    uint32_t *sm_tail = nullptr, *sm_tail_start = nullptr;
     std::vector<uint32_t> h_sm_class;  // [n_keys] hot column, kSmHot + mid rank, or kSmTail
     std::vector<uint32_t> h_sm_slots;  // [sm_mid] slots of a (query, key) pair
     uint64_t bytes = 0;

@@ -1115,6 +1115,14 @@ static int build_key_pos(DevIndex& d)
     return GENIE_OK;
 }
 
+// Whether an optional copy of an index may take `bytes`: up to a quarter of
+// what is free, so that plans keep the most of it.
+static bool copy_fits(uint64_t bytes)
+{
+    size_t free_b = 0, total = 0;
+    return hipMemGetInfo(&free_b, &total) == hipSuccess && bytes <= free_b / 4;
+}
+
 // Tile-major copy of the postings for the direct-mapped scan (kernels_runs.h):
 // the directory, and with `copy` the 16-bit ids, from the device posting
 // array.  An index whose lists are too short per tile, or a device without
@@ -1125,6 +1133,9 @@ static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
     if (d.n_postings * kRunTile < (uint64_t)kRunMinPerTile * K * N || K * nt >= 0x7FFFFFFFull)
         return GENIE_OK;
     const uint32_t n = (uint32_t)(K * nt), nb = (n + 1023) / 1024;
+    const uint64_t bytes = (n + 1ull) * sizeof(uint2) + (copy ? (d.n_postings + kRunPad) * sizeof(uint16_t) : 0);
+    if (!copy_fits(bytes))
+        return GENIE_OK;
     uint32_t *cnt = nullptr, *pre = nullptr, *sums = nullptr, *total = nullptr;
     uint2* tf = nullptr;
     uint16_t* ids = nullptr;
@@ -1157,7 +1168,7 @@ static int build_runs(DevIndex& d, const uint32_t* post, bool copy)
     d.run_tf = tf;
     d.run_ids = ids;
     d.run_tiles = (uint32_t)nt;
-    d.bytes += (n + 1ull) * sizeof(uint2) + (copy ? (d.n_postings + kRunPad) * sizeof(uint16_t) : 0);
+    d.bytes += bytes;
     return GENIE_OK;
 }
 
@@ -1289,28 +1300,35 @@ static int build_set_matrix(DevIndex& d, const uint32_t* post)
         }
     }
     d.sm_max_tail = 0;
-    for (uint32_t k = 0; k < K; ++k)
-        if (d.h_sm_class[k] == kSmTail)
-            d.sm_max_tail = std::max(d.sm_max_tail, (uint32_t)len(k));
-    if (n_mid_ids >= 1ull << 30) {  // the kernels read them through 32-bit byte offsets
+    std::vector<uint32_t> tail_start(K + 1, 0);  // the tail keys' postings, one list after the other
+    for (uint32_t k = 0; k < K; ++k) {
+        const uint32_t l = d.h_sm_class[k] == kSmTail ? (uint32_t)len(k) : 0u;
+        d.sm_max_tail = std::max(d.sm_max_tail, l);
+        tail_start[k + 1] = tail_start[k] + l;
+    }
+    const uint32_t R = (uint32_t)mid.size(), n = (uint32_t)(nt * R), nb = (n + 1023) / 1024;
+    const uint64_t hot_bytes = nt * kSmTile * kSmHot;
+    const uint64_t tail_bytes = d.codec ? (tail_start[K] + K + 1ull) * 4 : 0;  // uncompressed tables read `post`
+    const uint64_t bytes = hot_bytes + (n_mid_ids + kSmMidPad) * 2 + (n + 1ull) * 4 + tail_bytes;
+    // (the kernels read the mid ids through 32-bit byte offsets)
+    if (n_mid_ids >= 1ull << 30 || !copy_fits(bytes)) {
         d.h_sm_class.clear();
         return GENIE_OK;
     }
-    const uint32_t R = (uint32_t)mid.size(), n = (uint32_t)(nt * R), nb = (n + 1023) / 1024;
     uint32_t *d_hot_keys = nullptr, *d_mid_keys = nullptr, *cnt = nullptr, *sums = nullptr, *total = nullptr;
     uint2* tf = nullptr;
     auto room = [](auto** p, uint64_t count) {
         return hipMalloc((void**)p, std::max<uint64_t>(1, count) * sizeof(**p)) == hipSuccess;
     };
     hipError_t e = hipSuccess;
-    const uint64_t hot_bytes = nt * kSmTile * kSmHot;
     const bool ok = room(&d_hot_keys, hot.size()) && room(&d_mid_keys, R) && room(&cnt, n) && room(&sums, nb) &&
                     room(&total, 1) && room(&tf, n + 1ull) && room(&d.sm_hot, hot_bytes) &&
                     room(&d.sm_mid_ids, n_mid_ids + kSmMidPad) && room(&d.sm_mid_ptr, n + 1ull) &&
-                    (d.codec == 0 || room(&d.sm_post, d.n_postings));
+                    (d.codec == 0 || (room(&d.sm_tail, tail_start[K]) && room(&d.sm_tail_start, K + 1ull)));
     if (ok) {
-        if (d.codec != 0)
-            e = hipMemcpy(d.sm_post, post, d.n_postings * 4, hipMemcpyDeviceToDevice);
+        if (d.codec != 0 &&
+            !(e = hipMemcpy(d.sm_tail_start, tail_start.data(), (K + 1ull) * 4, hipMemcpyHostToDevice)))
+            k_set_tail<<<std::min(K, 65536u), kWave>>>(post, d.key_start, d.sm_tail_start, K, d.sm_tail);
         if (!e)
             e = hipMemset(d.sm_hot, 0, hot_bytes);
         if (!e && !hot.empty())
@@ -1347,14 +1365,15 @@ static int build_set_matrix(DevIndex& d, const uint32_t* post)
         dev_free(d.sm_hot);
         dev_free(d.sm_mid_ids);
         dev_free(d.sm_mid_ptr);
-        dev_free(d.sm_post);
+        dev_free(d.sm_tail);
+        dev_free(d.sm_tail_start);
         d.h_sm_class.clear();
         return e ? fail(GENIE_E_RUNTIME, std::string("matrix form: ") + hipGetErrorString(e)) : GENIE_OK;
     }
     d.sm = true;
     d.sm_tiles = (uint32_t)nt;
     d.sm_mid = R;
-    d.bytes += hot_bytes + (n_mid_ids + kSmMidPad) * 2 + (n + 1ull) * 4 + (d.codec ? d.n_postings * 4 : 0);
+    d.bytes += bytes;
     return GENIE_OK;
 }
 
@@ -1584,7 +1603,8 @@ int genie_hip_index_destroy(genie_index* ix)
     dev_free(d.sm_hot);
     dev_free(d.sm_mid_ids);
     dev_free(d.sm_mid_ptr);
-    dev_free(d.sm_post);
+    dev_free(d.sm_tail);
+    dev_free(d.sm_tail_start);
     delete ix;
     return GENIE_OK;
 }
@@ -3316,7 +3336,8 @@ static int run_dense(genie_plan* p, hipStream_t s)
     SetArgs sa{};
     if (sm) {
         sa = set_args(p);
-        k_set_events<<<p->dn_groups, 1024, 0, s>>>(d.codec == 0 ? d.post : d.sm_post, d.key_start, p->d_sm_pairs,
+        k_set_events<<<p->dn_groups, 1024, 0, s>>>(d.codec == 0 ? d.post : d.sm_tail,
+                                                   d.codec == 0 ? d.key_start : d.sm_tail_start, p->d_sm_pairs,
                                                    p->d_sm_pair_ptr, d.sm_tiles, p->d_sm_evbase, p->d_sm_evptr,
                                                    p->d_sm_events);
         if (int rc = launch_sets<true>(p, sa, s))

@@ -96,6 +96,18 @@ __global__ void __launch_bounds__(256) k_set_hot(const uint32_t* __restrict__ po
     }
 }
 
+// The tail keys' postings one list after the other (start[k + 1] = start[k] for
+// the other keys): a wave per key, or every gridDim.x-th.
+__global__ void __launch_bounds__(kWave) k_set_tail(const uint32_t* __restrict__ post,
+                                                    const uint32_t* __restrict__ key_start,
+                                                    const uint32_t* __restrict__ start, uint32_t n_keys,
+                                                    uint32_t* __restrict__ out)
+{
+    for (uint32_t k = blockIdx.x; k < n_keys; k += gridDim.x)
+        for (uint32_t i = threadIdx.x; i < start[k + 1] - start[k]; i += kWave)
+            out[start[k] + i] = post[key_start[k] + i];
+}
+
 // ---- per run ---------------------------------------------------------------
 
 // Tail pairs (key, query | weight << 5) of each group, their postings sorted

@@ -107,6 +107,13 @@ def test_matrix_form_of_unordered_postings():
     assert_topk_equal(ids, cnt, oi, oc, k, q, "unordered")
 
 
+def test_matrix_form_keeps_a_compressed_index_small():
+    rp, v = genie_amd.synth.sets(5, 70_001, 3, 30, 40_000, 1.05)
+    plain = Table.from_sets(rp, v)
+    comp = Table.from_sets(rp, v, max_length=1024, load_balance=True, codec=11)
+    assert comp.device().bytes() < plain.device().bytes()
+
+
 def check(t, ranges, n, q, k, codec):
     items = t.compile(ranges, q, merge_runs=bool(codec))
     export = t.export()
