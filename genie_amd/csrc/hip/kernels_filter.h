@@ -308,7 +308,7 @@ __device__ __forceinline__ void fill_add(uint32_t* tab, uint32_t kb, uint32_t id
 // among the objects of one posting.  Lists ascend, so these lie in the first
 // postings of every list: all ids below a bound are counted in a table, the
 // bound first set for the number needed and doubled until enough objects of
-// one posting are below it.
+// one posting are below it, or halved back when more than the table takes are.
 __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
 {
     __shared__ uint32_t s_tab[1u << kHashLogMax];
@@ -339,8 +339,10 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
     if (posts == 0)
         return;
     // ids that should lie below the bound: those needed, the objects of more
-    // postings, and a margin
+    // postings, and a margin.  Ids crowd in places, so a bound with too many
+    // below it is halved towards the largest that had too few.
     uint64_t x = (uint64_t)a.n_objects * (need + need / 4 + 64u) / posts + 1;
+    uint32_t few = 0, many = 0;  // bounds with too few and (once met) too many ids below
     for (;;) {
         const uint32_t bound = (uint32_t)min<uint64_t>(x, a.n_objects);
         const uint32_t kb = 32u - (uint32_t)__builtin_clz(bound);  // keys are 1..bound (below 2^30)
@@ -375,14 +377,9 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
         if (lane == 0)
             atomicAdd(&s_in, in);
         __syncthreads();
-        if (s_in > kFiltFillMost) {
-            if (tid == 0) {
-                fa.hov[q] = 1u;  // too crowded for the table: the direct kernels
-                *fa.hov_any = 1u;
-            }
-            return;
-        }
-        below([&](uint32_t id) { fill_add(s_tab, kb, id); });
+        const bool crowded = s_in > kFiltFillMost;
+        if (!crowded)
+            below([&](uint32_t id) { fill_add(s_tab, kb, id); });
         __syncthreads();
         uint32_t ones = 0;
 #pragma unroll
@@ -394,11 +391,19 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
         if (lane == 0)
             atomicAdd(&s_ones, ones);
         __syncthreads();
-        if (s_ones >= need || bound == a.n_objects) {
+        if (!crowded && (s_ones >= need || bound == a.n_objects)) {
             hash_select(a, fa.gkey, s_tab, 1u << kHashLogMax, kb, q, 0, s_res, s_red, need, 1u, 1u, false, w);
             return;
         }
-        x *= 2;
+        (crowded ? many : few) = bound;
+        if (many != 0 && many - few <= 1u) {
+            if (tid == 0) {
+                fa.hov[q] = 1u;  // more at one id than the table takes: the direct kernels
+                *fa.hov_any = 1u;
+            }
+            return;
+        }
+        x = many ? few + (many - few) / 2 : 2 * x;
         __syncthreads();
     }
 }

@@ -26,6 +26,7 @@ def check(t, items, u, n, q, k, hashed=None):
         p.run()
         ids, cnt = p.download()
         assert_topk_equal(ids, cnt, oi, oc, k, q, f"n={n}")
+    return p
 
 
 @pytest.mark.parametrize("n,d,buckets,k,weight", [
@@ -58,6 +59,21 @@ def test_filter_crowded_low_ids():
     t = Table.from_rows(rows)
     items = t.compile(r, q)
     check(t, items, items, n, q, 300)
+
+
+@pytest.mark.parametrize("at", [0, 300_000])
+def test_fill_among_crowded_ids(at):
+    """Objects of one posting only, all within 9,000 ids: more of them below the
+    fill's first bound than its table takes, though few are needed."""
+    n, d, q = 600_000, 6, 3
+    rows = genie_amd.synth.rows(3, n, d, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 3999, 4000)
+    for j in range(d):
+        rows[at + 1500 * j:at + 1500 * j + 1500, j] = 5000
+    r = W.single_ranges(np.full((q, d), 5000, np.int32), 0)
+    t = Table.from_rows(rows)
+    items = t.compile(r, q)
+    p = check(t, items, items, n, q, 300, q)
+    assert p.hash_queries() == q  # none was given to the direct kernels
 
 
 def test_filter_sets():
