@@ -128,6 +128,7 @@ struct genie_plan {
     std::vector<uint4> h_hq;              // per query: directory tiles per tile, key bits, log2 slots, tiles
     std::vector<uint32_t> h_dq;           // queries of the direct-mapped kernels
     uint32_t max_hash_tiles = 0;
+    uint32_t max_hash_emits = 0;          // most selections of a hash-form query (select_parts)
     bool plain_stats = false;             // h_qpost / h_qbound hold this batch's figures
     uint32_t* d_hwork = nullptr;
     uint64_t hwork_alloc = 0;
@@ -137,7 +138,8 @@ struct genie_plan {
     uint32_t *d_fwork = nullptr, *d_fq = nullptr;
     uint4* d_fhq = nullptr;
     uint2* d_fspan = nullptr;             // [tiles][items]
-    uint64_t fwork_alloc = 0, fq_alloc = 0, fhq_alloc = 0, fspan_alloc = 0;
+    uint32_t *d_fover_n = nullptr, *d_fover = nullptr;  // [queries], [queries][max_hash_tiles] tiles whose table filled up
+    uint64_t fwork_alloc = 0, fq_alloc = 0, fhq_alloc = 0, fspan_alloc = 0, fover_n_alloc = 0, fover_alloc = 0;
     uint4* d_hq = nullptr;
     uint32_t* d_dq = nullptr;
     uint32_t* d_hov = nullptr;
@@ -352,6 +354,8 @@ static void plan_free_buffers(genie_plan* p)
     dev_free(p->d_fq);
     dev_free(p->d_fhq);
     dev_free(p->d_fspan);
+    dev_free(p->d_fover_n);
+    dev_free(p->d_fover);
     dev_free(p->d_hq);
     dev_free(p->d_dq);
     dev_free(p->d_hov);
@@ -1846,7 +1850,7 @@ static uint32_t plan_n_tiles(const genie_plan* p)
 static uint32_t max_cap_factor(const genie_plan* p)
 {
     if (!dense_active(p))
-        return std::max(plan_n_tiles(p), lane_form(p) ? 0u : p->max_hash_tiles);
+        return std::max(plan_n_tiles(p), lane_form(p) ? 0u : p->max_hash_emits);
     uint32_t kmin = 0xFFFFFFFFu;
     for (uint32_t q = 0; q < p->n_queries; ++q)
         kmin = std::min(kmin, p->h_kq[q]);
@@ -1867,6 +1871,13 @@ static uint32_t initial_cap_factor(const genie_plan* p)
 // (dense_want).
 static uint32_t dense_mult_max(const genie_plan* p) { return (p->ix->d.n_objects + 1023) / 1024; }
 
+// Selections of a hash-form query, of at most k each: one per tile, or (filter)
+// per part of a tile whose table fills up.
+static uint32_t select_parts(const genie_plan* p, uint32_t q)
+{
+    return p->h_hq[q].w * (p->h_fhq[q].w ? kFiltParts : 1u);
+}
+
 // Candidate capacity per query: cap_factor x k, at most what the form can emit.
 static int plan_size_candidates(genie_plan* p)
 {
@@ -1881,10 +1892,8 @@ static int plan_size_candidates(genie_plan* p)
         // the dense form emits each object at most once; the tile forms at
         // most k per tile (a hash-form query: per tile of its own)
         uint64_t tiles = n_tiles;
-        if (plain && q < p->h_hq.size() && p->h_hq[q].x) {
-            const uint64_t tobj = (uint64_t)p->h_hq[q].x * kDirTile;
-            tiles = (p->ix->d.n_objects + tobj - 1) / tobj;
-        }
+        if (plain && q < p->h_hq.size() && p->h_hq[q].x)
+            tiles = select_parts(p, q);
         const uint64_t limit = dn ? (uint64_t)p->ix->d.n_objects : tiles * p->h_kq[q];
         // the dense form's device sizing lays each query's ask out in this
         // total; a query whose counts crowd at its threshold asks for its
@@ -2606,7 +2615,7 @@ static void split_queries(genie_plan* p, bool filter)
     p->h_fq.clear();
     p->h_dq.clear();
     p->h_hq.assign(nq, make_uint4(0, 0, 0, 0));
-    p->max_hash_tiles = 0;
+    p->max_hash_tiles = p->max_hash_emits = 0;
     p->est_postings = 0;
     p->h_fhq.assign(nq, make_uint4(0, 0, 0, 0));
     p->hash_whole = true;
@@ -2642,6 +2651,7 @@ static void split_queries(genie_plan* p, bool filter)
                 }
             }
             p->max_hash_tiles = std::max(p->max_hash_tiles, p->h_hq[q].w);
+            p->max_hash_emits = std::max(p->max_hash_emits, select_parts(p, q));
         }
         if (!dtpt) {
             p->h_dq.push_back(q);
@@ -2707,6 +2717,10 @@ static int plan_split_plain(genie_plan* p)
         if (int rc = grow_buf(p, &p->d_fhq, &p->fhq_alloc, nq))
             return rc;
         if (int rc = grow_buf(p, &p->d_fspan, &p->fspan_alloc, filter_span_count(p)))
+            return rc;
+        if (int rc = grow_buf(p, &p->d_fover_n, &p->fover_n_alloc, nq))
+            return rc;
+        if (int rc = grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles))
             return rc;
         if (int rc = h2d(p, &p->d_fhq, p->h_fhq.data(), nq * sizeof(uint4)))
             return rc;
@@ -2779,9 +2793,11 @@ static int plan_upload(genie_plan* p, const genie_dim_t* items, uint64_t n_items
     p->plain_stats = false;
     p->h_force_direct.assign(n_queries, 0);
     p->h_hwork.clear();
+    p->h_fwork.clear();
+    p->h_fq.clear();
     p->h_dq.clear();
     p->h_hq.clear();
-    p->max_hash_tiles = 0;
+    p->max_hash_tiles = p->max_hash_emits = 0;
     // count bound of this batch
     if (p->count_bound == 0) {
         if (p->dense_ok && p->dense_wp == 1) {
@@ -3089,6 +3105,9 @@ static int launch_scan(genie_plan* p, hipStream_t s)
         fa.n_items = (uint32_t)p->n_items;
         fa.item_qptr = p->d_item_qptr;
         fa.spans = p->d_fspan;
+        fa.over_n = p->d_fover_n;
+        fa.over = p->d_fover;
+        fa.max_tiles = p->max_hash_tiles;
         fa.hov = p->d_hov;
         fa.hov_any = p->d_hov_any;
         fa.gkey = p->d_gkey;

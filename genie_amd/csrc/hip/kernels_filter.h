@@ -5,12 +5,16 @@
 // k_scan_hash inserts every posting into an LDS hash table (a compare-and-swap
 // and its probes each, eight tiles and eight radix selects a query on LSH
 // batches) to find that out.  Here a tile's ids first go through a bit per
-// hashed id: an id that meets its bit set is entered in a small table; a second
-// pass over the same ids (kept in registers) counts those that are in the
-// table, so that every object of two or more postings has its exact count.
-// Tiles hold four times the postings.  Queries left with fewer than k such
-// objects take the smallest ids among the objects of one posting
-// (k_filter_fill).
+// hashed id: an id that meets its bit set is entered in a small table and
+// counted; a second pass over the same ids (kept in registers) counts those that
+// met it clear, where they are in the table, so that every object of two or more
+// postings has its exact count.
+// Tiles hold four times the postings.  A tile whose table fills up (many of its
+// objects have several postings, as where buckets go together), or with far
+// more postings than its share, is counted by k_filter_fill, a quarter at a
+// time with every id in the table.  Queries left
+// with fewer than k such objects take the smallest ids among the objects of one
+// posting (k_filter_fill).
 #pragma once
 #include "kernels_hash.h"
 #include "kernels_runs.h"
@@ -22,10 +26,15 @@ constexpr int kFiltWaves = kFiltThreads / kWave;
 constexpr uint32_t kFiltBitsLog = 18;          // 32 KiB of bits: 1 in 16 set when a full tile is done
 constexpr uint32_t kFiltLogSlots = 13;         // table slots, 32 KiB
 constexpr uint32_t kFiltTarget = 16384;        // postings per (query, tile) aimed at
-constexpr uint32_t kFiltMost = kFiltTarget + kFiltTarget / 8;  // a tile of more flags its query for the direct kernels
+constexpr uint32_t kFiltMost = kFiltTarget + kFiltTarget / 8;  // bits set: a tile of more is counted in parts
+constexpr uint32_t kFiltParts = 4;             // parts of a tile whose table fills up
+constexpr uint32_t kFiltProbes = 256;          // taken slots in a row after which the table counts as full,
+constexpr uint32_t kFiltPartProbes = 1024;     // ... and a part's (97% of the slots)
 constexpr uint32_t kFiltMaxK = 1024;
 constexpr uint32_t kFiltUnit = 4 * kWave;      // ids a wave loads at a time, 16 bytes a lane
 constexpr int kFiltUnits = 5;                  // units a wave keeps in registers
+constexpr uint32_t kFiltSeen = 8;              // units of a wave whose hits pass 1 counts, a bit an id
+constexpr uint32_t kFiltLater = 1u << 31;      // an entered id that pass 2 counts (ids are below 2^30)
 constexpr uint32_t kFiltList = 2048;           // ids on their way into (or counted in) the table, a part a wave
 constexpr uint32_t kFiltFillMost = (1u << kHashLogMax) / 4 * 3;  // postings k_filter_fill enters in its table
 
@@ -38,6 +47,9 @@ struct FilterArgs {
     uint32_t n_items;
     const uint32_t* item_qptr;
     uint2* spans;               // [tiles][n_items] every item's postings that can hold ids of the tile
+    uint32_t* over_n;           // [n_queries] tiles to count in parts
+    uint32_t* over;             // [n_queries][max_tiles] these tiles
+    uint32_t max_tiles;
     uint32_t* hov;
     uint32_t* hov_any;
     unsigned long long* gkey;
@@ -56,6 +68,7 @@ __global__ void __launch_bounds__(256) k_filter_spans(FilterArgs fa, KeyPos kp)
     if (prm.w == 0)
         return;
     const ScanArgs& a = fa.s;
+    fa.over_n[it.query] = 0;
     const bool empty = it.end_pos <= it.start_pos || it.weight == 0.0f;
     const uint32_t sp = empty ? 0u : (uint32_t)it.start_pos, ep = empty ? 0u : (uint32_t)it.end_pos;
     uint32_t ks = 0, doff = kNoDir;
@@ -103,7 +116,10 @@ __device__ __forceinline__ uint32_t filter_bit(uint32_t loc)
 // One workgroup per (query, tile).  Ids are kept tile-local; lanes past a
 // span's end, and ids of other tiles, hold 0xFFFFFFFF.
 // 4M x 64 LSH (8,192 buckets), 4,096 queries: k_scan_hash 1.20 ms; here the
-// spans 21 us, this kernel 508 us and the fill 26 us.
+// spans 21 us, this kernel 475 us (488 when pass 1 entered without counting and
+// pass 2 counted every posting) and the fill 25 us.  Where four fifths of a
+// 1,000-object cluster share a bucket (1M x 64 in 4,096 buckets), 1,024
+// queries: k_scan_hash 306 us, here 317; a tenth of 3,000: 1,270 and 165.
 __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
 {
     __shared__ uint32_t s_bits[1u << (kFiltBitsLog - 5)];
@@ -111,7 +127,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     __shared__ uint32_t s_red[3 * kMaxWaves];
     __shared__ uint32_t s_res[8];
     __shared__ uint32_t s_list[kFiltList];
-    __shared__ uint32_t s_posts;  // ids of this tile
+    __shared__ uint32_t s_set;    // bits set
     __shared__ uint32_t s_n;      // some id is listed
     const ScanArgs& a = fa.s;
     const uint32_t q = fa.work[2 * blockIdx.x], t = fa.work[2 * blockIdx.x + 1];
@@ -127,7 +143,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
         reinterpret_cast<uint4*>(s_tab)[i] = make_uint4(0, 0, 0, 0);
     if (tid == 0) {
         s_res[7] = 0;
-        s_posts = 0;
+        s_set = 0;
         s_n = 0;
     }
     __syncthreads();
@@ -161,13 +177,21 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
                 if (mine < (uint32_t)kFiltUnits)
                     keep(mine, load);
                 else
-                    take(load());
+                    take(load(), mine);
             }
             turn = (turn + kFiltWaves - total % kFiltWaves) % kFiltWaves;
         });
     };
-    bool ok = true;
-    uint32_t posts = 0, listed = 0;
+    uint32_t bits = 0, seen = 0, listed = 0;
+    auto enter = [&](uint32_t id) {
+        if (!hash_add(s_tab, kFiltLogSlots, kb, id & ~kFiltLater, id & kFiltLater ? 0u : w, kFiltProbes))
+            s_res[7] = 1;
+    };
+    // past the list: none is tried once one has failed (each goes past kFiltProbes slots)
+    auto enter_now = [&](uint32_t id) {
+        if (!*(volatile uint32_t*)&s_res[7])
+            enter(id);
+    };
     // the few ids that hit go on the wave's part of the list, which all lanes
     // work off together afterwards (a hash insert by the odd lane of nearly
     // every wave took most of the kernel's instructions); `now` when it is full
@@ -184,20 +208,23 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
                 now(id);
         }
     };
-    auto pass1 = [&](const uint4& v) {
+    auto pass1 = [&](const uint4& v, uint32_t m) {  // the wave's unit m
         const uint32_t x[4] = {v.x, v.y, v.z, v.w};
         uint32_t old[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             const uint32_t h = filter_bit(x[j]);
-            posts += (uint32_t)__popcll(ballot(x[j] != ~0u));
             old[j] = 0;
             if (x[j] != ~0u)  // (lanes without an id would meet in one word)
                 old[j] = atomicOr(&s_bits[h >> 5], 1u << (h & 31u)) >> (h & 31u) & 1u;
         }
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            list_hit(old[j] != 0, x[j], [&](uint32_t id) { ok &= hash_add(s_tab, kFiltLogSlots, kb, id, 0u); });
+        for (int j = 0; j < 4; ++j) {
+            bits += (uint32_t)__popcll(ballot(x[j] != ~0u && !old[j]));
+            if (m < kFiltSeen)  // uniform
+                seen |= old[j] << (4u * m + j);
+            list_hit(old[j] != 0, m < kFiltSeen ? x[j] : x[j] | kFiltLater, enter_now);
+        }
     };
     // counts a posting of an id that is in the table (another id of its bit is not)
     auto count = [&](uint32_t id) {
@@ -214,7 +241,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
             s = (s + 1u) & ((1u << kFiltLogSlots) - 1u);
         }
     };
-    auto pass2 = [&](const uint4& v) {
+    auto pass2 = [&](const uint4& v, uint32_t m) {
         const uint32_t x[4] = {v.x, v.y, v.z, v.w};
         uint32_t in[4];
 #pragma unroll
@@ -224,7 +251,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
         }
 #pragma unroll
         for (int j = 0; j < 4; ++j)
-            list_hit(in[j] != 0 && x[j] != ~0u, x[j], count);
+            list_hit(in[j] != 0 && x[j] != ~0u && (m >= kFiltSeen || !((seen >> (4u * m + j)) & 1u)), x[j], count);
     };
     // f on the listed ids, every lane of the wave one
     auto list_all = [&](auto&& f) {
@@ -244,21 +271,17 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     }, pass1);
 #pragma unroll
     for (int i = 0; i < kFiltUnits; ++i)
-        pass1(kept[i]);
-    list_all([&](uint32_t id) { ok &= hash_add(s_tab, kFiltLogSlots, kb, id, 0u); });
+        pass1(kept[i], (uint32_t)i);
+    list_all(enter);
     if (lane == 0) {
-        atomicAdd(&s_posts, posts);
+        atomicAdd(&s_set, bits);
         if (listed)
             s_n = 1;
     }
-    if (!ok)
-        s_res[7] = 1;
     __syncthreads();
-    if (s_res[7] || s_posts > kFiltMost) {
-        if (tid == 0) {
-            fa.hov[q] = 1u;
-            *fa.hov_any = 1u;
-        }
+    if (s_res[7] || s_set > kFiltMost) {
+        if (tid == 0)
+            fa.over[(uint64_t)q * fa.max_tiles + atomicAdd(&fa.over_n[q], 1u)] = t;
         return;
     }
     if (s_n == 0)
@@ -279,7 +302,7 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_scan_filter(FilterArgs fa)
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < kFiltUnits; ++i)
-        pass2(kept[i]);
+        pass2(kept[i], (uint32_t)i);
     units([](uint32_t, auto&&) {}, pass2);
     list_all(count);
     __syncthreads();
@@ -304,6 +327,8 @@ __device__ __forceinline__ void fill_add(uint32_t* tab, uint32_t kb, uint32_t id
     }
 }
 
+// First the query's tiles left to be counted in parts: the objects of several
+// postings of a quarter at a time, every posting counted in the table.
 // Queries that the filter left with fewer than k candidates: the smallest ids
 // among the objects of one posting.  Lists ascend, so these lie in the first
 // postings of every list: all ids below a bound are counted in a table, the
@@ -317,13 +342,59 @@ __global__ void __launch_bounds__(kFiltThreads, 8) k_filter_fill(FilterArgs fa)
     __shared__ uint32_t s_posts, s_in, s_ones;
     const ScanArgs& a = fa.s;
     const uint32_t q = fa.fq[blockIdx.x];
-    const uint32_t k = a.kq[q], have = a.cand_cnt[q];
-    if (have >= k || fa.hov[q])
+    const uint32_t k = a.kq[q], n_over = fa.over_n[q];
+    uint32_t have = a.cand_cnt[q];
+    if (have >= k && n_over == 0)
         return;
-    const uint32_t need = k - have;
     const uint32_t w = fa.hq[q].z;
     const uint32_t tid = threadIdx.x, lane = lane_id();
     const uint32_t wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+#pragma unroll 1
+    for (uint32_t i = 0; i < n_over * kFiltParts; ++i) {
+        const uint32_t t = fa.over[(uint64_t)q * fa.max_tiles + i / kFiltParts];
+        const uint32_t part = fa.hq[q].x * (kDirTile / kFiltParts), tile0 = t * fa.hq[q].x * kDirTile;
+        const uint32_t o0 = tile0 + i % kFiltParts * part;  // ids [o0, o0 + part), keys from the part's start
+        if (o0 >= a.n_objects)
+            continue;
+        for (uint32_t j = tid; j < 1u << kHashLogMax; j += kFiltThreads)
+            s_tab[j] = 0;
+        if (tid == 0)
+            s_res[7] = 0;
+        __syncthreads();
+        filter_spans(fa, q, t, false, [&](uint32_t lo, uint32_t hi) {
+            const uint64_t some = ballot(hi > lo);
+            for (uint32_t r = wv; r < (uint32_t)kWave; r += kFiltWaves) {
+                if (!((some >> r) & 1u))
+                    continue;
+                const uint32_t s = __builtin_amdgcn_readlane(lo, r), e = __builtin_amdgcn_readlane(hi, r);
+                for (uint32_t p = s + lane; p < e; p += kWave) {
+                    const uint32_t loc = a.post[p] - o0;
+                    if (loc < part && !*(volatile uint32_t*)&s_res[7] &&
+                        !hash_add(s_tab, kHashLogMax, fa.hq[q].y, loc, w, kFiltPartProbes))
+                        s_res[7] = 1;
+                }
+            }
+        });
+        __syncthreads();
+        if (s_res[7]) {
+            if (tid == 0) {
+                fa.hov[q] = 1u;  // the direct kernels
+                *fa.hov_any = 1u;
+            }
+            return;
+        }
+        hash_select(a, fa.gkey, s_tab, 1u << kHashLogMax, fa.hq[q].y, q, o0, s_res, s_red, k, 2u * w, 0xFFFFFFFFu, true);
+        __syncthreads();
+    }
+    if (n_over) {  // the loop added to it
+        if (tid == 0)
+            s_in = __hip_atomic_load(&a.cand_cnt[q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        __syncthreads();
+        have = s_in;
+    }
+    if (have >= k)
+        return;
+    const uint32_t need = k - have;
     if (tid == 0)
         s_posts = 0;
     __syncthreads();

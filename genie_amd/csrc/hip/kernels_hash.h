@@ -151,14 +151,16 @@ __global__ void __launch_bounds__(kDecodeWaves * kWave) __attribute__((amdgpu_wa
 // Adds w to the count of tile-local id `loc`.  A slot word holds key = loc + 1
 // in its high kb bits and the count in the low 32 - kb bits (the host sizes
 // kb and checks that every count fits); 0 is an empty slot.  Linear probing
-// from a multiplicative hash; false when the table is full.
-__device__ __forceinline__ bool hash_add(uint32_t* tab, uint32_t lhs, uint32_t kb, uint32_t loc, uint32_t w)
+// from a multiplicative hash; false when the table is full (`probes`: when that
+// many slots in a row are).
+__device__ __forceinline__ bool hash_add(uint32_t* tab, uint32_t lhs, uint32_t kb, uint32_t loc, uint32_t w,
+                                         uint32_t probes = 1u << kHashLogMax)
 {
     const uint32_t key = (loc + 1u) << (32u - kb);
     const uint32_t kmask = ~0u << (32u - kb);
     const uint32_t smask = (1u << lhs) - 1u;
     uint32_t h = (loc * 0x9E3779B1u) >> (32u - lhs);
-    for (uint32_t probe = 0; probe <= smask; ++probe) {
+    for (uint32_t probe = 0; probe <= smask && probe < probes; ++probe) {
         // claim an empty slot outright (most ids of a selective query arrive
         // once); a taken slot returns its word
         const uint32_t v = atomicCAS(&tab[h], 0u, key | w);

@@ -76,6 +76,31 @@ def test_fill_among_crowded_ids(at):
     assert p.hash_queries() == q  # none was given to the direct kernels
 
 
+@pytest.mark.parametrize("n,shared,span,k", [
+    (2_000_000, 9000, 900_000, 60),       # two tiles, every id in the first: its table fills up
+    (2_000_000, 9000, 900_000, 1024),
+    (4_000_000, 16_200, 1_900_000, 700),  # two tiles, more bits set than a tile's share
+    (2_000_000, 8100, 900_000, 60),       # nearly full
+])
+def test_filter_tiles_of_many_shared_objects(n, shared, span, k):
+    """Objects that share two or three of a query's values, more of them in a
+    tile than the table of the filter takes: counted in quarters."""
+    d, q = 8, 6
+    rng = np.random.default_rng(shared)
+    rows = genie_amd.synth.rows(3, n, d, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 3999, 4000)
+    at = rng.choice(span, shared, replace=False)
+    i = np.arange(shared)
+    for e in (0, 1):
+        rows[at, (i + e) % d] = 5000
+    rows[at[::50], (i[::50] + 2) % d] = 5000
+    r = W.single_ranges(np.full((q, d), 5000, np.int32), 0, np.full(q * d, 2))
+    r = r[(r["query"] != 1) | (r["dim"] < 6)]
+    t = Table.from_rows(rows)
+    items = t.compile(r, q)
+    p = check(t, items, items, n, q, k, q)
+    assert p.hash_queries() == q  # none was given to the direct kernels
+
+
 def test_filter_sets():
     n, q = 500_000, 20
     rp, v = genie_amd.synth.sets(5, n, 3, 30, 3000, 0.2)
