@@ -21,6 +21,7 @@ pytestmark = pytest.mark.gpu
     (70_001, 70, 40_000, 1.05, 4, 50),   # hot, mid and tail keys
     (70_001, 40, 40_000, 1.05, 60, 50),  # 16-bit counters
     (30_000, 100, 30_000, 0.0, 1, 20),   # a flat vocabulary: short runs, many ties
+    (40_001, 64, 1500, 0.0, 1, 30),      # ties that half fill a tile's stage
 ])
 @pytest.mark.parametrize("codec", [0, 11])
 def test_matrix_form_equals_oracle(n, q, vocab, skew, wmax, k, codec):
