@@ -1267,6 +1267,32 @@ static int build_sets(const genie_index_desc* desc, DevIndex& d, const uint32_t*
     return build_set_matrix(d, post);
 }
 
+// The choice between the two set forms: time per group and tile, in ns, fitted to
+// 240 measured batches (60,000 to 1M documents of 1-140 tokens, flat and Zipf
+// vocabularies of 150 to 200,000, 48 and 1,024 queries of up to 8 and 40 tokens,
+// weights to 1 and 20).  The forms differ by
+//   the lists:   8 + 1.5 a token of the mean document;
+//   the matrix:  3.6 (4.2 with 16-bit counters) for every 512 window slots past
+//                the 1,024 that its workgroups keep in registers, and 0.02 a tail
+//                posting, of which a group's are sorted by one workgroup (0.6 for
+//                a group alone);
+// each over the share of the chip that it fills: the matrix form's blocks of 4
+// tiles at least and two a CU, the lists' 4,096-object tiles.  The faster form is
+// chosen but for 5 of the 240 (0.88 of the other's speed at worst); slots and
+// token counts alone chose the slower one 22 times (0.46 at worst).
+static double set_lists_ns(const DevIndex& d, uint32_t G)
+{
+    const double fill = std::min(1.0, (double)G * ((d.sm_tiles + 1) / 2) / 512.0);
+    return G * (8.0 + 1.5 * (double)d.n_postings / std::max(1u, d.n_objects) / fill);
+}
+
+// Window slots of G groups past which the lists are chosen whatever else a batch
+// holds.
+static uint64_t set_matrix_slots(const DevIndex& d, uint32_t G)
+{
+    return (uint64_t)((kSmSlots * G + set_lists_ns(d, G) / 3.6) * kSmThreads);
+}
+
 // The matrix form's copies of a set-valued table (kernels_sets.h): keys
 // classed by list length, the hot matrix and the mid keys' tile-major ids
 // built on the device from its posting array `post` (of a compressed index, the
@@ -1707,9 +1733,12 @@ int genie_hip_plan_estimate(const genie_index* ix, uint32_t n_queries, uint64_t 
     if (dense)  // query-mask tables per group (8 queries at the fewest) and the sample histograms
         b += (nq + 7) / 8 * (uint64_t)std::max<uint32_t>(d.dense_dpad, 1) * kDenseKeysPerDim * 4 +
              nq * kDenseBins * 4ull;
-    if (d.sm && mode != 0)  // matrix form: hot weights, window slots, tail postings sorted by tile
-        b += (nq + 31) / 32 * (32ull * kSmHot + (d.sm_tiles + 1ull) * 4) + ni * 32 +
+    if (d.sm && mode != 0) {  // matrix form: hot weights, window slots, tail postings sorted by tile
+        const uint32_t per = d.h_sm_slots.empty() ? 1u : *std::max_element(d.h_sm_slots.begin(), d.h_sm_slots.end());
+        b += (nq + 31) / 32 * (32ull * kSmHot + (d.sm_tiles + 1ull) * 4) +
+             std::min(ni * per, set_matrix_slots(d, (n_queries + 31) / 32)) * sizeof(uint2) + ni * sizeof(uint2) +
              std::min<uint64_t>(ni * d.sm_max_tail, kSmMaxEvents) * 4;
+    }
     if (d.codec != 0 && mode != 1)  // decode scratch of the plain form, full-layout and tile-major
         b += d.n_postings * 4 + (d.run_tf ? (d.n_postings + kRunPad) * 2 : 0);
     if (mode != 1)  // selective queries' spans: at most N / 16 postings over tiles of kFiltTarget
@@ -2017,9 +2046,11 @@ struct SetMatrixBatch {
     uint32_t G, g = 0;
     bool wide = false;  // some query of the group needs 16-bit counters
     bool on;
+    uint64_t slots_limit = 0;
     std::vector<std::pair<uint32_t, uint32_t>> cold;  // weight, multiplicity
     SetMatrixBatch(genie_plan* plan, uint32_t groups) : p(plan), d(plan->ix->d), G(groups), on(d.sm)
     {
+        slots_limit = on ? set_matrix_slots(d, G) : 0;
         p->sm_ok = false;
         p->h_sm_slots.clear();
         p->h_sm_pairs.clear();
@@ -2079,25 +2110,28 @@ struct SetMatrixBatch {
         } else {
             p->h_sm_units8.push_back(g);
         }
-        if (p->sm_events > kSmMaxEvents)
-            on = false;
-        else if (g + 1 < G)
+        if (p->sm_events > kSmMaxEvents || p->h_sm_slots.size() > slots_limit) {
+            on = false;  // the lists will be faster, or have to do
+            std::vector<uint2>().swap(p->h_sm_slots);
+            std::vector<uint2>().swap(p->h_sm_pairs);
+            return;
+        }
+        if (g + 1 < G)
             p->h_sm_evbase[g + 1] = (uint32_t)p->sm_events;
         wide = false;
         ++g;
     }
-    // The matrix form costs a group and tile about 6,000 CU cycles whatever the
-    // documents hold, and 1,260 for every 512 window slots past the 1,024 that
-    // its workgroups keep in registers; the forward lists about 1,030 for every
-    // token of the mean document.  Skewed tables have few slots (2M documents,
-    // Zipf(1.05): 22.6 ms on the lists, 6.0 here); a uniform vocabulary of 300
-    // has 18,000 of them (1.4 ms on the lists, 3.0 here); they meet at 750 per
-    // token (uniform over 2,000: 1.73 and 1.70 ms).
+    // Whether the matrix form is the faster one (set_lists_ns).
     bool finish() const
     {
-        const double slots = (double)p->h_sm_slots.size() / std::max(1u, G);
-        const double mean_len = (double)d.n_postings / std::max(1u, d.n_objects);
-        return on && 1260.0 * (slots / kSmThreads - kSmSlots) <= 750.0 * mean_len;
+        if (!on)
+            return false;
+        const double wide_groups = (double)p->h_sm_units16.size() / 2;
+        const double past = std::max(0.0, (double)p->h_sm_slots.size() / G / kSmThreads - kSmSlots);
+        const double tail = (double)p->sm_events / G / d.sm_tiles;
+        const double fill = std::min(1.0, (G + wide_groups) * std::max(1u, d.sm_tiles / 4) / 512.0);
+        return ((3.6 * (G - wide_groups) + 4.2 * wide_groups) * past) / fill + std::max(0.02 * G / fill, 0.6) * tail <=
+               set_lists_ns(d, G);
     }
 };
 
