@@ -93,6 +93,11 @@ using namespace gh;
 // Plan
 // ===========================================================================
 
+// Set form: weight w of key `key` in query q of its group.
+struct SetKey {
+    uint32_t key, q, w;
+};
+
 struct genie_plan {
     genie_index* ix = nullptr;
     int mode = 0;
@@ -225,6 +230,8 @@ struct genie_plan {
     std::vector<uint32_t> h_skeys;   // set form: every group's sorted keys,
     std::vector<uint4> h_smask;      // their weight planes (two uint4 per key)
     std::vector<uint32_t> h_sgptr;   // and the groups' entry ranges
+    std::vector<SetKey> h_set_keys;  // matrix form: what the entries would be made from,
+    std::vector<uint32_t> h_set_kptr;  // group by group
     std::vector<uint32_t> h_sshift;  // per query: sample histogram shift
     uint32_t* d_skeys = nullptr;
     uint4* d_smask = nullptr;
@@ -2037,53 +2044,42 @@ static bool dense_batch_ok(genie_plan* p, uint32_t n_queries)
     return true;
 }
 
-// Gathers a set-valued batch for the matrix form, query by query: the hot
-// weights, a slot per window of the mid keys, the tail pairs, and whether the
-// counts that the scatter adds for a query fit a byte.
+// A set-valued batch for the matrix form.  Looked at query by query: the window
+// slots and tail postings that it would have, and whether the counts that the
+// scatter adds for a query fit a byte; filled in (fill) once the form is chosen.
 struct SetMatrixBatch {
     genie_plan* p;
     const DevIndex& d;
     uint32_t G, g = 0;
     bool wide = false;  // some query of the group needs 16-bit counters
     bool on;
-    uint64_t slots_limit = 0;
+    uint64_t slots = 0, pairs = 0, slots_limit = 0;
     std::vector<std::pair<uint32_t, uint32_t>> cold;  // weight, multiplicity
     SetMatrixBatch(genie_plan* plan, uint32_t groups) : p(plan), d(plan->ix->d), G(groups), on(d.sm)
     {
         slots_limit = on ? set_matrix_slots(d, G) : 0;
         p->sm_ok = false;
-        p->h_sm_slots.clear();
-        p->h_sm_pairs.clear();
         p->h_sm_units8.clear();
         p->h_sm_units16.clear();
         p->sm_events = 0;
-        if (on) {
-            p->h_sm_wq.assign((uint64_t)G * 32 * kSmHot, 0);
-            p->h_sm_slot_ptr.assign(G + 1, 0);
-            p->h_sm_pair_ptr.assign(G + 1, 0);
+        if (on)
             p->h_sm_evbase.assign(G, 0);
-        }
     }
-    template <class KW>
-    void query(uint32_t j, const KW* b, const KW* e)
+    void query(const SetKey* b, const SetKey* e)
     {
         if (!on)
             return;
         cold.clear();
         for (; b != e; ++b) {
             const uint32_t c = d.h_sm_class[b->key];
-            if (c < kSmHot) {
-                p->h_sm_wq[((uint64_t)g * 32 + j) * kSmHot + c] = (uint8_t)b->w;
+            if (c < kSmHot)
                 continue;
-            }
             cold.push_back({b->w, d.h_key_mult[b->key]});
             if (c == kSmTail) {
-                p->h_sm_pairs.push_back(make_uint2(b->key, j | b->w << 5));
+                ++pairs;
                 p->sm_events += d.h_key_start[b->key + 1] - d.h_key_start[b->key];
             } else {
-                const uint32_t n = d.h_sm_slots[c - kSmHot];
-                for (uint32_t i = 0; i < n; ++i)
-                    p->h_sm_slots.push_back(make_uint2((c - kSmHot) | j << 16 | b->w << 21, i | n << 16));
+                slots += d.h_sm_slots[c - kSmHot];
             }
         }
         // an object holds at most set_max_len occurrences, each key's at most
@@ -2098,25 +2094,19 @@ struct SetMatrixBatch {
         }
         wide |= bound > 255;
     }
-    void group_end(uint32_t)
+    void group_end()
     {
         if (!on)
             return;
-        p->h_sm_slot_ptr[g + 1] = (uint32_t)p->h_sm_slots.size();
-        p->h_sm_pair_ptr[g + 1] = (uint32_t)p->h_sm_pairs.size();
         if (wide) {
             p->h_sm_units16.push_back(2 * g);
             p->h_sm_units16.push_back(2 * g + 1);
         } else {
             p->h_sm_units8.push_back(g);
         }
-        if (p->sm_events > kSmMaxEvents || p->h_sm_slots.size() > slots_limit) {
+        if (p->sm_events > kSmMaxEvents || slots > slots_limit)
             on = false;  // the lists will be faster, or have to do
-            std::vector<uint2>().swap(p->h_sm_slots);
-            std::vector<uint2>().swap(p->h_sm_pairs);
-            return;
-        }
-        if (g + 1 < G)
+        else if (g + 1 < G)
             p->h_sm_evbase[g + 1] = (uint32_t)p->sm_events;
         wide = false;
         ++g;
@@ -2127,13 +2117,72 @@ struct SetMatrixBatch {
         if (!on)
             return false;
         const double wide_groups = (double)p->h_sm_units16.size() / 2;
-        const double past = std::max(0.0, (double)p->h_sm_slots.size() / G / kSmThreads - kSmSlots);
+        const double past = std::max(0.0, (double)slots / G / kSmThreads - kSmSlots);
         const double tail = (double)p->sm_events / G / d.sm_tiles;
         const double fill = std::min(1.0, (G + wide_groups) * std::max(1u, d.sm_tiles / 4) / 512.0);
         return ((3.6 * (G - wide_groups) + 4.2 * wide_groups) * past) / fill + std::max(0.02 * G / fill, 0.6) * tail <=
                set_lists_ns(d, G);
     }
+    // From the kept groups: the hot weights, a slot per window of the mid keys,
+    // the tail pairs.
+    void fill()
+    {
+        p->h_sm_wq.assign((uint64_t)G * 32 * kSmHot, 0);
+        p->h_sm_slots.clear();
+        p->h_sm_slots.reserve(slots);
+        p->h_sm_pairs.clear();
+        p->h_sm_pairs.reserve(pairs);
+        p->h_sm_slot_ptr.assign(G + 1, 0);
+        p->h_sm_pair_ptr.assign(G + 1, 0);
+        for (uint32_t i = 0; i < G; ++i) {
+            for (uint32_t x = p->h_set_kptr[i]; x < p->h_set_kptr[i + 1]; ++x) {
+                const SetKey& k = p->h_set_keys[x];
+                const uint32_t c = d.h_sm_class[k.key];
+                if (c < kSmHot) {
+                    p->h_sm_wq[((uint64_t)i * 32 + k.q) * kSmHot + c] = (uint8_t)k.w;
+                } else if (c == kSmTail) {
+                    p->h_sm_pairs.push_back(make_uint2(k.key, k.q | k.w << 5));
+                } else {
+                    const uint32_t n = d.h_sm_slots[c - kSmHot];
+                    for (uint32_t j = 0; j < n; ++j)
+                        p->h_sm_slots.push_back(make_uint2((c - kSmHot) | k.q << 16 | k.w << 21, j | n << 16));
+                }
+            }
+            p->h_sm_slot_ptr[i + 1] = (uint32_t)p->h_sm_slots.size();
+            p->h_sm_pair_ptr[i + 1] = (uint32_t)p->h_sm_pairs.size();
+        }
+    }
 };
+
+// The forward lists' entries of one more group: keys ascending, bit j of plane b =
+// bit b of query j's weight for the key.  False when the table of a workgroup does
+// not hold them.
+static bool set_group_entries(genie_plan* p, SetKey* b, SetKey* e)
+{
+    std::sort(b, e, [](const SetKey& x, const SetKey& y) { return x.key < y.key; });
+    const size_t first = p->h_skeys.size();
+    while (b != e) {
+        uint32_t m[8] = {};
+        const uint32_t key = b->key;
+        for (; b != e && b->key == key; ++b)
+            for (int i = 0; i < kSetWeightPlanes; ++i)
+                m[i] |= ((b->w >> i) & 1u) << b->q;
+        p->h_skeys.push_back(key);
+        p->h_smask.push_back(make_uint4(m[0], m[1], m[2], m[3]));
+        p->h_smask.push_back(make_uint4(m[4], m[5], m[6], m[7]));
+    }
+    p->h_sgptr.push_back((uint32_t)p->h_skeys.size());
+    return p->h_skeys.size() - first <= kSetEntries;
+}
+
+// ... of the groups that were kept for the matrix form (seen to fit).
+static void set_kept_entries(genie_plan* p)
+{
+    for (size_t g = 0; g + 1 < p->h_set_kptr.size(); ++g)
+        (void)set_group_entries(p, p->h_set_keys.data() + p->h_set_kptr[g], p->h_set_keys.data() + p->h_set_kptr[g + 1]);
+    p->h_set_keys.clear();
+    p->h_set_kptr.assign(1, 0);
+}
 
 // Whether the uploaded batch can run the set form (set-valued tables with
 // forward lists): per query, the sum of its items' weights over the
@@ -2141,9 +2190,9 @@ struct SetMatrixBatch {
 // constant over every key it touches, i.e. a weight per key, at most
 // kSetMaxWeight; the longest forward list times the query's largest weight is
 // below kSetNoQuery (that threshold marks "no query"); a group of 32 queries
-// holds at most kSetEntries keys.  Builds every group's entries (keys
-// ascending, bit j of plane b = bit b of query j's weight for the key) and
-// every query's sample histogram shift (its count bound >> shift < 256).
+// holds at most kSetEntries keys.  Builds every group's part of the matrix form's
+// batch, or its entries when the forward lists run it, and every query's sample
+// histogram shift (its count bound >> shift < 256).
 static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
 {
     const DevIndex& d = p->ix->d;
@@ -2154,15 +2203,14 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
         uint64_t pos;
         int64_t dw;
     };
-    struct KW {
-        uint32_t key, q, w;
-    };
     std::vector<Ev> ev;
-    std::vector<KW> gk;  // the group's (key, query in group, weight)
+    std::vector<SetKey> gk;  // the group's keys
     const uint32_t G = (n_queries + 31) / 32;
     p->h_skeys.clear();
     p->h_smask.clear();
-    p->h_sgptr.assign(G + 1, 0);
+    p->h_sgptr.assign(1, 0);
+    p->h_set_keys.clear();
+    p->h_set_kptr.assign(1, 0);
     p->h_sshift.assign(n_queries, 0);
     SetMatrixBatch sm(p, G);
     for (uint32_t g = 0; g < G; ++g) {
@@ -2217,25 +2265,31 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
             while ((bound >> sh) > 255)
                 ++sh;
             p->h_sshift[q] = sh;
-            sm.query(q - g * 32, gk.data() + first, gk.data() + gk.size());
+            sm.query(gk.data() + first, gk.data() + gk.size());
         }
-        sm.group_end(g);
-        std::sort(gk.begin(), gk.end(), [](const KW& x, const KW& y) { return x.key < y.key; });
-        for (size_t i = 0; i < gk.size();) {
-            uint32_t m[8] = {};
-            const uint32_t key = gk[i].key;
-            for (; i < gk.size() && gk[i].key == key; ++i)
-                for (int b = 0; b < kSetWeightPlanes; ++b)
-                    m[b] |= ((gk[i].w >> b) & 1u) << gk[i].q;
-            p->h_skeys.push_back(key);
-            p->h_smask.push_back(make_uint4(m[0], m[1], m[2], m[3]));
-            p->h_smask.push_back(make_uint4(m[4], m[5], m[6], m[7]));
+        sm.group_end();
+        if (sm.on) {  // kept, for the entries should the lists run the batch after all
+            p->h_set_keys.insert(p->h_set_keys.end(), gk.begin(), gk.end());
+            p->h_set_kptr.push_back((uint32_t)p->h_set_keys.size());
+            if (gk.size() > kSetEntries) {
+                std::sort(gk.begin(), gk.end(), [](const SetKey& x, const SetKey& y) { return x.key < y.key; });
+                uint32_t keys = 0;
+                for (size_t i = 0; i < gk.size(); ++i)
+                    keys += i == 0 || gk[i].key != gk[i - 1].key;
+                if (keys > kSetEntries)
+                    return false;
+            }
+        } else {
+            set_kept_entries(p);
+            if (!set_group_entries(p, gk.data(), gk.data() + gk.size()))
+                return false;
         }
-        if (p->h_skeys.size() - p->h_sgptr[g] > kSetEntries)
-            return false;
-        p->h_sgptr[g + 1] = (uint32_t)p->h_skeys.size();
     }
     p->sm_ok = sm.finish();
+    if (p->sm_ok)
+        sm.fill();
+    else
+        set_kept_entries(p);
     return true;
 }
 

@@ -108,6 +108,31 @@ def test_matrix_form_of_unordered_postings():
     assert_topk_equal(ids, cnt, oi, oc, k, q, "unordered")
 
 
+def test_forms_of_successive_batches():
+    """Batches for the matrix form and for the forward lists in turn through one
+    plan (the slots of a batch of long runs end its gathering before its last
+    group), and a group of more keys than the lists' table holds."""
+    n, k = 150_000, 20
+    rp, v = genie_amd.synth.sets(8, n, 3, 12, 4000, 0.0)
+    v = np.where(np.arange(len(v)) % 3 > 0, v % 130, v).astype(np.int32)  # 130 tokens of long runs
+    t = Table.from_sets(rp, v)
+    rng = np.random.default_rng(4)
+    few = [rng.choice(np.arange(130, 4000), 5, replace=False) for _ in range(100)]
+    many = [rng.choice(130, 100, replace=False) for _ in range(70)]
+    last = [rng.choice(np.arange(130, 4000), 3, replace=False) for _ in range(32)] + many[:64]
+    wide = [np.arange(200 * (j % 19), 200 * (j % 19) + 200) for j in range(40)]  # 3,800 keys in 32 queries
+    p = Plan(t.device(), 100, 20_000, k, 0, mode=2)
+    for qs, form in ((few, "set"), (many, "set"), (few, "set"), (last, "set"), (wide, "plain"), (few, "set")):
+        q, qp = len(qs), np.concatenate([[0], np.cumsum([len(x) for x in qs])])
+        items = t.compile(W.set_ranges(qp, np.concatenate(qs).astype(np.int32), np.full(int(qp[-1]), 3)), q)
+        oi, oc = oracle_search_sample(t.export()["inv"].view(np.uint32), items, n, np.full(q, k), np.arange(q))
+        p.upload(items, q, np.full(q, k, np.uint32))
+        assert p.form() == form
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, q, form)
+
+
 def test_matrix_form_keeps_a_compressed_index_small():
     rp, v = genie_amd.synth.sets(5, 70_001, 3, 30, 40_000, 1.05)
     plain = Table.from_sets(rp, v)
