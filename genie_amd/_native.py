@@ -71,6 +71,7 @@ _sig(_hip, "genie_hip_plan_set_timing", C.c_int, _p, C.c_int)
 _sig(_hip, "genie_hip_plan_kernel_ms", C.c_int, _p, C.c_char_p, C.POINTER(C.c_double))
 _sig(_hip, "genie_hip_plan_bytes", C.c_int, _p, C.POINTER(_u64), C.POINTER(_u64))
 _sig(_hip, "genie_hip_plan_set_graph", C.c_int, _p, C.c_int)
+_sig(_hip, "genie_hip_plan_set_scratch", C.c_int, _p, _u64)
 _sig(_hip, "genie_hip_plan_set_config", C.c_int, _p, _u32, _u32, _u32)
 _sig(_hip, "genie_hip_plan_get_config", C.c_int, _p, C.POINTER(_u32), C.POINTER(_u32), C.POINTER(_u32),
      C.POINTER(_u32))
@@ -359,6 +360,11 @@ class Plan:
 
     def set_graph(self, on=True):
         _chk_hip(_hip.genie_hip_plan_set_graph(self.handle, 1 if on else 0))
+
+    def set_scratch(self, max_bytes=0):
+        """Most bytes of a buffer that a faster form takes and another does
+        without (0: no limit), from the next upload."""
+        _chk_hip(_hip.genie_hip_plan_set_scratch(self.handle, max_bytes))
 
     def set_config(self, block, tile_objs, seglen):
         _chk_hip(_hip.genie_hip_plan_set_config(self.handle, block, tile_objs, seglen))

@@ -68,6 +68,7 @@ static int dev_alloc(T** p, size_t n, uint64_t* acct = nullptr)
     hipError_t e = hipMalloc((void**)p, n * sizeof(T));
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // reported here, not by the next launch's check
         return fail(e == hipErrorOutOfMemory ? GENIE_E_OOM : GENIE_E_RUNTIME,
                     std::string("hipMalloc(") + std::to_string(n * sizeof(T)) +
                         " B): " + hipGetErrorString(e));
@@ -251,6 +252,7 @@ struct genie_plan {
              *d_sm_units16 = nullptr, *d_sm_events = nullptr, *d_sm_evptr = nullptr;
     uint64_t sm_wq_alloc = 0, sm_slots_alloc = 0, sm_pairs_alloc = 0, sm_slot_ptr_alloc = 0, sm_pair_ptr_alloc = 0,
              sm_evbase_alloc = 0, sm_units8_alloc = 0, sm_units16_alloc = 0, sm_events_alloc = 0, sm_evptr_alloc = 0;
+    uint64_t scratch_max = 0;        // most bytes of an optional buffer (0: no limit)
     uint32_t dn_groups = 0;
     uint32_t* d_dtab = nullptr;      // [dn_groups][dpad * 256] query masks
     uint64_t dtab_alloc = 0;
@@ -2293,12 +2295,41 @@ static bool sets_batch_ok(genie_plan* p, uint32_t n_queries)
     return true;
 }
 
+// Whether the plan may take an optional buffer of that size, one that a slower
+// form does without.
+static bool scratch_allowed(const genie_plan* p, uint64_t bytes) { return p->scratch_max == 0 || bytes <= p->scratch_max; }
+
+// Device buffers of the matrix form for the uploaded batch; false without room for
+// them (the forward lists need none).
+static bool set_matrix_buffers(genie_plan* p)
+{
+    auto room = [&](auto** buf, uint64_t* alloc, uint64_t n) {
+        n = std::max<uint64_t>(1, n);
+        return scratch_allowed(p, n * sizeof(**buf)) && grow_buf(p, buf, alloc, n) == GENIE_OK;
+    };
+    p->dn_groups = (p->n_queries + 31) / 32;
+    return room(&p->d_sm_wq, &p->sm_wq_alloc, p->h_sm_wq.size()) &&
+           room(&p->d_sm_slots, &p->sm_slots_alloc, p->h_sm_slots.size()) &&
+           room(&p->d_sm_pairs, &p->sm_pairs_alloc, p->h_sm_pairs.size()) &&
+           room(&p->d_sm_slot_ptr, &p->sm_slot_ptr_alloc, p->h_sm_slot_ptr.size()) &&
+           room(&p->d_sm_pair_ptr, &p->sm_pair_ptr_alloc, p->h_sm_pair_ptr.size()) &&
+           room(&p->d_sm_evbase, &p->sm_evbase_alloc, p->h_sm_evbase.size()) &&
+           room(&p->d_sm_units8, &p->sm_units8_alloc, p->h_sm_units8.size()) &&
+           room(&p->d_sm_units16, &p->sm_units16_alloc, p->h_sm_units16.size()) &&
+           room(&p->d_sm_events, &p->sm_events_alloc, p->sm_events) &&
+           room(&p->d_sm_evptr, &p->sm_evptr_alloc, p->dn_groups * (p->ix->d.sm_tiles + 1ull));
+}
+
 // Device buffers of the dense form for the uploaded batch: the query mask
 // tables, the sample histogram and the sample tile list (evenly spread tiles,
 // at least 16 and at least 1/16 of all tiles).
 static int prepare_dense(genie_plan* p)
 {
     const DevIndex& d = p->ix->d;
+    if (!p->dense_ok && p->sm_ok && !set_matrix_buffers(p)) {
+        p->sm_ok = false;
+        set_kept_entries(p);
+    }
     p->dn_groups = (p->n_queries + dense_qpg(p) - 1) / dense_qpg(p);
     const uint64_t tw = (uint64_t)d.dense_dpad * kDenseKeysPerDim;
     if (p->dense_ok) {
@@ -2323,22 +2354,12 @@ static int prepare_dense(genie_plan* p)
                 return rc;
         }
     } else if (p->sm_ok) {  // set form on the matrix cores
-        auto put = [&](auto** buf, uint64_t* alloc, const auto& v) -> int {
-            if (int rc = grow_buf(p, buf, alloc, std::max<uint64_t>(1, v.size())))
-                return rc;
-            return h2d(p, buf, v.data(), v.size() * sizeof(v[0]));
-        };
+        auto put = [&](auto** buf, const auto& v) { return h2d(p, buf, v.data(), v.size() * sizeof(v[0])); };
         int rc = 0;
-        if ((rc = put(&p->d_sm_wq, &p->sm_wq_alloc, p->h_sm_wq)) ||
-            (rc = put(&p->d_sm_slots, &p->sm_slots_alloc, p->h_sm_slots)) ||
-            (rc = put(&p->d_sm_pairs, &p->sm_pairs_alloc, p->h_sm_pairs)) ||
-            (rc = put(&p->d_sm_slot_ptr, &p->sm_slot_ptr_alloc, p->h_sm_slot_ptr)) ||
-            (rc = put(&p->d_sm_pair_ptr, &p->sm_pair_ptr_alloc, p->h_sm_pair_ptr)) ||
-            (rc = put(&p->d_sm_evbase, &p->sm_evbase_alloc, p->h_sm_evbase)) ||
-            (rc = put(&p->d_sm_units8, &p->sm_units8_alloc, p->h_sm_units8)) ||
-            (rc = put(&p->d_sm_units16, &p->sm_units16_alloc, p->h_sm_units16)) ||
-            (rc = grow_buf(p, &p->d_sm_events, &p->sm_events_alloc, std::max<uint64_t>(1, p->sm_events))) ||
-            (rc = grow_buf(p, &p->d_sm_evptr, &p->sm_evptr_alloc, p->dn_groups * (d.sm_tiles + 1ull))))
+        if ((rc = put(&p->d_sm_wq, p->h_sm_wq)) || (rc = put(&p->d_sm_slots, p->h_sm_slots)) ||
+            (rc = put(&p->d_sm_pairs, p->h_sm_pairs)) || (rc = put(&p->d_sm_slot_ptr, p->h_sm_slot_ptr)) ||
+            (rc = put(&p->d_sm_pair_ptr, p->h_sm_pair_ptr)) || (rc = put(&p->d_sm_evbase, p->h_sm_evbase)) ||
+            (rc = put(&p->d_sm_units8, p->h_sm_units8)) || (rc = put(&p->d_sm_units16, p->h_sm_units16)))
             return rc;
         if (!p->d_sshift)
             if ((rc = dev_alloc(&p->d_sshift, p->max_queries)))
@@ -2571,6 +2592,8 @@ static int plan_full_decode(genie_plan* p)
     // the layouts that the batch's kernels read: tile-major for the
     // direct-mapped scan over runs, the posting lists' for the others
     const bool tiled = runs_active(p);
+    if (!scratch_allowed(p, d.n_postings * sizeof(uint32_t)))
+        return GENIE_OK;
     if (tiled && !p->d_runs)
         if (dev_alloc(&p->d_runs, d.n_postings + kRunPad) != GENIE_OK)
             return GENIE_OK;  // no room for the scratch: in-kernel decode
@@ -2773,7 +2796,12 @@ static int plan_split_plain(genie_plan* p)
     // the filter form reads posting lists, decoded ones on a compressed index
     bool filter = d.key_start && (d.codec == 0 || p->decode_mode != 0) && d.n_objects < (1u << 30);
     split_queries(p, filter);
-    if (filter_span_count(p) > 1ull << 27)  // a GiB of spans: many items over many tiles
+    // a GiB of spans: many items over many tiles; or no room for them
+    const uint64_t spans = filter_span_count(p);
+    if (spans > 1ull << 27 ||
+        (spans && !(scratch_allowed(p, spans * sizeof(uint2)) &&
+                    grow_buf(p, &p->d_fspan, &p->fspan_alloc, spans) == GENIE_OK &&
+                    grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles) == GENIE_OK)))
         split_queries(p, filter = false);
     if (int rc = plan_full_decode(p))
         return rc;
@@ -2784,9 +2812,8 @@ static int plan_split_plain(genie_plan* p)
     else if (int rc = plan_decoded_spans(p))
         return rc;
     p->hash_whole = p->hash_whole && !p->h_hwork.empty() && (d.codec == 0 || p->dec_full);
-    if (p->hash_whole)
-        if (int rc = grow_buf(p, &p->d_sspan, &p->sspan_alloc, std::max<uint64_t>(1, p->n_items)))
-            return rc;
+    if (p->hash_whole && grow_buf(p, &p->d_sspan, &p->sspan_alloc, std::max<uint64_t>(1, p->n_items)) != GENIE_OK)
+        p->hash_whole = false;  // no room for the spans: chunks
     if (p->h_hwork.size() > p->hwork_alloc) {
         dev_free(p->d_hwork);
         p->hwork_alloc = 0;
@@ -2804,11 +2831,7 @@ static int plan_split_plain(genie_plan* p)
             return rc;
         if (int rc = grow_buf(p, &p->d_fhq, &p->fhq_alloc, nq))
             return rc;
-        if (int rc = grow_buf(p, &p->d_fspan, &p->fspan_alloc, filter_span_count(p)))
-            return rc;
         if (int rc = grow_buf(p, &p->d_fover_n, &p->fover_n_alloc, nq))
-            return rc;
-        if (int rc = grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles))
             return rc;
         if (int rc = h2d(p, &p->d_fhq, p->h_fhq.data(), nq * sizeof(uint4)))
             return rc;
@@ -3697,6 +3720,14 @@ int genie_hip_plan_run(genie_plan* p, void* stream)
     }
     HIP_TRY(hipGraphLaunch(p->gexec, s));
     p->ran = true;
+    return GENIE_OK;
+}
+
+int genie_hip_plan_set_scratch(genie_plan* p, uint64_t max_bytes)
+{
+    if (!p)
+        return fail(GENIE_E_INVALID, "null plan");
+    p->scratch_max = max_bytes;
     return GENIE_OK;
 }
 

@@ -153,6 +153,12 @@ int genie_hip_plan_kernel_ms(genie_plan* p, const char* name, double* ms);
 /* Replay the run as a captured hipGraph (captured at the next run, again
  * after any upload or configuration change).  Timing runs bypass the graph. */
 int genie_hip_plan_set_graph(genie_plan* p, int on);
+/* Most bytes of a buffer that a faster form takes and another does without (the
+ * decoded postings of a compressed batch, the filter kernels' spans, the matrix
+ * form's slots and tail postings): a batch that would need more, like one that
+ * finds no room, runs the other form.  From the next upload; 0 (default): as
+ * much as there is. */
+int genie_hip_plan_set_scratch(genie_plan* p, uint64_t max_bytes);
 /* Batched-form configuration: threads per workgroup (256/512/1024), objects
  * per tile (a multiple of 8192 whose 8-byte counters fit LDS) and the
  * longest posting span one wave takes at a time. */

@@ -119,3 +119,34 @@ def test_batch_without_items(mode):
     p.run()
     ids, cnt = p.download()
     assert not ids.any() and not cnt.any()
+
+
+@pytest.mark.parametrize("kind", ["filter", "compressed", "sets"])
+def test_batches_without_room_for_a_form(kind):
+    """A plan that may not take a form's buffers runs the form without them, in
+    turn with batches that may."""
+    n, q, k = 400_000, 60, 40
+    codec = dict(max_length=1024, load_balance=True, codec=11) if kind != "filter" else {}
+    if kind == "sets":
+        n = 60_000
+        rp, v = genie_amd.synth.sets(5, n, 3, 30, 40_000, 1.0)
+        qp, qv = genie_amd.synth.sets(6, q, 1, 30, 40_000, 1.0)
+        t, r = Table.from_sets(rp, v, **codec), W.set_ranges(qp, qv, np.full(len(qv), 2))
+    else:
+        rows = genie_amd.synth.rows(7, n, 40, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 1999, 2000)
+        t, r = Table.from_rows(rows, **codec), W.single_ranges(rows[:q], 0)
+    items = t.compile(r, q, merge_runs=bool(codec))
+    u = posting_items(t.export(), items) if codec else items
+    oi, oc = oracle_search_sample(t.export()["inv"].view(np.uint32), u, n, np.full(q, k), np.arange(q))
+    p = Plan(t.device(), q, len(items), k, 0, mode=2 if kind == "sets" else 0)
+    for limit in (0, 1, 0, 1):
+        p.set_scratch(limit)
+        p.upload(items, q, np.full(q, k, np.uint32))
+        if kind == "sets":
+            assert p.form() == "set"
+        else:
+            assert p.hash_queries() == q
+            assert p.decode_active() == (kind == "compressed" and limit == 0)
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, q, f"{kind} {limit}")
