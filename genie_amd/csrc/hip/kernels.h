@@ -1344,7 +1344,10 @@ struct MergeArgs {
 };
 
 constexpr uint32_t kMergePacked = kMergeMaxK;  // candidates sorted whole as 32-bit words
-constexpr uint32_t kMergeWave = 8 * kWave;     // ... by one wave
+// ... by one wave: 1,024 queries of 257 to 512 candidates take 10 us so and 14 by
+// the workgroup, 2,048 of k = 200 16 and 17 (22 with 128 here), the headline
+// batch's ~450 18 either way.
+constexpr uint32_t kMergeWave = 8 * kWave;
 
 __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
 {
@@ -1553,7 +1556,7 @@ __device__ __forceinline__ bool merge_packed(const MergeArgs& a, const uint64_t*
 // count and id are sorted whole instead (merge_packed; up to 512 of them by the
 // first wave alone, with no barrier): 333 queries of k = 1,000, 58 us selected
 // and sorted as 64 bits, 22 here; 384 of k = 100, 12 and 7; the headline batch,
-// 1,024 of k = 100 from ~450, 16 and 19.
+// 1,024 of k = 100 from ~450, 18 either way.
 // Otherwise candidates are staged in LDS when they fit; the bin holding the k-th key
 // is found with a wave-parallel suffix scan; the select stops as soon as a
 // bin holds exactly the keys still needed.

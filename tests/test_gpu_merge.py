@@ -1,4 +1,4 @@
-"""The merge at the sizes of its sorts (one wave up to 256 candidates, the
+"""The merge at the sizes of its sorts (one wave up to 512 candidates, the
 workgroup to 4,096, the select past that), with counts that pack into a word
 beside the id and counts too far apart for that, against the oracle."""
 import numpy as np
@@ -35,6 +35,35 @@ def test_merge_sizes(n, far):
     p.run()
     ids, cnt = p.download()
     assert_topk_equal(ids, cnt, oi, oc, k, q, f"n={n}")
+
+
+@pytest.mark.parametrize("far", [False, True])
+@pytest.mark.parametrize("k", [1000, 2048, 4096])
+def test_merge_of_more_candidates_than_the_stage(k, far):
+    """Six tiles that all hold k objects or more of the least count reached (so
+    each emits k): the select, its id bytes skipped, and the selected keys sorted
+    packed or, with counts too far apart, as they are."""
+    n, q = 6 * 65536 - 17, 3
+    rng = np.random.default_rng(k)
+    rows = np.stack([np.zeros(n, np.int64), rng.integers(0, 500, n), rng.integers(0, 3000, n)], 1).astype(np.int32)
+    r = np.zeros(3 * q, RANGE_DTYPE)
+    r["query"] = np.repeat(np.arange(q), 3)
+    r["dim"] = r["order"] = np.tile(np.arange(3), q)
+    r["low"] = [0, 7, 11] * q
+    r["up"] = [0, 7, 11] * q
+    r["weight"] = [1, 2, 60_000 if far else 4] * q
+    assert 6 * k > 4096
+    t = Table.from_rows(rows)
+    items = t.compile(r, q)
+    kq = np.full(q, k, np.uint32)
+    oi, oc = oracle_search_sample(t.export()["inv"].view(np.uint32), items, n, kq, np.arange(q))
+    assert (oc.reshape(q, k)[:, -1] == 1).all()  # the first item's ties
+    p = Plan(t.device(), q, len(items), k, 0, mode=0)
+    p.upload(items, q, kq)
+    for _ in range(2):
+        p.run()
+        ids, cnt = p.download()
+        assert_topk_equal(ids, cnt, oi, oc, k, q, f"k={k}")
 
 
 def test_merge_few_candidates():
