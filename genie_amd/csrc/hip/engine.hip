@@ -3142,6 +3142,14 @@ static int launch_decode_jobs(const DevIndex& d, const uint2* jobs, uint32_t nj,
 
 static KeyPos key_pos_of(const DevIndex& d) { return KeyPos{d.kpos, d.kpos_n, d.kpos_shift, d.key_start}; }
 
+template <bool C>
+static void launch_hash(HashArgs h, uint64_t nwork, hipStream_t s)
+{
+    const uint64_t most = launch_limit(kScanThreads);
+    for (uint64_t b = 0; b < nwork; b += most, h.work += 2 * most)
+        k_scan_hash<C><<<(uint32_t)std::min(most, nwork - b), kScanThreads, 0, s>>>(h);
+}
+
 // The plain form's scan: the hash kernel over the (query, tile) work of the
 // selective queries, then the direct-mapped kernel over the other queries.
 static int launch_scan(genie_plan* p, hipStream_t s)
@@ -3188,9 +3196,9 @@ static int launch_scan(genie_plan* p, hipStream_t s)
                 k_item_spans<<<(ni + 255) / 256, 256, 0, s>>>(p->dec_full ? p->d_uitems : p->d_items, ni, p->d_sspan);
             h.spans = p->d_sspan;
             h.sq_ptr = p->d_item_qptr;
-            k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
+            launch_hash<false>(h, nwork, s);
         } else if (a.codec == 0) {
-            k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
+            launch_hash<false>(h, nwork, s);
         } else if (p->dec_spans) {
             const uint32_t nj = (uint32_t)p->h_djobs.size();
             if (nj)
@@ -3203,9 +3211,9 @@ static int launch_scan(genie_plan* p, hipStream_t s)
             h.s.post = p->d_scratch;
             h.spans = p->d_sspan;
             h.sq_ptr = p->d_sq_ptr;
-            k_scan_hash<false><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
+            launch_hash<false>(h, nwork, s);
         } else {
-            k_scan_hash<true><<<(uint32_t)nwork, kScanThreads, 0, s>>>(h);
+            launch_hash<true>(h, nwork, s);
         }
     }
     if (nfwork) {
@@ -3254,10 +3262,21 @@ static int launch_scan(genie_plan* p, hipStream_t s)
                 else
                     k_scan_runs<16><<<n, kRunThreads, 0, s>>>(ra);
             }
-        } else if (plain_sparse(p, a.n_tiles))
-            launch_scan_t<true>(p->lane_bits, a, (uint32_t)blocks, s);
-        else
-            launch_scan_t<false>(p->lane_bits, a, (uint32_t)blocks, s);
+        } else {
+            const bool sparse = plain_sparse(p, a.n_tiles);
+            const uint64_t most = std::max(1u, launch_limit(kScanThreads) / a.n_tiles);  // queries of a launch
+            for (uint64_t b = 0; b < ndq; b += most) {
+                const uint32_t n = (uint32_t)std::min(most, ndq - b);
+                if (ndq > most) {
+                    a.qlist = p->d_dq + b;
+                    a.n_qlist = n;
+                }
+                if (sparse)
+                    launch_scan_t<true>(p->lane_bits, a, n * a.n_tiles, s);
+                else
+                    launch_scan_t<false>(p->lane_bits, a, n * a.n_tiles, s);
+            }
+        }
     }
     return GENIE_OK;
 }

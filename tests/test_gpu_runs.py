@@ -99,24 +99,35 @@ def test_runs_sets():
     check(t, items, items, n, q, 60, "sets")
 
 
-def test_runs_more_pairs_than_a_launch():
-    """(tile, query) pairs past what one launch of 1,024-thread workgroups
-    takes (2^32 threads)."""
-    n, q = 10_000_000, 27_500
+@pytest.mark.parametrize("form,q,threads", [("runs", 27_500, 1024), ("lists", 55_500, 512), ("hash", 15_000, 512)])
+def test_more_pairs_than_a_launch(form, q, threads):
+    """(tile, query) pairs past what one launch takes (2^32 threads), in each
+    scan of the plain form; two items of different weights a query."""
+    n = 10_000_000
     rows = np.arange(n, dtype=np.int32)[:, None] % 3
     rows[n // 2 + 1::4] = 3
-    assert -(-n // 65536) * q * 1024 > 1 << 32
-    first = np.array([np.argmax(rows[:, 0] == v) for v in range(4)])
+    rows[-4096:] = 4
+    first = np.array([np.argmax(rows[:, 0] == v) for v in range(5)])
     t = Table.from_rows(rows)
-    v = np.random.default_rng(1).integers(0, 4, q).astype(np.int32)
-    items = t.compile(W.single_ranges(v[:, None], 0), q)
-    p = Plan(t.device(), q, len(items), 1, 0, mode=0)
-    p.set_hash(0)
+    v = np.random.default_rng(1).integers(0, 4, (q, 2))
+    if form == "hash":  # 3 M postings a query: hash tiles of at most 16,384 objects; the result in the last one
+        v[:, 0] %= 3
+        v[:, 1] = 4
+    r = W.single_ranges(np.concatenate([v[:, :1], v[:, 1:]], 0).astype(np.int32), 0, np.repeat([1, 2], q))
+    r["query"] %= q
+    r = r[np.argsort(r["query"], kind="stable")]
+    items = t.compile(r, q)
+    p = Plan(t.device(), q, len(items), 1, 3, mode=0)  # a given bound: not the filter
+    p.set_hash(form == "hash")
+    p.set_sparse(1 if form == "lists" else 0)
     p.upload(items, q, np.ones(q, np.uint32))
-    assert not p.sparse_active()
+    assert p.hash_queries() == (q if form == "hash" else 0)
+    assert -(-n // (16384 if form == "hash" else 65536)) * q * threads > 1 << 32
     p.run()
     ids, cnt = p.download()
-    assert np.array_equal(ids, first[v]) and (cnt == 1).all()
+    assert p.hash_queries() == (q if form == "hash" else 0)
+    same = v[:, 0] == v[:, 1]
+    assert np.array_equal(ids, first[v[:, 1]]) and np.array_equal(cnt, np.where(same, 3, 2))
 
 
 def test_runs_of_more_keys_than_a_launch_of_workgroups():
