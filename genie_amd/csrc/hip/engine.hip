@@ -2796,9 +2796,11 @@ static int plan_split_plain(genie_plan* p)
     // the filter form reads posting lists, decoded ones on a compressed index
     bool filter = d.key_start && (d.codec == 0 || p->decode_mode != 0) && d.n_objects < (1u << 30);
     split_queries(p, filter);
-    // a GiB of spans: many items over many tiles; or no room for them
+    // a GiB of spans: many items over many tiles; or no room for them; or a few
+    // filter tiles beside queries whose items are compiled into chunks anyway
     const uint64_t spans = filter_span_count(p);
-    if (spans > 1ull << 27 ||
+    const bool chunks = (!p->h_hwork.empty() && !p->hash_whole) || (!p->h_dq.empty() && !runs_active(p));
+    if (spans > 1ull << 27 || (chunks && p->h_fwork.size() / 2 < kFiltFew) ||
         (spans && !(scratch_allowed(p, spans * sizeof(uint2)) &&
                     grow_buf(p, &p->d_fspan, &p->fspan_alloc, spans) == GENIE_OK &&
                     grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles) == GENIE_OK)))

@@ -31,6 +31,12 @@ constexpr uint32_t kFiltParts = 4;             // parts of a tile whose table fi
 constexpr uint32_t kFiltProbes = 256;          // taken slots in a row after which the table counts as full,
 constexpr uint32_t kFiltPartProbes = 1024;     // ... and a part's (97% of the slots)
 constexpr uint32_t kFiltMaxK = 1024;
+// Fewer filter tiles than this run on the hash kernel where chunks are compiled
+// for other queries anyway: the filter's three kernels take about 35 us however
+// few the tiles, and save 0.05 us a tile (25 us for 512 tiles at a time; the hash
+// kernel 20 us for 768 of a quarter).  78 queries of two tiles, 22 of them the
+// filter's: 119 us on the hash kernel, 148 with the filter.
+constexpr uint32_t kFiltFew = 640;
 constexpr uint32_t kFiltUnit = 4 * kWave;      // ids a wave loads at a time, 16 bytes a lane
 constexpr int kFiltUnits = 5;                  // units a wave keeps in registers
 constexpr uint32_t kFiltSeen = 8;              // units of a wave whose hits pass 1 counts, a bit an id

@@ -121,6 +121,19 @@ def test_batch_without_items(mode):
     assert not ids.any() and not cnt.any()
 
 
+@pytest.mark.parametrize("q", [21, 701])  # few filter tiles: the hash kernel takes them; many: both kernels
+@pytest.mark.parametrize("codec", [0, 13])
+def test_filter_and_hash_queries_in_one_batch(q, codec):
+    n, d = 1_000_000, 36
+    rows = genie_amd.synth.rows(11, n, d, genie_amd.synth.UNIFORM, 0.0, 0.0, 0, 1499, 1500)
+    qv, _ = genie_amd.synth.queries(12, rows, q, redraw_p=0.4, n_values=1500)
+    w = np.ones((q, d), np.int64)
+    w[::2, 3] = 2  # every second query: two weights
+    t = Table.from_rows(rows, **(dict(max_length=1024, load_balance=True, codec=codec) if codec else {}))
+    items = t.compile(W.single_ranges(qv, 0, w.reshape(-1)), q, merge_runs=bool(codec))
+    check(t, items, posting_items(t.export(), items) if codec else items, n, q, 30, q)
+
+
 @pytest.mark.parametrize("kind", ["filter", "compressed", "sets"])
 def test_batches_without_room_for_a_form(kind):
     """A plan that may not take a form's buffers runs the form without them, in
