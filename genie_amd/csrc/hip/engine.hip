@@ -2800,10 +2800,11 @@ static int plan_split_plain(genie_plan* p)
     // filter tiles beside queries whose items are compiled into chunks anyway
     const uint64_t spans = filter_span_count(p);
     const bool chunks = (!p->h_hwork.empty() && !p->hash_whole) || (!p->h_dq.empty() && !runs_active(p));
-    if (spans > 1ull << 27 || (chunks && p->h_fwork.size() / 2 < kFiltFew) ||
-        (spans && !(scratch_allowed(p, spans * sizeof(uint2)) &&
-                    grow_buf(p, &p->d_fspan, &p->fspan_alloc, spans) == GENIE_OK &&
-                    grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles) == GENIE_OK)))
+    if (spans != 0 &&
+        (spans > 1ull << 27 || (chunks && p->h_fwork.size() / 2 < kFiltFew) ||
+         !scratch_allowed(p, spans * sizeof(uint2)) ||
+         grow_buf(p, &p->d_fspan, &p->fspan_alloc, spans) != GENIE_OK ||
+         grow_buf(p, &p->d_fover, &p->fover_alloc, (uint64_t)nq * p->max_hash_tiles) != GENIE_OK))
         split_queries(p, filter = false);
     if (int rc = plan_full_decode(p))
         return rc;
